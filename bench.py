@@ -307,7 +307,7 @@ def bench_vcm(args):
             "unit": "GB/s",
             "frac": round(achieved_closest / HBM_PEAK_GBS, 4),
             "traffic": load_traffic("traffic_bvh_intersect_vcm_1Mtri.json"),
-            "kernel": ("k_trace8<false,false,false> (closest hit, 8-wide nodes, all launches of the timed jobs)"
+            "kernel": ("k_trace8 (closest hit, 8-wide nodes, all launches of the timed jobs)"
                        if node_bytes == 128 else "k_trace<false,false,false> (closest hit, all launches)"),
             "node_bytes": node_bytes,
             "launches": st["closest_launches"],
@@ -811,7 +811,7 @@ def bench_pt(args):
                            f"ray + {PT_B_CONT} B per continuation ray + {PT_B_MISS} B per miss"}
     closest = {"bound": "hbm", "achieved": round(tot["closest_rays"] * bytes_per_ray / (tot["closest_ms"] / 1e3) / 1e9, 1),
                "peak": HBM_PEAK_GBS, "unit": "GB/s", "traffic": None,
-               "kernel": "k_trace8<false,false,false> (closest hit, all launches of the timed images)",
+               "kernel": "k_trace8 (closest hit, all launches of the timed images)",
                "launches": tot["bounces"], "avg_launch_ms": round(tot["closest_ms"] / b, 4),
                "bytes_per_ray": round(bytes_per_ray, 1), "nodes_per_ray": round(nodes_per_ray, 3),
                "tris_per_ray": round(tris_per_ray, 3)}
@@ -1191,7 +1191,7 @@ def bench_instances(args):
         "top_tree_build_ms": round(build_ms, 1),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "k_trace8i<false,false,false> (closest hit; 64-B instance records not counted)",
+                     "kernel": "k_trace8, instanced (closest hit; instance nodes not counted)",
                      "bytes_per_ray": round(bytes_per_ray, 1)},
         "cpu_baseline": None,
     }

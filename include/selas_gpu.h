@@ -114,7 +114,8 @@ typedef struct sgpu_tuning {
                                      one is used up), a lane the next ray of its wave's chunk when its
                                      ray is done: 1..32 (default 8) */
     uint32_t trace_tree;          /* traversal tree: 0 binary nodes (64 B), 1 8-wide compressed
-                                     nodes (128 B, default); both are built at commit */
+                                     nodes (128 B, default; the triangle records lie among
+                                     them); both are built at commit */
     uint32_t trace_lds_nodes;     /* 8-wide single-scene launches: this many top nodes (breadth-first)
                                      read from LDS instead of memory: 0..9 (default 0) */
     uint32_t vcm_graphs;          /* 1 (default): each VCM wavefront replays its light and camera
@@ -264,8 +265,8 @@ int sgpu_occluded(sgpu_scene scene, const sgpu_rays_soa* rays, uint32_t* occlude
  * a fixed 64 MiB array in device memory instead, one per GPU (looked up at sgpu_context_create and
  * held until the process ends); the grid is capped so that its spill fits (rays beyond it are taken
  * grid-stride). Results equal sgpu_intersect's. Fails with SGPU_E_RANGE when even one block's
- * stacks would not fit (a scene whose stack bound, sgpu_scene_info's depth x 7, exceeds 65,552
- * entries). Calls that overlap on one GPU (other streams, other threads) share the array and race:
+ * stacks would not fit (a scene whose stack bound exceeds 65,552 words a lane: the binary tree's depth,
+ * or two words per level of the 8-wide tree). Calls that overlap on one GPU (other streams, other threads) share the array and race:
  * order them. */
 int sgpu_intersect_noalloc(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t n,
                            void* stream);

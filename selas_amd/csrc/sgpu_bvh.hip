@@ -13,7 +13,8 @@
 //                 are split by position, so every key is distinct. A node covers a run of leaves,
 //                 and so does each child: the node's record (both child boxes + child links) is
 //                 written at once from the pyramid's aligned runs.
-//   6. k_reorder  triangle records in leaf order; k_depth the deepest leaf (traversal stack size).
+//   6. k_depth    the deepest leaf (traversal stack size); then the 8-wide tree (build_wide) with the
+//                 triangle records in its slots.
 //
 // Boxes are inflated by 2^-18 of the scene's largest absolute coordinate. The boxes only cull;
 // the inflation keeps culling conservative with respect to the triangle test's rounding, so
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(const float* __restrict pos, ui
         r.a = make_float4(v0.x, v0.y, v0.z, __uint_as_float(i));
         r.b = make_float4(e1.x, e1.y, e1.z, __uint_as_float(g));
         r.c = make_float4(e2.x, e2.y, e2.z, __uint_as_float(prim));
+        r.pad = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         rec[i] = r;
         f3 lo = mk3(fminf(v0.x, fminf(v1.x, v2.x)), fminf(v0.y, fminf(v1.y, v2.y)), fminf(v0.z, fminf(v1.z, v2.z)));
         f3 hi = mk3(fmaxf(v0.x, fmaxf(v1.x, v2.x)), fmaxf(v0.y, fmaxf(v1.y, v2.y)), fmaxf(v0.z, fmaxf(v1.z, v2.z)));
@@ -311,14 +313,6 @@ __global__ void k_single(const float4* __restrict blo, const float4* __restrict 
     nodes[0] = nd;
 }
 
-__global__ __launch_bounds__(kBlock) void k_reorder(const TriRecord* __restrict in,
-                                                    const uint32_t* __restrict order, uint32_t n,
-                                                    TriRecord* __restrict out)
-{
-    uint32_t j = blockIdx.x * kBlock + threadIdx.x;
-    if (j < n) out[j] = in[order[j]];
-}
-
 // ---- PLOC: the binary tree by parallel locally-ordered clustering ----------------------------------
 //
 // Meister and Bittner, "Parallel Locally-Ordered Clustering for Bounding Volume Hierarchy
@@ -463,10 +457,19 @@ __global__ __launch_bounds__(kBlock) void k_depth(int n, const int* __restrict p
 //
 // A wide node starts from its binary node's two children and repeatedly opens the internal child
 // of largest surface area (the first such child on ties) until it has 8 children or only leaves.
-// k_wide_expand writes each task's children (binary refs and boxes) and its count of internal
-// children; an exclusive scan of those counts numbers the next level's nodes in task order, so
-// the numbering (and the tree) is deterministic; k_wide_emit quantizes the boxes and writes the
-// node and the next level's tasks.
+// A task is a binary node and the slot its wide node goes to. k_wide_expand writes each task's
+// children (binary refs and boxes) and the counts of its internal children and of the slots its
+// children take; an exclusive scan of those counts numbers the next level's tasks and slots in task
+// order, so the numbering (and the tree) is deterministic and a node's children are contiguous;
+// k_wide_emit quantizes the boxes and writes the node's first slot (internal children first), the
+// next level's tasks and the leaves' slots. In the top tree of an instanced scene leaves are nodes
+// too: a task ~k stands for leaf k, whose node is its instance's (InstNode). A node has 8 children
+// or only leaves, so there are at most 4 n / 7 nodes over n leaves.
+
+struct WideTask {
+    int ref;        // binary node, or ~leaf in a top tree
+    uint32_t slot;
+};
 
 __device__ __forceinline__ float half_area(const float* b)
 {
@@ -484,16 +487,24 @@ __device__ __forceinline__ void child_box(const BvhNode& nd, int c, float* b)
     b[5] = c ? nd.z.w : nd.z.y;
 }
 
-__global__ __launch_bounds__(kBlock) void k_wide_expand(const int* __restrict tasks, uint32_t n_tasks,
+template <bool TOP>
+__global__ __launch_bounds__(kBlock) void k_wide_expand(const WideTask* __restrict tasks, uint32_t n_tasks,
                                                         const BvhNode* __restrict bn, int* __restrict cref,
                                                         float* __restrict cbox, uint32_t* __restrict nchild,
-                                                        uint32_t* __restrict ninternal)
+                                                        uint64_t* __restrict counts)
 {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= n_tasks) return;
+    const int task = tasks[t].ref;
+    if (TOP && task < 0) {  // an instance's node
+        cref[8 * (size_t)t] = task;
+        nchild[t] = 0;
+        counts[t] = 0;
+        return;
+    }
     int ref[8];
     float box[8][6];
-    const BvhNode root = bn[tasks[t]];
+    const BvhNode root = bn[task];
     ref[0] = root.child.x;
     ref[1] = root.child.y;
     child_box(root, 0, box[0]);
@@ -518,14 +529,20 @@ __global__ __launch_bounds__(kBlock) void k_wide_expand(const int* __restrict ta
         child_box(nd, 1, box[m]);
         ++m;
     }
-    uint32_t internal = 0;
-    for (uint32_t k = 0; k < m; ++k) {
-        cref[8 * (size_t)t + k] = ref[k];
-        for (int a = 0; a < 6; ++a) cbox[48 * (size_t)t + 6 * k + a] = box[k][a];
-        internal += ref[k] >= 0 ? 1u : 0u;
-    }
-    nchild[t] = m;
-    ninternal[t] = internal;
+    uint32_t internal = 0, out = 0;
+    for (uint32_t k = 0; k < m; ++k) internal += (TOP || ref[k] >= 0) ? 1u : 0u;
+    // internal children first, both kinds in the order found
+    for (int pass = 0; pass < 2; ++pass)
+        for (uint32_t k = 0; k < m; ++k) {
+            if ((TOP || ref[k] >= 0) != (pass == 0)) continue;
+            cref[8 * (size_t)t + out] = ref[k];
+            for (int a = 0; a < 6; ++a) cbox[48 * (size_t)t + 6 * out + a] = box[k][a];
+            ++out;
+        }
+    nchild[t] = internal | (m << 8);
+    // slots: two per node, one per leaf after the first, an even number (nodes stay 128-byte aligned)
+    const uint32_t slots = (2 * internal + (m > internal ? m - internal - 1 : 0) + 1) & ~1u;
+    counts[t] = (uint64_t)internal | ((uint64_t)slots << 32);
 }
 
 // Smallest e in [-126, 127] with ext <= 254 * 2^e (ext >= 0).
@@ -538,15 +555,44 @@ __device__ __forceinline__ int plane_exponent(double ext)
     return e < -126 ? -126 : (e > 127 ? 127 : e);
 }
 
-__global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t level_base, uint32_t next_base,
-                                                      const uint32_t* __restrict offsets, const int* __restrict cref,
+// The largest float not above x whose low 11 bits are zero.
+__device__ __forceinline__ float origin_floor(float x)
+{
+    uint32_t u = __float_as_uint(x);
+    if (x < 0.0f && (u & ~kOriginMask)) u += ~kOriginMask + 1u;
+    return __uint_as_float(u & kOriginMask);
+}
+
+// The first slot of a node (or an instance's node), as the traversal reads it.
+struct NodeSlot {
+    uint32_t w[16];
+};
+
+template <bool TOP>
+__global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t level_base, uint32_t slot_base,
+                                                      const WideTask* __restrict tasks,
+                                                      const uint64_t* __restrict offsets, const int* __restrict cref,
                                                       const float* __restrict cbox, const uint32_t* __restrict nchild,
-                                                      WideNode* __restrict wide, int* __restrict next_tasks,
-                                                      uint32_t* __restrict bad)
+                                                      NodeSlot* __restrict out, uint32_t* __restrict out_slot,
+                                                      WideTask* __restrict next_tasks,
+                                                      uint32_t* __restrict leaf_slot,
+                                                      const InstRecord* __restrict insts,
+                                                      const uint32_t* __restrict order, uint32_t* __restrict bad)
 {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= n_tasks) return;
-    const uint32_t m = nchild[t];
+    const uint32_t ni = nchild[t] & 0xFFu, m = nchild[t] >> 8, slot = tasks[t].slot;
+    out_slot[level_base + t] = slot;
+    NodeSlot w;
+    if (TOP && m == 0) {
+        InstNode in;
+        in.index = order[~cref[8 * (size_t)t]];
+        in.unused[0] = in.unused[1] = 0;
+        in.meta = 0;
+        for (int r = 0; r < 3; ++r) in.w2l[r] = insts[in.index].w2l[r];
+        *reinterpret_cast<InstNode*>(&out[level_base + t]) = in;
+        return;
+    }
     const float* B = cbox + 48 * (size_t)t;
     float lo[3] = {B[0], B[1], B[2]}, hi[3] = {B[3], B[4], B[5]};
     for (uint32_t k = 1; k < m; ++k)
@@ -554,45 +600,79 @@ __global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t
             lo[a] = fminf(lo[a], B[6 * k + a]);
             hi[a] = fmaxf(hi[a], B[6 * k + 3 + a]);
         }
-    WideNode w;
-    w.ox = lo[0];
-    w.oy = lo[1];
-    w.oz = lo[2];
-    uint32_t meta = m << 24;
+    const uint32_t base = slot_base + (uint32_t)(offsets[t] >> 32);
+    uint32_t meta = ni << 24 | m << 28;
     for (int a = 0; a < 3; ++a) {
-        w.qlo[a][0] = w.qlo[a][1] = 0;
-        w.qhi[a][0] = w.qhi[a][1] = 0;
-        const int e = plane_exponent((double)hi[a] - (double)lo[a]);
+        const float og = origin_floor(lo[a]);
+        w.w[a] = __float_as_uint(og) | ((a == 0 ? base : a == 1 ? base >> 11 : base >> 22) & ~kOriginMask);
+        const int e = plane_exponent((double)hi[a] - (double)og);
         const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
         const double sd = (double)sc;
-        meta |= (uint32_t)(e + 127) << (8 * a);
-        for (uint32_t k = 0; k < m; ++k) {
-            const float clo = B[6 * k + a], chi = B[6 * k + 3 + a];
-            double ql = floor(((double)clo - (double)lo[a]) / sd);
-            double qh = ceil(((double)chi - (double)lo[a]) / sd);
-            int qlo = ql < 0.0 ? 0 : (ql > 255.0 ? 255 : (int)ql);
-            int qhi = qh < 0.0 ? 0 : (qh > 255.0 ? 255 : (int)qh);
-            // the decoded planes (one FP32 rounding, as the traversal decodes them) must contain the box
-            while (qlo > 0 && fmaf((float)qlo, sc, lo[a]) > clo) --qlo;
-            while (qhi < 255 && fmaf((float)qhi, sc, lo[a]) < chi) ++qhi;
-            if (fmaf((float)qlo, sc, lo[a]) > clo || fmaf((float)qhi, sc, lo[a]) < chi) atomicOr(bad, 1u);
-            w.qlo[a][k >> 2] |= (uint32_t)qlo << (8 * (k & 3));
-            w.qhi[a][k >> 2] |= (uint32_t)qhi << (8 * (k & 3));
+        meta |= ((uint32_t)e & 0xFFu) << (8 * a);
+        uint32_t qw[2][2] = {{0, 0}, {0, 0}};
+        for (uint32_t k = 0; k < 8; ++k) {
+            int qlo = 255, qhi = 0;  // an empty box
+            if (k < m) {
+                const float clo = B[6 * k + a], chi = B[6 * k + 3 + a];
+                double ql = floor(((double)clo - (double)og) / sd);
+                double qh = ceil(((double)chi - (double)og) / sd);
+                qlo = ql < 0.0 ? 0 : (ql > 255.0 ? 255 : (int)ql);
+                qhi = qh < 0.0 ? 0 : (qh > 255.0 ? 255 : (int)qh);
+                // the decoded planes (one FP32 rounding) must contain the box
+                while (qlo > 0 && fmaf((float)qlo, sc, og) > clo) --qlo;
+                while (qhi < 255 && fmaf((float)qhi, sc, og) < chi) ++qhi;
+                if (fmaf((float)qlo, sc, og) > clo || fmaf((float)qhi, sc, og) < chi) atomicOr(bad, 1u);
+            }
+            qw[0][k >> 2] |= (uint32_t)qlo << (8 * (k & 3));
+            qw[1][k >> 2] |= (uint32_t)qhi << (8 * (k & 3));
+        }
+        for (int h = 0; h < 2; ++h) {
+            w.w[4 + 2 * a + h] = qw[0][h];
+            w.w[10 + 2 * a + h] = qw[1][h];
         }
     }
-    w.meta = meta;
-    uint32_t rank = 0;
-    for (uint32_t k = 0; k < 8; ++k) {
-        int r = k < m ? cref[8 * (size_t)t + k] : -1;
-        if (k < m && r >= 0) {
-            next_tasks[offsets[t] + rank] = r;
-            r = (int)(next_base + offsets[t] + rank);
-            ++rank;
-        }
-        w.child[k] = r;
+    w.w[3] = meta;
+    const uint32_t task_off = (uint32_t)(offsets[t] & 0xFFFFFFFFull);
+    for (uint32_t k = 0; k < m; ++k) {
+        const int r = cref[8 * (size_t)t + k];
+        if (k < ni)
+            next_tasks[task_off + k] = WideTask{r, base + 2 * k};
+        else
+            leaf_slot[~r] = k == ni ? slot + 1 : base + ni + k - 1;  // leaf k - ni: the node's second slot, or base + 2 ni + (k - ni) - 1
     }
-    for (int k = 0; k < 8; ++k) w.pad[k] = 0;
-    wide[level_base + t] = w;
+    out[level_base + t] = w;
+}
+
+// The nodes' first slots and the triangle records in their slots.
+__global__ __launch_bounds__(kBlock) void k_place_nodes(const NodeSlot* __restrict in, const uint32_t* __restrict slot,
+                                                        uint32_t n, NodeSlot* __restrict out)
+{
+    // four lanes a slot
+    const size_t k = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (k / 4 >= n) return;
+    reinterpret_cast<uint4*>(out + slot[k / 4])[k % 4] = reinterpret_cast<const uint4*>(in + k / 4)[k % 4];
+}
+
+__global__ __launch_bounds__(kBlock) void k_place_tris(const TriRecord* __restrict in, const uint32_t* __restrict order,
+                                                       const uint32_t* __restrict leaf_slot, uint32_t n,
+                                                       NodeSlot* __restrict out)
+{
+    const size_t k = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    const size_t j = k / 4;
+    if (j >= n) return;
+    reinterpret_cast<uint4*>(out + leaf_slot[j])[k % 4] = reinterpret_cast<const uint4*>(in + order[j])[k % 4];
+}
+
+// The binary tree's leaves named by their records' slots.
+__global__ __launch_bounds__(kBlock) void k_relabel(BvhNode* __restrict nodes, uint32_t n_int,
+                                                    const uint32_t* __restrict leaf_slot)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n_int) return;
+    int4 c = nodes[i].child;
+    if (c.x < 0) c.x = ~(int)leaf_slot[~c.x];
+    if (c.y < 0) c.y = ~(int)leaf_slot[~c.y];
+    nodes[i].child = c;
 }
 
 template <typename T>
@@ -605,69 +685,106 @@ struct DevBuf {
     }
 };
 
-// Collapses the binary tree (nodes, n_int internal nodes, root 0) into 8-wide nodes.
-int build_wide(sgpu_scene scene, const BvhNode* nodes, uint32_t n_int, hipStream_t stream)
+// Collapses the binary tree (nodes, root 0, over n leaves) into the scene's 8-wide tree, with the
+// triangle records rec[order[j]] of its leaves j. The top tree of an instanced scene passes its
+// instance records instead of triangles (order[j]: the instance of leaf j): its leaves become nodes.
+int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
+               const TriRecord* rec, const InstRecord* insts)
 {
-    DevBuf<int> d_tasks, d_next, d_cref;
+    const bool top = insts != nullptr;
+    const uint32_t n_leaves = std::max(n, 2u);  // a tree of one leaf has a root with two children, the leaf twice
+    const size_t max_nodes = (size_t)n_leaves * 4 / 7 + 2 + (top ? n_leaves : 0);
+    DevBuf<WideTask> d_tasks, d_next;
+    DevBuf<int> d_cref;
     DevBuf<float> d_cbox;
-    DevBuf<uint32_t> d_nch, d_nint, d_off, d_bad;
-    DevBuf<WideNode> d_all;
+    DevBuf<uint32_t> d_nch, d_bad, d_slot, d_leaf_slot;
+    DevBuf<uint64_t> d_cnt, d_off;
+    DevBuf<NodeSlot> d_all;
     DevBuf<uint8_t> d_tmp;
-    SGPU_HIP_TRY(d_tasks.alloc(n_int));
-    SGPU_HIP_TRY(d_next.alloc(n_int));
-    SGPU_HIP_TRY(d_cref.alloc(8 * (size_t)n_int));
-    SGPU_HIP_TRY(d_cbox.alloc(48 * (size_t)n_int));
-    SGPU_HIP_TRY(d_nch.alloc(n_int));
-    SGPU_HIP_TRY(d_nint.alloc(n_int));
-    SGPU_HIP_TRY(d_off.alloc(n_int));
+    SGPU_HIP_TRY(d_tasks.alloc(max_nodes));
+    SGPU_HIP_TRY(d_next.alloc(max_nodes));
+    SGPU_HIP_TRY(d_cref.alloc(8 * max_nodes));
+    SGPU_HIP_TRY(d_cbox.alloc(48 * max_nodes));
+    SGPU_HIP_TRY(d_nch.alloc(max_nodes));
+    SGPU_HIP_TRY(d_cnt.alloc(max_nodes));
+    SGPU_HIP_TRY(d_off.alloc(max_nodes));
     SGPU_HIP_TRY(d_bad.alloc(1));
-    SGPU_HIP_TRY(d_all.alloc(n_int));
+    SGPU_HIP_TRY(d_all.alloc(max_nodes));
+    SGPU_HIP_TRY(d_slot.alloc(max_nodes));
+    SGPU_HIP_TRY(d_leaf_slot.alloc(n_leaves));
     size_t tmp_bytes = 0;
-    SGPU_HIP_TRY(rocprim::exclusive_scan(nullptr, tmp_bytes, d_nint.p, d_off.p, 0u, (size_t)n_int,
-                                         rocprim::plus<uint32_t>(), stream));
+    SGPU_HIP_TRY(rocprim::exclusive_scan(nullptr, tmp_bytes, d_cnt.p, d_off.p, (uint64_t)0, max_nodes,
+                                         rocprim::plus<uint64_t>(), stream));
     SGPU_HIP_TRY(d_tmp.alloc(tmp_bytes));
-    const int root = 0;
-    SGPU_HIP_TRY(hipMemcpyAsync(d_tasks.p, &root, sizeof(int), hipMemcpyHostToDevice, stream));
+    const WideTask root{0, 0};
+    SGPU_HIP_TRY(hipMemcpyAsync(d_tasks.p, &root, sizeof(root), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemsetAsync(d_bad.p, 0, sizeof(uint32_t), stream));
     uint32_t level_base = 0, n_tasks = 1, depth = 0;
+    uint64_t slot_base = 2;
     while (n_tasks > 0) {
         const uint32_t grid = (n_tasks + kBlock - 1) / kBlock;
-        hipLaunchKernelGGL(k_wide_expand, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes, d_cref.p,
-                           d_cbox.p, d_nch.p, d_nint.p);
+        if (top)
+            hipLaunchKernelGGL(k_wide_expand<true>, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes,
+                               d_cref.p, d_cbox.p, d_nch.p, d_cnt.p);
+        else
+            hipLaunchKernelGGL(k_wide_expand<false>, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes,
+                               d_cref.p, d_cbox.p, d_nch.p, d_cnt.p);
         SGPU_HIP_TRY(hipGetLastError());
-        SGPU_HIP_TRY(rocprim::exclusive_scan(d_tmp.p, tmp_bytes, d_nint.p, d_off.p, 0u, (size_t)n_tasks,
-                                             rocprim::plus<uint32_t>(), stream));
-        uint32_t last[2] = {0, 0};
-        SGPU_HIP_TRY(hipMemcpyAsync(&last[0], d_off.p + n_tasks - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        SGPU_HIP_TRY(hipMemcpyAsync(&last[1], d_nint.p + n_tasks - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        const uint32_t next_base = level_base + n_tasks;
-        hipLaunchKernelGGL(k_wide_emit, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base, next_base, d_off.p,
-                           d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_next.p, d_bad.p);
-        SGPU_HIP_TRY(hipGetLastError());
+        SGPU_HIP_TRY(rocprim::exclusive_scan(d_tmp.p, tmp_bytes, d_cnt.p, d_off.p, (uint64_t)0, (size_t)n_tasks,
+                                             rocprim::plus<uint64_t>(), stream));
+        uint64_t last[2] = {0, 0};
+        SGPU_HIP_TRY(hipMemcpyAsync(&last[0], d_off.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(&last[1], d_cnt.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
         SGPU_HIP_TRY(hipStreamSynchronize(stream));
-        const uint32_t n_next = last[0] + last[1];
-        if ((uint64_t)next_base + n_next > n_int) return sgpu_fail(SGPU_E_RANGE, "wide tree larger than the binary tree");
+        const uint64_t total = last[0] + last[1];
+        const uint32_t n_next = (uint32_t)(total & 0xFFFFFFFFull), n_new = (uint32_t)(total >> 32);
+        if ((uint64_t)level_base + n_tasks + n_next > max_nodes)
+            return sgpu_fail(SGPU_E_STATE, "wide tree larger than its bound");
+        if (slot_base + n_new > 0x7FFFFFFFull) return sgpu_fail(SGPU_E_RANGE, "wide tree takes more than 2^31 slots");
+        if (top)
+            hipLaunchKernelGGL(k_wide_emit<true>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
+                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
+                               d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
+        else
+            hipLaunchKernelGGL(k_wide_emit<false>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
+                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
+                               d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
+        SGPU_HIP_TRY(hipGetLastError());
         std::swap(d_tasks.p, d_next.p);
-        level_base = next_base;
+        level_base += n_tasks;
+        slot_base += n_new;
         n_tasks = n_next;
         ++depth;
     }
     uint32_t bad = 0;
-    SGPU_HIP_TRY(hipMemcpy(&bad, d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost));
+    SGPU_HIP_TRY(hipMemcpyAsync(&bad, d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+    SGPU_HIP_TRY(hipStreamSynchronize(stream));
     if (bad) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
-    WideNode* wide = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&wide, (size_t)level_base * sizeof(WideNode)));
-    hipError_t e = hipMemcpyAsync(wide, d_all.p, (size_t)level_base * sizeof(WideNode), hipMemcpyDeviceToDevice, stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) {
-        (void)hipFree(wide);
-        return sgpu_fail(SGPU_E_HIP, std::string("wide tree copy: ") + hipGetErrorString(e));
-    }
-    scene->d_wide = wide;
+    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_wide, slot_base * kSlotBytes));
+    scene->n_slots = (uint32_t)slot_base;
     scene->n_wide = level_base;
     scene->wide_depth = depth;
+    NodeSlot* const slots = reinterpret_cast<NodeSlot*>(scene->d_wide);
+    auto grid4 = [](size_t k) { return dim3((uint32_t)((4 * k + kBlock - 1) / kBlock)); };
+    hipLaunchKernelGGL(k_place_nodes, grid4(level_base), dim3(kBlock), 0, stream, d_all.p, d_slot.p, level_base, slots);
+    SGPU_HIP_TRY(hipGetLastError());
+    if (!top) {
+        // (of the two slots of a single triangle one stays empty: zeros, which no ray hits)
+        if (n == 1) SGPU_HIP_TRY(hipMemsetAsync(slots + 1, 0, (slot_base - 1) * kSlotBytes, stream));
+        hipLaunchKernelGGL(k_place_tris, grid4(n), dim3(kBlock), 0, stream, rec, order, d_leaf_slot.p, n, slots);
+        SGPU_HIP_TRY(hipGetLastError());
+        const uint32_t n_int = n > 1 ? n - 1 : 1;
+        hipLaunchKernelGGL(k_relabel, dim3((n_int + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, nodes, n_int,
+                           d_leaf_slot.p);
+        SGPU_HIP_TRY(hipGetLastError());
+    }
+    SGPU_HIP_TRY(hipStreamSynchronize(stream));
     return SGPU_OK;
 }
+
+// Words of traversal stack a scene's trees can need: the binary one a word per level, the 8-wide one
+// an entry of two words per level.
+uint32_t tree_stack_words(uint32_t depth, uint32_t wide_depth) { return std::max(depth + 1, 2 * (wide_depth + 1)); }
 
 }  // namespace
 
@@ -1013,26 +1130,11 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
         scene->box[k] = host_ord2f(hb[k]);
         scene->box[3 + k] = host_ord2f(~hb[3 + k]);
     }
-    TriRecord* tris = nullptr;
-    hipError_t e = hipMalloc((void**)&tris, (size_t)n * sizeof(TriRecord));
-    if (e != hipSuccess) {
-        (void)hipFree(nodes);
-        return sgpu_fail(SGPU_E_NOMEM, "hipMalloc of triangle records failed");
-    }
-    hipLaunchKernelGGL(k_reorder, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order.p, n, tris);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) {
-        (void)hipFree(nodes);
-        (void)hipFree(tris);
-        return sgpu_fail(SGPU_E_HIP, std::string("triangle reorder: ") + hipGetErrorString(e));
-    }
     scene->d_nodes = nodes;
-    scene->d_tris = tris;
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
-    rc = build_wide(scene, nodes, scene->n_nodes, stream);
-    scene->stack_cap = std::max(scene->max_depth + 1, kWideMaxPush * scene->wide_depth + 1);
+    rc = build_wide(scene, nodes, n, stream, d_order.p, d_rec.p, nullptr);
+    scene->stack_cap = tree_stack_words(scene->max_depth, scene->wide_depth);
     return rc;
 }
 
@@ -1173,7 +1275,7 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
         for (int r = 0; r < 3; ++r)
             xrec[e].w2l[r] = make_float4((float)w2l[4 * r], (float)w2l[4 * r + 1], (float)w2l[4 * r + 2], (float)w2l[4 * r + 3]);
         xrec[e].wide = nullptr;
-        xrec[e].tris = nullptr;
+        xrec[e].pad = 0;
         xids[2 * e] = extra[e].id0;
         xids[2 * e + 1] = extra[e].id1;
     }
@@ -1219,13 +1321,13 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
             }
         WideNode w;
         SGPU_HIP_TRY(hipMemcpy(&w, b->d_wide, sizeof(WideNode), hipMemcpyDeviceToHost));
-        const uint32_t nch = w.meta >> 24;
-        const float o[3] = {w.ox, w.oy, w.oz};
-        float sc[3];
+        const uint32_t nch = w.meta >> 28;
+        float o[3], sc[3];
         for (int a = 0; a < 3; ++a) {
-            const uint32_t bits = ((w.meta >> (8 * a)) & 0xFFu) << 23;
-            std::memcpy(&sc[a], &bits, sizeof(float));
+            const uint32_t bits = w.origin_base[a] & kOriginMask;
+            std::memcpy(&o[a], &bits, sizeof(float));
         }
+        for (int a = 0; a < 3; ++a) sc[a] = std::ldexp(1.0f, (int)(int8_t)((w.meta >> (8 * a)) & 0xFFu));
         out.clear();
         for (uint32_t c = 0; c < nch && c < 8; ++c)
             for (int side = 0; side < 2; ++side)
@@ -1289,7 +1391,7 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
         for (int r = 0; r < 3; ++r)
             rec[k].w2l[r] = make_float4((float)w2l[4 * r], (float)w2l[4 * r + 1], (float)w2l[4 * r + 2], (float)w2l[4 * r + 3]);
         rec[k].wide = f.blas->d_wide;
-        rec[k].tris = f.blas->d_tris;
+        rec[k].pad = 0;
         scene->comp_blas.push_back(f.blas);
         for (int r = 0; r < 3; ++r)
             for (int c = 0; c < 3; ++c) scene->comp_l2w.push_back((float)f.l2w[4 * r + c]);
@@ -1324,23 +1426,9 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     int rc = build_binary(n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
                           scene->ctx->bvh_builder);
     if (rc != SGPU_OK) return rc;
-    // the top tree's leaves name composed instances by their composition index (instance i, then
-    // its instance j), so the closest-hit tie rule follows (inst_id0, inst_id1)
-    std::vector<uint32_t> order(n);
-    const uint32_t n_int = n > 1 ? n - 1 : 1;
-    std::vector<BvhNode> hn(n_int);
-    hipError_t e = hipMemcpy(order.data(), d_order.p, n * sizeof(uint32_t), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(hn.data(), nodes, n_int * sizeof(BvhNode), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) {
-        for (BvhNode& nd : hn) {
-            if (nd.child.x < 0) nd.child.x = ~(int)order[~nd.child.x];
-            if (nd.child.y < 0) nd.child.y = ~(int)order[~nd.child.y];
-        }
-        e = hipMemcpy(nodes, hn.data(), n_int * sizeof(BvhNode), hipMemcpyHostToDevice);
-    }
     InstRecord* d_inst = nullptr;
     uint32_t* d_ids = nullptr;
-    if (e == hipSuccess) e = hipMalloc((void**)&d_inst, rec.size() * sizeof(InstRecord));
+    hipError_t e = hipMalloc((void**)&d_inst, rec.size() * sizeof(InstRecord));
     if (e == hipSuccess) e = hipMalloc((void**)&d_ids, ids.size() * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemcpy(d_inst, rec.data(), rec.size() * sizeof(InstRecord), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_ids, ids.data(), ids.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -1357,9 +1445,11 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
     scene->blas_stack_cap = blas_cap;
-    rc = build_wide(scene, nodes, scene->n_nodes, stream);
+    // instance nodes name composed instances by their composition index (instance i, then its instance
+    // j), so the closest-hit tie rule follows (inst_id0, inst_id1)
+    rc = build_wide(scene, nodes, n, stream, d_order.p, nullptr, d_inst);
     // the top tree's stack, the exit entry, and the deepest placed tree's stack
-    scene->stack_cap = std::max(scene->max_depth + 1, kWideMaxPush * scene->wide_depth + 1) + 1 + blas_cap;
+    scene->stack_cap = tree_stack_words(scene->max_depth, scene->wide_depth) + 2 + blas_cap;
     if (rc != SGPU_OK) return rc;
     return bake_instance_curves(scene, composed(), stream);
 }

@@ -707,7 +707,6 @@ int sgpu_scene_release(sgpu_scene scene)
     if (scene->d_inst_geom_base) (void)hipFree(scene->d_inst_geom_base);
     if (scene->d_inst_l2w) (void)hipFree(scene->d_inst_l2w);
     if (scene->d_nodes) (void)hipFree(scene->d_nodes);
-    if (scene->d_tris) (void)hipFree(scene->d_tris);
     if (scene->d_wide) (void)hipFree(scene->d_wide);
     if (scene->d_cnodes) (void)hipFree(scene->d_cnodes);
     if (scene->d_curves) (void)hipFree(scene->d_curves);
@@ -1163,8 +1162,7 @@ int sgpu_scene_device_bytes(sgpu_scene scene, uint64_t* bytes)
 {
     if (!scene || !bytes) return sgpu_fail(SGPU_E_INVALID, "sgpu_scene_device_bytes: NULL argument");
     if (!scene->committed) return sgpu_fail(SGPU_E_STATE, "sgpu_scene_device_bytes: scene not committed");
-    uint64_t b = (uint64_t)scene->n_nodes * sizeof(BvhNode) + (uint64_t)scene->n_wide * sizeof(WideNode) +
-                 (uint64_t)scene->n_tris * sizeof(TriRecord) +
+    uint64_t b = (uint64_t)scene->n_nodes * sizeof(BvhNode) + (uint64_t)scene->n_slots * kSlotBytes +
                  sizeof(uint32_t) + (uint64_t)scene->n_materials * 22 * sizeof(float) +
                  (uint64_t)scene->n_geom_material * sizeof(uint32_t) + (uint64_t)scene->n_lights * sizeof(sgpu_light) +
                  (uint64_t)scene->n_geom_tex * sizeof(sgpu::PtexTex) +

@@ -18,8 +18,8 @@
 // BVH node: a binary node that stores the boxes of both children, laid out per axis so that
 // the two slab tests of one visit use three float4 loads plus one int4 load (64 B):
 //   x = (c0.lo.x, c0.hi.x, c1.lo.x, c1.hi.x), y = (...), z = (...), child = (c0, c1, 0, 0).
-// A child index >= 0 names an internal node; a negative index ~j names the triangle record j
-// (leaves hold one triangle).
+// A child index >= 0 names an internal node; a negative index ~j names the triangle record in slot j
+// of the 8-wide tree's array (leaves hold one triangle).
 struct BvhNode {
     float4 x;
     float4 y;
@@ -28,7 +28,7 @@ struct BvhNode {
 };
 static_assert(sizeof(BvhNode) == 64, "BvhNode must be 64 bytes");
 
-// Triangle record, 48 B, in BVH leaf order:
+// Triangle record, 64 B (48 used: half a cache line, so that four lanes fetch one in one access):
 //   a = (v0.x, v0.y, v0.z, bits(global triangle index)),
 //   b = (e1.x, e1.y, e1.z, bits(geomID)),    e1 = v1 - v0
 //   c = (e2.x, e2.y, e2.z, bits(primID)),    e2 = v2 - v0
@@ -37,34 +37,49 @@ struct TriRecord {
     float4 a;
     float4 b;
     float4 c;
+    float4 pad;
 };
-static_assert(sizeof(TriRecord) == 48, "TriRecord must be 48 bytes");
+static_assert(sizeof(TriRecord) == 64, "TriRecord must be 64 bytes");
 
-// 8-wide node, 128 B (one cache line), built by collapsing the binary tree. Child boxes are
-// quantized to 8 bits per plane relative to the node's box: plane = fma(q, 2^(e - 127), origin)
-// in FP32 (q * 2^(e - 127) is exact, so the decode rounds once), with q chosen in the builder so
-// that the decoded box contains the binary tree's (inflated) child box. child[c] >= 0: wide node
-// index; < 0: ~(triangle record index); slots c >= nchild are unused.
+// 8-wide tree, built by collapsing the binary tree: one array of 64-byte slots holding nodes (two
+// slots, 128 B, a cache line) and triangle records (one slot). A node's first slot is what a visit
+// reads; its second holds its first leaf's triangle. A node's other children are contiguous from its
+// base: internal child c at slot base + 2 c, leaf k >= 1 at base + 2 ni + k - 1. Child boxes are
+// quantized to 8 bits per plane relative to the node's origin: plane = fma(q, 2^e, origin) in FP32
+// (q * 2^e is exact, so the decode rounds once), with q chosen in the builder so that the decoded box
+// contains the binary tree's (inflated) child box. Child c < ni is internal, ni <= c < nch the leaf
+// c - ni; the other children's boxes are empty (lo 255, hi 0).
 struct WideNode {
-    float ox, oy, oz;
-    uint32_t meta;       // ex | ey << 8 | ez << 16 | nchild << 24 (biased exponents of the plane scales)
+    // the origin rounded down to 21 bits (float, the low 11 bits cut) above 11, 11 and 10 bits of base:
+    // the grid this leaves is finer than the boxes' inflation after quantization
+    uint32_t origin_base[3];
+    uint32_t meta;       // ex | ey << 8 | ez << 16 (signed exponents) | ni << 24 | nch << 28
     uint32_t qlo[3][2];  // axis a, child c: byte (c & 3) of qlo[a][c >> 2]
     uint32_t qhi[3][2];
-    int32_t child[8];
-    uint32_t pad[8];
+    TriRecord leaf0;
 };
 static_assert(sizeof(WideNode) == 128, "WideNode must be 128 bytes");
-constexpr uint32_t kWideMaxPush = 7;  // stack entries a wide node can push
+constexpr uint32_t kOriginMask = 0xFFFFF800u;
+constexpr uint32_t kSlotBytes = 64;
 
-// One composed instance of an instanced scene as the traversal reads it (64 bytes): the rows of
-// its world-to-local affine transform (x' = w.x x + w.y y + w.z z + w.w) and the 8-wide tree and
-// triangle records of the scene of geometries it places.
+// One composed instance of an instanced scene (64 bytes): the rows of its world-to-local affine
+// transform (x' = w.x x + w.y y + w.z z + w.w) and the 8-wide tree of the scene of geometries it
+// places.
 struct InstRecord {
     float4 w2l[3];
     const WideNode* wide;
-    const TriRecord* tris;
+    uint64_t pad;
 };
 static_assert(sizeof(InstRecord) == 64, "InstRecord must be 64 bytes");
+// A composed instance as a node of the top tree (its leaves are nodes like the others): meta = 0 (no
+// children), its index among the composed instances and its transform.
+struct InstNode {
+    uint32_t index;
+    uint32_t unused[2];
+    uint32_t meta;
+    float4 w2l[3];
+};
+static_assert(sizeof(InstNode) == kSlotBytes, "an instance node takes a node's first slot");
 // Round B-spline curve segment, 80 B, in curve-tree leaf order: the four control points (xyz,
 // radius; in world space, also for the curves of an instanced scene's placed scenes, which are
 // carried into world space at its commit), the geometry id (in the placed scene for an instanced
@@ -78,11 +93,11 @@ static_assert(sizeof(CurveRecord) == 80, "CurveRecord must be 80 bytes");
 // Stack entries of the curve tree's traversal (a binary tree: its depth must stay below this).
 constexpr uint32_t kCurveStack = 96;
 
-// The traversal stack entry that returns from an instance's tree to the top tree.
-constexpr int kInstExit = (int)0x80000000;
-
-// Slots of the LDS part of the per-lane traversal stack; deeper entries spill to global memory.
+// 32-bit words of the LDS part of the per-lane traversal stack; deeper entries spill to global memory.
+// The binary traversal's entries are one word (a child), the 8-wide one's two (the children of a node
+// still to visit), at most one entry per level of the tree.
 #define SGPU_STACK_LDS 16
+constexpr uint32_t kWideStackLds = SGPU_STACK_LDS / 2;
 #define SGPU_TRACE_BLOCK 256
 
 // The traversal grid is at most kMaxTraceBlocksPerCu blocks per CU (sgpu_tuning bound); spill
@@ -132,11 +147,11 @@ struct sgpu_scene_s {
     uint32_t n_nodes = 0;
     uint32_t max_depth = 0;
     BvhNode* d_nodes = nullptr;
-    TriRecord* d_tris = nullptr;
-    WideNode* d_wide = nullptr;  // the same tree collapsed to 8-wide nodes (breadth-first order)
+    WideNode* d_wide = nullptr;  // the same tree collapsed to 8-wide nodes (breadth-first order): the slots
+    uint32_t n_slots = 0;
     uint32_t n_wide = 0;
     uint32_t wide_depth = 0;
-    uint32_t stack_cap = 0;      // traversal stack entries either tree can need
+    uint32_t stack_cap = 0;      // words of traversal stack either tree can need
     // set to non-zero by a traversal whose stack would exceed the tree depth (never expected)
     uint32_t* d_overflow = nullptr;
     // shading data (sgpu_scene_set_materials / sgpu_scene_set_lights)
@@ -325,7 +340,7 @@ __device__ __forceinline__ uint32_t sgpu_block_reserve(uint32_t n, uint32_t* cou
 }
 
 // ---- internal entry points between translation units --------------------------------------------
-// Builds d_nodes/d_tris (and the 8-wide d_wide) for the scene's triangles (sgpu_bvh.hip).
+// Builds d_nodes and the 8-wide d_wide with the triangle records (sgpu_bvh.hip).
 int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream);
 // Composes an instanced scene's instances and builds its top tree (d_nodes, d_wide over the
 // composed instances, d_inst, d_inst_ids) (sgpu_bvh.hip).
@@ -355,9 +370,8 @@ constexpr uint32_t kTraceWorkWords = 64;
 void sgpu_trace_work_zero(uint32_t* spill, hipStream_t stream);
 // A scene's trees as a multi-scene traversal launch reads them (one table entry per scene).
 struct TraceScene {
-    const BvhNode* nodes;
+    const BvhNode* nodes;      // its leaves name slots of `wide`
     const WideNode* wide;
-    const TriRecord* tris;
     uint32_t n_tris;
     uint32_t n_inst;           // > 0: an instanced scene (wide = its top tree over `insts`)
     const InstRecord* insts;

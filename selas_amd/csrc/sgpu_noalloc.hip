@@ -10,8 +10,8 @@
 
 #include "sgpu_internal.h"
 
-// 64 MiB: a spill depth of 62 entries (the 8-wide tree of a million triangles) still fits 1,056
-// blocks of 256 lanes (4 per CU of MI355X).
+// 64 MiB: a spill depth of 16 words (the trees of a million triangles) still fits 4,095 blocks of 256
+// lanes (16 per CU of MI355X).
 static constexpr size_t kScratchWords = (size_t)16 << 20;
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 
@@ -57,7 +57,7 @@ extern "C" int sgpu_intersect_noalloc(sgpu_scene scene, const sgpu_rays_soa* ray
     const size_t fit = (kScratchWords - kTraceWorkWords) / (depth * SGPU_TRACE_BLOCK);
     if (fit == 0)
         return sgpu_fail(SGPU_E_RANGE, "sgpu_intersect_noalloc: the scene's traversal stack (" +
-                                           std::to_string(scene->stack_cap) + " entries) needs more than the " +
+                                           std::to_string(scene->stack_cap) + " words) needs more than the " +
                                            std::to_string(kScratchWords * 4 >> 20) + " MiB scratch per block");
     const uint32_t cap = (uint32_t)std::min<size_t>(fit, UINT32_MAX);
     return sgpu_trace_launch(scene, rays, hits, nullptr, n, false, nullptr, (hipStream_t)stream, ptr, nullptr, nullptr,

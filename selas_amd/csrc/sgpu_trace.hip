@@ -130,7 +130,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) void k_trace(const BvhNode* __res
         if (MULTI) {
             const TraceScene ts = table[ray_scene[i]];
             rn = ts.nodes;
-            rt = ts.tris;
+            rt = reinterpret_cast<const TriRecord*>(ts.wide);
             rnt = ts.n_tris;
         }
 
@@ -224,285 +224,6 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) void k_trace(const BvhNode* __res
     }
 }
 
-// Compare-exchange of (key, ref) pairs: ascending keys.
-__device__ __forceinline__ void cswap(float& ka, int& ra, float& kb, int& rb)
-{
-    const bool sw = kb < ka;
-    const float k = sw ? kb : ka;
-    const int r = sw ? rb : ra;
-    kb = sw ? ka : kb;
-    rb = sw ? ra : rb;
-    ka = k;
-    ra = r;
-}
-
-// 8-wide traversal of the collapsed tree (WideNode). Per node the 8 quantized child boxes are
-// decoded and slab-tested in registers. Triangle children whose box is hit are tested at once;
-// internal children whose box is hit are ordered by entry distance with a fixed sorting network
-// (closest hit; the any-hit query keeps slot order), the nearest is entered and the rest are pushed
-// far to near. Hits are the triangle test's, independent of the tree and of the visiting order.
-// Waves take rays in chunks of 64 and a lane whose ray is done takes the next one of its wave's
-// chunk at once (one node visit per loop trip), so lanes do not wait for the wave's longest ray;
-// a wave whose chunk is used up takes the next from a counter, so waves do not wait for the
-// launch's longest chunk. Measured on MI355X against the one-ray-per-lane grid-stride loop: the
-// traversal workload (16M rays, 2M triangles) 1027 -> 1824 Mrays/s, the VCM job's closest-hit and
-// shadow traversals 13.2 + 12.2 -> 13.4 + 11.2 ms, both at 8 blocks per CU; held to 7 waves per
-// SIMD (72 VGPRs): at 8 the refill state spills and costs more than the eighth wave gives.
-// Wide nodes of a single-scene launch that may be kept in LDS (sgpu_tuning.trace_lds_nodes): the root
-// and the next breadth-first nodes (the root's children when it has 8 internal ones), visited by
-// nearly every ray. Measured on MI355X they hit in L1/L2 anyway, and the LDS branch costs 1-3 %.
-constexpr uint32_t kTopNodes = 9;
-constexpr uint32_t kTraceChunk = 64;  // rays a wave takes from the launch's counter at a time
-
-template <bool ANY, bool STATS, bool MULTI>
-__global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_trace8(const WideNode* __restrict wnodes, uint32_t n_top,
-                                                             const TriRecord* __restrict tris, uint32_t n_tris,
-                                                             const TraceScene* __restrict table,
-                                                             const uint32_t* __restrict ray_scene,
-                                                             sgpu_rays_soa rays, sgpu_hits_soa hits,
-                                                             uint32_t* __restrict occluded, uint32_t n,
-                                                            const uint32_t* __restrict n_ptr,
-                                                             uint32_t* __restrict spill, uint32_t stack_cap,
-                                                             unsigned long long* __restrict stats,
-                                                             uint32_t* __restrict overflow, uint32_t* __restrict work)
-{
-    __shared__ uint32_t lds_stack[SGPU_STACK_LDS][SGPU_TRACE_BLOCK];
-    __shared__ uint4 lds_top[kTopNodes * 6];  // the 96 bytes of each top node the traversal reads
-    const uint32_t lane = threadIdx.x;
-    const uint32_t gtid = blockIdx.x * SGPU_TRACE_BLOCK + threadIdx.x;
-    const uint32_t stride = gridDim.x * SGPU_TRACE_BLOCK;
-    unsigned long long cnt_nodes = 0, cnt_tris = 0;
-    if (n_ptr) n = *n_ptr;  // the count written on the device by the kernel that queued the rays
-    if (MULTI) n_top = 0;
-    for (uint32_t k = threadIdx.x; k < 6 * n_top; k += SGPU_TRACE_BLOCK)
-        lds_top[k] = reinterpret_cast<const uint4*>(wnodes + k / 6)[k % 6];
-    __syncthreads();
-
-    // Rays come in chunks of 64: wave w's first chunk is chunk w, the next ones come from the
-    // launch's counter (work[0], zeroed before the launch) past the grid's first chunks. A lane
-    // whose ray is done takes the next ray of its wave's chunk at once, and a wave whose chunk is
-    // used up takes the next chunk, so that lanes do not idle while a wave's longest ray is
-    // traversed and waves do not idle while others hold rays; a launch of at most one chunk per
-    // wave takes no atomic. Positions in a chunk come from a ballot, so `next` and `end` stay
-    // wave-uniform.
-    const uint32_t grid_rays = (gridDim.x * SGPU_TRACE_BLOCK / 64) * kTraceChunk;
-    uint32_t next = min(n, (gtid >> 6) * kTraceChunk);
-    uint32_t end = min(n, next + kTraceChunk);
-    bool drained = false;
-    const unsigned long long below = (1ull << (threadIdx.x & 63u)) - 1ull;
-
-    bool active = false;
-    uint32_t i = 0;
-    f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0), inv = mk3(0, 0, 0), oinv = mk3(0, 0, 0);
-    float tnear = 0.0f, tfar = 0.0f;
-    const WideNode* __restrict rw = wnodes;
-    const TriRecord* __restrict rt = tris;
-    uint32_t rnt = n_tris;
-    float best_t = 0.0f;
-    uint32_t best_key = 0xFFFFFFFFu, best_tri = 0xFFFFFFFFu;
-    float best_u = 0.0f, best_v = 0.0f;
-    bool hit_any = false;
-    // the per-lane stack: top SGPU_STACK_LDS entries in LDS (a ring), deeper ones spilled
-    uint32_t sp = 0;
-    bool overflowed = false;
-    int node = -1;
-
-    auto push = [&](int x) {
-        if (sp >= stack_cap) {
-            overflowed = true;
-            return;
-        }
-        if (sp < SGPU_STACK_LDS) {
-            lds_stack[sp][lane] = (uint32_t)x;
-        } else {
-            const uint32_t slot = sp % SGPU_STACK_LDS;
-            spill[(size_t)(sp - SGPU_STACK_LDS) * stride + gtid] = lds_stack[slot][lane];
-            lds_stack[slot][lane] = (uint32_t)x;
-        }
-        ++sp;
-    };
-    auto test_tri = [&](int ref) -> bool {  // true: any-hit found
-        const uint32_t j = (uint32_t)(~ref);
-        const TriRecord r = rt[j];
-        if (STATS) ++cnt_tris;
-        float t, u, v;
-        if (tri_test(r, o, d, tnear, t, u, v)) {
-            if (ANY) {
-                if (t <= tfar) return true;
-            } else {
-                uint32_t key = __float_as_uint(r.a.w);
-                if (t < best_t || (t == best_t && key < best_key)) {
-                    best_t = t;
-                    best_key = key;
-                    best_tri = j;
-                    best_u = u;
-                    best_v = v;
-                }
-            }
-        }
-        return false;
-    };
-
-    for (;;) {
-        // lanes without a ray take the next rays of the chunk (a new chunk when it is used up)
-        const unsigned long long idle = __ballot(!active);
-        if (idle && next >= end && !drained) {
-            if (grid_rays >= n) {
-                drained = true;  // the first chunks held every ray
-            } else {
-                uint32_t base = 0;
-                if ((threadIdx.x & 63u) == 0) base = grid_rays + atomicAdd(&work[0], kTraceChunk);
-                base = (uint32_t)__shfl((int)base, 0, 64);
-                if (base >= n) {
-                    drained = true;
-                } else {
-                    next = base;
-                    end = min(n, base + kTraceChunk);
-                }
-            }
-        }
-        if (idle && next < end) {
-            const uint32_t r = next + (uint32_t)__popcll(idle & below);
-            if (!active && r < end) {
-                i = r;
-                active = true;
-                o = mk3(rays.org_x[i], rays.org_y[i], rays.org_z[i]);
-                d = mk3(rays.dir_x[i], rays.dir_y[i], rays.dir_z[i]);
-                tnear = rays.tnear[i];
-                tfar = rays.tfar[i];
-                inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-                oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-                if (MULTI) {
-                    const TraceScene ts = table[ray_scene[i]];
-                    rw = ts.wide;
-                    rt = ts.tris;
-                    rnt = ts.n_tris;
-                }
-                best_t = tfar;
-                best_key = 0xFFFFFFFFu;
-                best_tri = 0xFFFFFFFFu;
-                best_u = 0.0f;
-                best_v = 0.0f;
-                hit_any = false;
-                sp = 0;
-                overflowed = false;
-                node = rnt > 0 ? 0 : -1;
-            }
-            next = min(end, next + (uint32_t)__popcll(idle));
-        }
-        if (__ballot(active) == 0) break;
-        if (!active) continue;
-        if (node >= 0) {
-            // ---- one node visit ----
-            uint4 w0, w1, w2, w3, w4, w5;
-            if ((uint32_t)node < n_top) {
-                const uint4* t = lds_top + 6 * node;
-                w0 = t[0], w1 = t[1], w2 = t[2], w3 = t[3], w4 = t[4], w5 = t[5];
-            } else {
-                const uint4* __restrict np = reinterpret_cast<const uint4*>(rw + node);
-                w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3], w4 = np[4], w5 = np[5];
-            }
-            if (STATS) ++cnt_nodes;
-            const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-            const uint32_t meta = w0.w;
-            const float sx = __uint_as_float((meta & 0xFFu) << 23);
-            const float sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23);
-            const float sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
-            const uint32_t nch = meta >> 24;
-            const uint32_t lox[2] = {w1.x, w1.y}, loy[2] = {w1.z, w1.w}, loz[2] = {w2.x, w2.y};
-            const uint32_t hix[2] = {w2.z, w2.w}, hiy[2] = {w3.x, w3.y}, hiz[2] = {w3.z, w3.w};
-            int ref[8] = {(int)w4.x, (int)w4.y, (int)w4.z, (int)w4.w, (int)w5.x, (int)w5.y, (int)w5.z, (int)w5.w};
-            float key[8];
-            uint32_t leaves = 0;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int sh = 8 * (c & 3), wi = c >> 2;
-                const float bx0 = fmaf((float)((lox[wi] >> sh) & 0xFFu), sx, ox);
-                const float bx1 = fmaf((float)((hix[wi] >> sh) & 0xFFu), sx, ox);
-                const float by0 = fmaf((float)((loy[wi] >> sh) & 0xFFu), sy, oy);
-                const float by1 = fmaf((float)((hiy[wi] >> sh) & 0xFFu), sy, oy);
-                const float bz0 = fmaf((float)((loz[wi] >> sh) & 0xFFu), sz, oz);
-                const float bz1 = fmaf((float)((hiz[wi] >> sh) & 0xFFu), sz, oz);
-                const float l_x = fmaf(bx0, inv.x, -oinv.x), h_x = fmaf(bx1, inv.x, -oinv.x);
-                const float l_y = fmaf(by0, inv.y, -oinv.y), h_y = fmaf(by1, inv.y, -oinv.y);
-                const float l_z = fmaf(bz0, inv.z, -oinv.z), h_z = fmaf(bz1, inv.z, -oinv.z);
-                const float tmin = fmaxf(fmaxf(fminf(l_x, h_x), fminf(l_y, h_y)), fmaxf(fminf(l_z, h_z), tnear));
-                const float tmax = fminf(fminf(fmaxf(l_x, h_x), fmaxf(l_y, h_y)), fminf(fmaxf(l_z, h_z), best_t));
-                const bool hit = (uint32_t)c < nch && tmin <= tmax;
-                // internal children: entry distance as the sort key (+inf: not to visit)
-                key[c] = hit && ref[c] >= 0 ? tmin : __int_as_float(0x7f800000);
-                if (hit && ref[c] < 0) leaves |= 1u << c;
-            }
-            // triangle children, in slot order
-            bool found = false;
-            while (leaves) {
-                const int c = __builtin_ctz(leaves);
-                leaves &= leaves - 1;
-                int r = ref[0];
-#pragma unroll
-                for (int k = 1; k < 8; ++k) r = c == k ? ref[k] : r;
-                if (test_tri(r)) {
-                    found = true;
-                    break;
-                }
-            }
-            if (ANY && found) {
-                hit_any = true;
-                node = -1;
-            } else {
-                const float inf = __int_as_float(0x7f800000);
-                if (!ANY) {
-                    // entry distances beyond the closest hit so far cannot hold a closer one
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) key[c] = key[c] <= best_t ? key[c] : inf;
-                    // ascending (key, ref): Batcher's odd-even merge sort network for 8 inputs
-                    cswap(key[0], ref[0], key[1], ref[1]); cswap(key[2], ref[2], key[3], ref[3]);
-                    cswap(key[4], ref[4], key[5], ref[5]); cswap(key[6], ref[6], key[7], ref[7]);
-                    cswap(key[0], ref[0], key[2], ref[2]); cswap(key[1], ref[1], key[3], ref[3]);
-                    cswap(key[4], ref[4], key[6], ref[6]); cswap(key[5], ref[5], key[7], ref[7]);
-                    cswap(key[1], ref[1], key[2], ref[2]); cswap(key[5], ref[5], key[6], ref[6]);
-                    cswap(key[0], ref[0], key[4], ref[4]); cswap(key[1], ref[1], key[5], ref[5]);
-                    cswap(key[2], ref[2], key[6], ref[6]); cswap(key[3], ref[3], key[7], ref[7]);
-                    cswap(key[2], ref[2], key[4], ref[4]); cswap(key[3], ref[3], key[5], ref[5]);
-                    cswap(key[1], ref[1], key[2], ref[2]); cswap(key[3], ref[3], key[4], ref[4]);
-                    cswap(key[5], ref[5], key[6], ref[6]);
-                }
-                // the nearest (first valid) is entered, the others pushed far to near
-                int nxt = -1;
-#pragma unroll
-                for (int c = 7; c >= 0; --c) {
-                    if (key[c] != inf) {
-                        if (nxt >= 0) push(nxt);
-                        nxt = ref[c];
-                    }
-                }
-                if (nxt >= 0) {
-                    node = nxt;
-                } else if (sp == 0) {
-                    node = -1;  // the ray is done
-                } else {
-                    // pop
-                    --sp;
-                    const uint32_t slot = sp % SGPU_STACK_LDS;
-                    node = (int)lds_stack[slot][lane];
-                    if (sp >= SGPU_STACK_LDS)
-                        lds_stack[slot][lane] = spill[(size_t)(sp - SGPU_STACK_LDS) * stride + gtid];
-                }
-            }
-            if (overflowed) node = -1;
-        }
-        if (node < 0) {
-            if (overflowed) atomicOr(overflow, 1u);
-            write_result<ANY>(i, hit_any, best_tri, best_t, best_u, best_v, rt, hits, occluded);
-            active = false;
-        }
-    }
-    if (STATS) {
-        atomicAdd(&stats[0], cnt_nodes);
-        atomicAdd(&stats[1], cnt_tris);
-    }
-}
-
 // A ray into an instance's space: x' = w.x x + w.y y + w.z z (+ w.w for points), summed by fused
 // multiply-adds from the last term (the arithmetic the oracle restates).
 __device__ __forceinline__ f3 inst_point(const float4* w, f3 p)
@@ -517,239 +238,381 @@ __device__ __forceinline__ f3 inst_vector(const float4* w, f3 v)
                fmaf(w[2].x, v.x, fmaf(w[2].y, v.y, w[2].z * v.z)));
 }
 
-// Traversal of an instanced scene: the top 8-wide tree over the composed instances, whose leaves
-// (~k: instance record k) are entered in entry-distance order like internal children; entering
-// one pushes kInstExit, moves the ray into the instance's space (t keeps its meaning: the
-// direction is not renormalized) and walks the instance's own 8-wide tree with triangles tested
-// inline; popping kInstExit restores the world ray. Composed instances are numbered in
-// composition order (instance i of the scene, then its instance j), so the closest hit is the
-// smallest t with ties to the smaller (composed instance, triangle) = (inst_id0, inst_id1, geomID,
-// primID).
-template <bool ANY, bool STATS, bool MULTI>
-__global__ __launch_bounds__(SGPU_TRACE_BLOCK) void k_trace8i(const WideNode* __restrict top, const TriRecord* __restrict top_tris,
-                                                              uint32_t top_n_tris, uint32_t n_inst,
-                                                              const InstRecord* __restrict insts,
-                                                              const uint32_t* __restrict inst_ids,
-                                                              const TraceScene* __restrict table,
-                                                              const uint32_t* __restrict ray_scene, sgpu_rays_soa rays,
-                                                              sgpu_hits_soa hits, uint32_t* __restrict occluded,
-                                                              uint32_t n, const uint32_t* __restrict n_ptr,
-                                                              uint32_t* __restrict spill, uint32_t stack_cap,
-                                                              unsigned long long* __restrict stats,
-                                                              uint32_t* __restrict overflow, uint32_t* __restrict comp_out)
+
+// Compare-exchange of sort keys, ascending.
+__device__ __forceinline__ void cswap(int& a, int& b)
 {
-    __shared__ uint32_t lds_stack[SGPU_STACK_LDS][SGPU_TRACE_BLOCK];
+    const int lo = min(a, b);
+    b = max(a, b);
+    a = lo;
+}
+
+// Wide nodes of a single-scene launch that may be kept in LDS (sgpu_tuning.trace_lds_nodes): the root
+// and the next breadth-first nodes (the root's children when it has 8 internal ones), visited by
+// nearly every ray. Measured on MI355X they hit in L1/L2 anyway, and the LDS branch costs 1-3 %.
+constexpr uint32_t kTopNodes = 9;
+constexpr uint32_t kTraceChunk = 64;  // rays a wave takes from the launch's counter at a time
+constexpr int kNext = -2;             // a lane that takes its next node once its triangles are tested
+
+// 8-wide traversal of the collapsed tree (WideNode), one ray per lane. In a trip of the wave's loop
+// every lane has at most one 64-byte slot to read: a triangle to test, or else a node to visit.
+// (Letting the lanes with triangles wait until 4, 8 or 16 of a wave have one cost 1-25 %.)
+//
+// Slots are fetched by the wave together: lane l asks for 16 bytes of the slot of lane 16 k + l / 4
+// in the k-th of four loads, straight into LDS, and each lane reads its own slot from there. A
+// divergent 16-byte load costs the address unit two cycles a lane whatever it hits; read lane by lane
+// (5 loads a node, 3 a triangle) the traversal workload kept that unit busy 84 % of the time.
+// The 16-byte pieces of a slot are permuted by bits 2-3 of its lane, so that the reads' banks differ.
+//
+// Node visit: the 8 quantized child boxes are slab-tested in registers, near and far planes picked
+// by the direction's signs, each plane one fused multiply-add t = q (2^e / d) + (origin - o) / d.
+// Leaf children hit become the lane's triangles to test (a slot base and a mask). Internal children
+// hit become a group: the base of the node's children and a list of their numbers, 4 bits each
+// (closest hit: by entry distance, a min/max network over keys that carry the number in their low
+// bits; any hit: the mask, in order). The group being walked is in registers, the groups above it on
+// the stack, so a visit pushes or pops one 8-byte entry at most and the stack is as deep as the tree.
+// Hits are the triangle test's, independent of the tree and of the visiting order.
+//
+// INST: scenes of instances. Leaves of the top tree are nodes (InstNode); visiting one saves the
+// group, pushes an exit entry (an empty group), moves the ray into the instance's space (t keeps its
+// meaning: the direction is not renormalized) and goes on at the instance's root; popping the exit
+// entry restores the world ray. Composed instances are numbered in composition order (instance i of
+// the scene, then its instance j), so the closest hit is the smallest t with ties to the smaller
+// (composed instance, triangle) = (inst_id0, inst_id1, geomID, primID).
+//
+// Waves take rays in chunks of 64 and a lane whose ray is done takes the next one of its wave's
+// chunk at once, so lanes do not wait for the wave's longest ray; a wave whose chunk is used up
+// takes the next from a counter, so waves do not wait for the launch's longest chunk.
+//
+// Bound by vector instructions now (81 % of the issue cycles on the traversal workload, address unit
+// 69 %); 32 KB of LDS a block allow 5 waves per SIMD. Against the version that read nodes and triangles
+// lane by lane, sorted (distance, child) pairs and kept a stack of children: 16M rays in 2M triangles
+// 15.3 -> 12.1 ms, 4M shadow rays in 1M triangles 2.67 -> 1.83 ms, 250K rays 0.62 -> 0.44 ms, 4M rays
+// through 256 instances (which had no refill) 10.1 -> 3.74 ms; hits the same bits.
+template <bool ANY, bool STATS, bool MULTI, bool INST, bool TOP>
+__global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace8(
+    TraceScene scene, const uint32_t* __restrict inst_ids, const TraceScene* __restrict table,
+    const uint32_t* __restrict ray_scene, sgpu_rays_soa rays, sgpu_hits_soa hits, uint32_t* __restrict occluded,
+    uint32_t n, const uint32_t* __restrict n_ptr, uint2* __restrict spill, uint32_t stack_cap,
+    unsigned long long* __restrict stats, uint32_t* __restrict overflow, uint32_t* __restrict work,
+    uint32_t* __restrict comp_out, uint32_t n_top)
+{
+    __shared__ uint2 lds_stack[kWideStackLds][SGPU_TRACE_BLOCK];
+    __shared__ uint4 lds_slots[4 * SGPU_TRACE_BLOCK];  // each lane's fetched slot, 4 KB a wave
+    __shared__ uint4 lds_top[TOP ? 4 * kTopNodes : 1];
     const uint32_t lane = threadIdx.x;
     const uint32_t gtid = blockIdx.x * SGPU_TRACE_BLOCK + threadIdx.x;
     const uint32_t stride = gridDim.x * SGPU_TRACE_BLOCK;
     unsigned long long cnt_nodes = 0, cnt_tris = 0;
-    const float inf = __int_as_float(0x7f800000);
     if (n_ptr) n = *n_ptr;  // the count written on the device by the kernel that queued the rays
+    if (TOP) {
+        for (uint32_t k = threadIdx.x; k < 4 * n_top; k += SGPU_TRACE_BLOCK)
+            lds_top[k] = reinterpret_cast<const uint4*>(scene.wide + k / 4)[k % 4];
+        __syncthreads();
+    }
 
-    for (uint32_t i = gtid; i < n; i += stride) {
-        const f3 wo = mk3(rays.org_x[i], rays.org_y[i], rays.org_z[i]);
-        const f3 wd = mk3(rays.dir_x[i], rays.dir_y[i], rays.dir_z[i]);
-        const float tnear = rays.tnear[i];
-        const float tfar = rays.tfar[i];
-        f3 o = wo, d = wd;
-        f3 inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-        f3 oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-        // the ray's scene: an instanced one (top tree over instances) or, in a multi-scene launch,
-        // possibly a scene of geometries (top tree over triangles)
-        const WideNode* __restrict tw = top;
-        const TriRecord* __restrict tt = top_tris;
-        uint32_t tn = top_n_tris, ni = n_inst;
-        const InstRecord* __restrict ri = insts;
-        if (MULTI) {
-            const TraceScene ts = table[ray_scene[i]];
-            tw = ts.wide;
-            tt = ts.tris;
-            tn = ts.n_tris;
-            ni = ts.n_inst;
-            ri = ts.insts;
+    // Rays come in chunks of 64: wave w's first chunk is chunk w, the next ones come from the
+    // launch's counter (work[0], zeroed before the launch) past the grid's first chunks. A launch of
+    // at most one chunk per wave takes no atomic. Positions in a chunk come from a ballot, so `next`
+    // and `end` stay wave-uniform.
+    const uint32_t grid_rays = (gridDim.x * SGPU_TRACE_BLOCK / 64) * kTraceChunk;
+    uint32_t next = min(n, (uint32_t)__builtin_amdgcn_readfirstlane(gtid >> 6) * kTraceChunk);
+    uint32_t end = min(n, next + kTraceChunk);
+    bool drained = false;
+    const unsigned long long below = (1ull << (threadIdx.x & 63u)) - 1ull;
+
+    bool active = false;
+    uint32_t i = 0;
+    f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0), inv = mk3(0, 0, 0), oinv = mk3(0, 0, 0);
+    float tnear = 0.0f;
+    float best_t = 0.0f;  // the any-hit query's tfar
+    uint32_t best_key = 0xFFFFFFFFu, best_tri = 0xFFFFFFFFu, best_inst = SGPU_INVALID_ID;
+    float best_u = 0.0f, best_v = 0.0f;
+    bool hit_any = false;
+    const WideNode* rw = scene.wide;
+    uint32_t cur = SGPU_INVALID_ID;  // INST: the instance being walked (none: the top tree)
+    int node = -1;                   // the slot of the node to visit, kNext: to be taken, -1: none left
+    uint32_t gbase = 0, glist = 0;   // the group being walked: children's base, children still to visit
+    uint32_t pfirst = 0, pbase = 0, pmask = 0;  // triangles to test: slot of leaf 0, base of the others, mask
+    uint32_t sp = 0;
+
+    // this wave's part of lds_slots and the lane's place in the fetches
+    const uint32_t wl = threadIdx.x & 63u;
+    uint4* const wave_slots = lds_slots + 4 * 64 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t piece = (wl & 3u) ^ ((wl >> 4) & 3u);
+    const uint32_t own = 4 * wl, swz = (wl >> 2) & 3u;
+
+    auto load_ray = [&](bool with_range) {
+        o = mk3(rays.org_x[i], rays.org_y[i], rays.org_z[i]);
+        d = mk3(rays.dir_x[i], rays.dir_y[i], rays.dir_z[i]);
+        if (with_range) {
+            tnear = rays.tnear[i];
+            best_t = rays.tfar[i];
         }
-        const bool has_inst = ni > 0;
-        const WideNode* __restrict rw = tw;
-        const TriRecord* __restrict rt = tt;
-        uint32_t cur = SGPU_INVALID_ID;  // the instance being walked; SGPU_INVALID_ID: the top tree
-
-        float best_t = tfar;
-        uint32_t best_key = 0xFFFFFFFFu, best_tri = 0xFFFFFFFFu, best_inst = 0xFFFFFFFFu;
-        float best_u = 0.0f, best_v = 0.0f;
-        bool hit_any = false;
-
-        uint32_t sp = 0;
-        bool overflowed = false;
-        auto push = [&](int x) {
-            if (sp >= stack_cap) {
-                overflowed = true;
-                return;
+    };
+    auto set_slopes = [&]() {
+        inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
+        oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+    };
+    // the stack: entries below kWideStackLds deep in LDS (a ring), deeper ones spilled
+    auto push = [&](uint32_t base, uint32_t list) {
+        if (sp >= stack_cap) {
+            atomicOr(overflow, 1u);
+            return;
+        }
+        const uint32_t slot = sp % kWideStackLds;
+        if (sp >= kWideStackLds) spill[(size_t)(sp - kWideStackLds) * stride + gtid] = lds_stack[slot][lane];
+        lds_stack[slot][lane] = make_uint2(base, list);
+        ++sp;
+    };
+    auto pop = [&]() {
+        --sp;
+        const uint32_t slot = sp % kWideStackLds;
+        const uint2 e = lds_stack[slot][lane];
+        if (sp >= kWideStackLds) lds_stack[slot][lane] = spill[(size_t)(sp - kWideStackLds) * stride + gtid];
+        gbase = e.x;
+        glist = e.y;
+    };
+    // the next node: the walked group's next child, or the top entry's
+    auto advance = [&]() {
+        while (glist == 0 && sp > 0) {
+            pop();
+            if (INST && glist == 0) {  // an exit entry: back in the top tree
+                load_ray(false);
+                set_slopes();
+                rw = MULTI ? table[ray_scene[i]].wide : scene.wide;
+                cur = SGPU_INVALID_ID;
             }
-            if (sp < SGPU_STACK_LDS) {
-                lds_stack[sp][lane] = (uint32_t)x;
+        }
+        if (glist == 0) {
+            node = -1;
+        } else if (ANY) {
+            node = (int)(gbase + 2u * (uint32_t)__builtin_ctz(glist));
+            glist &= glist - 1;
+        } else {
+            node = (int)(gbase + 2u * (glist & 7u));
+            glist >>= 4;
+        }
+    };
+
+    for (;;) {
+        // lanes without a ray take the next rays of the chunk (a new chunk when it is used up)
+        const unsigned long long idle = __ballot(!active);
+        if (idle && next >= end && !drained) {
+            if (grid_rays >= n) {
+                drained = true;  // the first chunks held every ray
             } else {
-                const uint32_t slot = sp % SGPU_STACK_LDS;
-                spill[(size_t)(sp - SGPU_STACK_LDS) * stride + gtid] = lds_stack[slot][lane];
-                lds_stack[slot][lane] = (uint32_t)x;
+                uint32_t base = 0;
+                if ((threadIdx.x & 63u) == 0) base = grid_rays + atomicAdd(&work[0], kTraceChunk);
+                base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                if (base >= n) {
+                    drained = true;
+                } else {
+                    next = base;
+                    end = min(n, base + kTraceChunk);
+                }
             }
-            ++sp;
-        };
-        auto pop = [&](int& x) -> bool {
-            if (sp == 0) return false;
-            --sp;
-            const uint32_t slot = sp % SGPU_STACK_LDS;
-            x = (int)lds_stack[slot][lane];
-            if (sp >= SGPU_STACK_LDS) lds_stack[slot][lane] = spill[(size_t)(sp - SGPU_STACK_LDS) * stride + gtid];
-            return true;
-        };
-        auto test_tri = [&](int ref) -> bool {  // true: any-hit found
-            const uint32_t j = (uint32_t)(~ref);
-            const TriRecord r = rt[j];
+        }
+        if (idle && next < end) {
+            const uint32_t r = next + (uint32_t)__popcll(idle & below);
+            if (!active && r < end) {
+                i = r;
+                active = true;
+                load_ray(true);
+                set_slopes();
+                bool walk;
+                if (MULTI) {
+                    const TraceScene ts = table[ray_scene[i]];
+                    rw = ts.wide;
+                    walk = ts.n_tris > 0 || (INST && ts.n_inst > 0);
+                } else {
+                    rw = scene.wide;
+                    walk = scene.n_tris > 0 || (INST && scene.n_inst > 0);
+                }
+                best_key = 0xFFFFFFFFu;
+                best_tri = 0xFFFFFFFFu;
+                best_inst = SGPU_INVALID_ID;
+                best_u = 0.0f;
+                best_v = 0.0f;
+                hit_any = false;
+                sp = 0;
+                glist = 0;
+                pmask = 0;
+                cur = SGPU_INVALID_ID;
+                node = walk ? 0 : -1;
+            }
+            next = min(end, next + (uint32_t)__popcll(idle));
+        }
+        if (__ballot(active) == 0) break;
+
+        const bool test = active && pmask != 0;
+        const bool visit = active && pmask == 0 && node >= 0;
+        int slot = visit ? node : -1;
+        if (test) {
+            const uint32_t k = (uint32_t)__builtin_ctz(pmask);
+            slot = (int)(k == 0 ? pfirst : pbase + k);
+            pmask &= pmask - 1;
+        }
+        // ---- the slots, fetched together ----
+        {
+            const bool in_top = TOP && (uint32_t)slot < 2 * n_top && visit;
+            const int ask = in_top ? -1 : slot;
+            unsigned long long from[4];
+            int s[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int src = 4 * (16 * k + (int)(wl >> 2));
+                const unsigned long long at = (unsigned long long)rw;
+                s[k] = __builtin_amdgcn_ds_bpermute(src, ask);
+                from[k] = at;
+                if (MULTI || INST)
+                    from[k] = (unsigned long long)(uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)at) |
+                              (unsigned long long)(uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)(at >> 32)) << 32;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (s[k] >= 0)
+                    __builtin_amdgcn_global_load_lds(
+                        (const __attribute__((address_space(1))) uint32_t*)(from[k] + (unsigned long long)(uint32_t)s[k] * kSlotBytes + 16 * piece),
+                        (__attribute__((address_space(3))) uint32_t*)(wave_slots + 64 * k), 16, 0, 0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        uint4 w0, w1, w2, w3;
+        if (TOP && visit && (uint32_t)slot < 2 * n_top) {
+            const uint4* t = lds_top + 2 * slot;
+            w0 = t[0], w1 = t[1], w2 = t[2], w3 = t[3];
+        } else {
+            w0 = wave_slots[own + (0 ^ swz)], w1 = wave_slots[own + (1 ^ swz)];
+            w2 = wave_slots[own + (2 ^ swz)], w3 = wave_slots[own + (3 ^ swz)];
+        }
+        if (test) {
+            // ---- one triangle test ----
+            TriRecord r;
+            r.a = make_float4(__uint_as_float(w0.x), __uint_as_float(w0.y), __uint_as_float(w0.z), __uint_as_float(w0.w));
+            r.b = make_float4(__uint_as_float(w1.x), __uint_as_float(w1.y), __uint_as_float(w1.z), __uint_as_float(w1.w));
+            r.c = make_float4(__uint_as_float(w2.x), __uint_as_float(w2.y), __uint_as_float(w2.z), __uint_as_float(w2.w));
             if (STATS) ++cnt_tris;
             float t, u, v;
             if (tri_test(r, o, d, tnear, t, u, v)) {
                 if (ANY) {
-                    if (t <= tfar) return true;
+                    if (t <= best_t) {
+                        hit_any = true;
+                        pmask = 0;
+                        node = -1;
+                    }
                 } else {
                     const uint32_t key = __float_as_uint(r.a.w);
-                    if (t < best_t || (t == best_t && (cur < best_inst || (cur == best_inst && key < best_key)))) {
+                    const bool first = INST ? (cur < best_inst || (cur == best_inst && key < best_key)) : key < best_key;
+                    if (t < best_t || (t == best_t && first)) {
                         best_t = t;
                         best_key = key;
-                        best_tri = j;
-                        best_inst = cur;
+                        best_tri = (uint32_t)slot;
+                        if (INST) best_inst = cur;
                         best_u = u;
                         best_v = v;
                     }
                 }
             }
-            return false;
-        };
-
-        int node = 0;
-        const bool walking = has_inst || tn > 0;
-        while (walking && !overflowed) {
-            // Leaving or entering an instance falls through to the node visit of the same trip: the
-            // entry popped after an exit is a top-tree entry (exits are only pushed on entering an
-            // instance from the top tree), and an entered instance starts at its root.
-            if (node == kInstExit) {
-                // back in the top tree
-                o = wo;
-                d = wd;
-                inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-                oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-                rw = tw;
-                cur = SGPU_INVALID_ID;
-                if (!pop(node)) break;
-            }
-            if (node < 0) {
-                // a leaf of the top tree: enter composed instance ~node
-                cur = (uint32_t)(~node);
-                const InstRecord ir = ri[cur];
-                o = inst_point(ir.w2l, wo);
-                d = inst_vector(ir.w2l, wd);
-                inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-                oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-                rw = ir.wide;
-                rt = ir.tris;
-                push(kInstExit);
-                if (overflowed) break;
-                node = 0;
-            }
-            const uint4* __restrict np = reinterpret_cast<const uint4*>(rw + node);
-            const uint4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3], w4 = np[4], w5 = np[5];
-            if (STATS) ++cnt_nodes;
-            const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
+        }
+        if (visit) {
+            // ---- one node visit ----
             const uint32_t meta = w0.w;
-            const float sx = __uint_as_float((meta & 0xFFu) << 23);
-            const float sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23);
-            const float sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
-            const uint32_t nch = meta >> 24;
-            const uint32_t lox[2] = {w1.x, w1.y}, loy[2] = {w1.z, w1.w}, loz[2] = {w2.x, w2.y};
-            const uint32_t hix[2] = {w2.z, w2.w}, hiy[2] = {w3.x, w3.y}, hiz[2] = {w3.z, w3.w};
-            int ref[8] = {(int)w4.x, (int)w4.y, (int)w4.z, (int)w4.w, (int)w5.x, (int)w5.y, (int)w5.z, (int)w5.w};
-            const bool in_top = cur == SGPU_INVALID_ID && has_inst;
-            float key[8];
-            uint32_t leaves = 0;
+            if (INST && (meta >> 28) == 0) {
+                // an instance: into its space, at its root
+                if (glist) push(gbase, glist);
+                push(0, 0);
+                const f3 wo = o, wd = d;
+                const float4 rows[3] = {make_float4(__uint_as_float(w1.x), __uint_as_float(w1.y), __uint_as_float(w1.z), __uint_as_float(w1.w)),
+                                        make_float4(__uint_as_float(w2.x), __uint_as_float(w2.y), __uint_as_float(w2.z), __uint_as_float(w2.w)),
+                                        make_float4(__uint_as_float(w3.x), __uint_as_float(w3.y), __uint_as_float(w3.z), __uint_as_float(w3.w))};
+                o = inst_point(rows, wo);
+                d = inst_vector(rows, wd);
+                set_slopes();
+                cur = w0.x;
+                rw = (MULTI ? table[ray_scene[i]].insts : scene.insts)[cur].wide;
+                node = 0;
+                glist = 0;
+            } else {
+                if (STATS) ++cnt_nodes;
+                const uint32_t ni = (meta >> 24) & 15u, nch = meta >> 28;
+                // per axis: slope a (per quantization step) and intercept b of the planes' distances
+                const float ax = __builtin_amdgcn_ldexpf(inv.x, (int)(meta << 24) >> 24);
+                const float ay = __builtin_amdgcn_ldexpf(inv.y, (int)(meta << 16) >> 24);
+                const float az = __builtin_amdgcn_ldexpf(inv.z, (int)(meta << 8) >> 24);
+                const float bx = fmaf(__uint_as_float(w0.x & kOriginMask), inv.x, -oinv.x);
+                const float by = fmaf(__uint_as_float(w0.y & kOriginMask), inv.y, -oinv.y);
+                const float bz = fmaf(__uint_as_float(w0.z & kOriginMask), inv.z, -oinv.z);
+                const uint32_t base = (w0.x & ~kOriginMask) | (w0.y & ~kOriginMask) << 11 | w0.z << 22;
+                const bool sx = __float_as_int(inv.x) < 0, sy = __float_as_int(inv.y) < 0, sz = __float_as_int(inv.z) < 0;
+                const uint32_t nx[2] = {sx ? w2.z : w1.x, sx ? w2.w : w1.y}, fx[2] = {sx ? w1.x : w2.z, sx ? w1.y : w2.w};
+                const uint32_t ny[2] = {sy ? w3.x : w1.z, sy ? w3.y : w1.w}, fy[2] = {sy ? w1.z : w3.x, sy ? w1.w : w3.y};
+                const uint32_t nz[2] = {sz ? w3.z : w2.x, sz ? w3.w : w2.y}, fz[2] = {sz ? w2.x : w3.z, sz ? w2.y : w3.w};
+                int key[8];
+                uint32_t hit = 0;
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int sh = 8 * (c & 3), wi = c >> 2;
-                const float bx0 = fmaf((float)((lox[wi] >> sh) & 0xFFu), sx, ox);
-                const float bx1 = fmaf((float)((hix[wi] >> sh) & 0xFFu), sx, ox);
-                const float by0 = fmaf((float)((loy[wi] >> sh) & 0xFFu), sy, oy);
-                const float by1 = fmaf((float)((hiy[wi] >> sh) & 0xFFu), sy, oy);
-                const float bz0 = fmaf((float)((loz[wi] >> sh) & 0xFFu), sz, oz);
-                const float bz1 = fmaf((float)((hiz[wi] >> sh) & 0xFFu), sz, oz);
-                const float l_x = fmaf(bx0, inv.x, -oinv.x), h_x = fmaf(bx1, inv.x, -oinv.x);
-                const float l_y = fmaf(by0, inv.y, -oinv.y), h_y = fmaf(by1, inv.y, -oinv.y);
-                const float l_z = fmaf(bz0, inv.z, -oinv.z), h_z = fmaf(bz1, inv.z, -oinv.z);
-                const float tmin = fmaxf(fmaxf(fminf(l_x, h_x), fminf(l_y, h_y)), fmaxf(fminf(l_z, h_z), tnear));
-                const float tmax = fminf(fminf(fmaxf(l_x, h_x), fmaxf(l_y, h_y)), fminf(fmaxf(l_z, h_z), best_t));
-                const bool hit = (uint32_t)c < nch && tmin <= tmax;
-                // the top tree's instance leaves are visited like internal children
-                const bool visit = hit && (ref[c] >= 0 || in_top);
-                key[c] = visit ? tmin : inf;
-                if (hit && ref[c] < 0 && !in_top) leaves |= 1u << c;
-            }
-            bool found = false;
-            while (leaves) {
-                const int c = __builtin_ctz(leaves);
-                leaves &= leaves - 1;
-                int r = ref[0];
-#pragma unroll
-                for (int k = 1; k < 8; ++k) r = c == k ? ref[k] : r;
-                if (test_tri(r)) {
-                    found = true;
-                    break;
+                for (int c = 0; c < 8; ++c) {
+                    const int sh = 8 * (c & 3), wi = c >> 2;
+                    const float t0x = fmaf((float)((nx[wi] >> sh) & 0xFFu), ax, bx);
+                    const float t0y = fmaf((float)((ny[wi] >> sh) & 0xFFu), ay, by);
+                    const float t0z = fmaf((float)((nz[wi] >> sh) & 0xFFu), az, bz);
+                    const float t1x = fmaf((float)((fx[wi] >> sh) & 0xFFu), ax, bx);
+                    const float t1y = fmaf((float)((fy[wi] >> sh) & 0xFFu), ay, by);
+                    const float t1z = fmaf((float)((fz[wi] >> sh) & 0xFFu), az, bz);
+                    const float tmin = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tnear));
+                    const float tmax = fminf(fminf(t1x, t1y), fminf(t1z, best_t));
+                    const bool in = tmin <= tmax;
+                    hit |= in ? 1u << c : 0u;
+                    // internal children: entry distance as the sort key, the slot (and 8) in its low bits
+                    if (!ANY) key[c] = in && (uint32_t)c < ni ? (__float_as_int(tmin) & ~15) | (8 | c) : 0x7FFFFFF0;
                 }
-            }
-            if (ANY && found) {
-                hit_any = true;
-                break;
-            }
-            if (!ANY) {
+                pmask = __builtin_amdgcn_ubfe(hit, ni, nch - ni);
+                pfirst = (uint32_t)node + 1;
+                pbase = base + 2 * ni - 1;
+                uint32_t list;
+                if (ANY) {
+                    list = __builtin_amdgcn_ubfe(hit, 0, ni);
+                } else {
+                    // Batcher's odd-even merge sort network for 8 keys
+                    cswap(key[0], key[1]); cswap(key[2], key[3]); cswap(key[4], key[5]); cswap(key[6], key[7]);
+                    cswap(key[0], key[2]); cswap(key[1], key[3]); cswap(key[4], key[6]); cswap(key[5], key[7]);
+                    cswap(key[1], key[2]); cswap(key[5], key[6]);
+                    cswap(key[0], key[4]); cswap(key[1], key[5]); cswap(key[2], key[6]); cswap(key[3], key[7]);
+                    cswap(key[2], key[4]); cswap(key[3], key[5]);
+                    cswap(key[1], key[2]); cswap(key[3], key[4]); cswap(key[5], key[6]);
+                    // the low 4 bits of each key, the nearest lowest
+                    list = 0;
 #pragma unroll
-                for (int c = 0; c < 8; ++c) key[c] = key[c] <= best_t ? key[c] : inf;
-                cswap(key[0], ref[0], key[1], ref[1]); cswap(key[2], ref[2], key[3], ref[3]);
-                cswap(key[4], ref[4], key[5], ref[5]); cswap(key[6], ref[6], key[7], ref[7]);
-                cswap(key[0], ref[0], key[2], ref[2]); cswap(key[1], ref[1], key[3], ref[3]);
-                cswap(key[4], ref[4], key[6], ref[6]); cswap(key[5], ref[5], key[7], ref[7]);
-                cswap(key[1], ref[1], key[2], ref[2]); cswap(key[5], ref[5], key[6], ref[6]);
-                cswap(key[0], ref[0], key[4], ref[4]); cswap(key[1], ref[1], key[5], ref[5]);
-                cswap(key[2], ref[2], key[6], ref[6]); cswap(key[3], ref[3], key[7], ref[7]);
-                cswap(key[2], ref[2], key[4], ref[4]); cswap(key[3], ref[3], key[5], ref[5]);
-                cswap(key[1], ref[1], key[2], ref[2]); cswap(key[3], ref[3], key[4], ref[4]);
-                cswap(key[5], ref[5], key[6], ref[6]);
-            }
-            // the nearest is entered, the others pushed far to near
-            bool have = false;
-            int next = 0;
-#pragma unroll
-            for (int c = 7; c >= 0; --c) {
-                if (key[c] != inf) {
-                    if (have) push(next);
-                    next = ref[c];
-                    have = true;
+                    for (int c = 0; c < 8; ++c) list = __builtin_amdgcn_alignbit((uint32_t)key[c], list, 4);
                 }
-            }
-            if (have) {
-                node = next;
-                continue;
-            }
-            if (!pop(node)) break;
-        }
-        if (overflowed) atomicOr(overflow, 1u);
-
-        uint32_t id0 = SGPU_INVALID_ID, id1 = SGPU_INVALID_ID;
-        const TriRecord* __restrict bt = tt;
-        if (!ANY && best_tri != 0xFFFFFFFFu && best_inst != SGPU_INVALID_ID) {
-            bt = ri[best_inst].tris;
-            if (inst_ids) {
-                id0 = inst_ids[2 * best_inst];
-                id1 = inst_ids[2 * best_inst + 1];
+                if (list) {
+                    if (glist) push(gbase, glist);
+                    gbase = base;
+                    glist = list;
+                }
+                node = kNext;
             }
         }
-        write_result<ANY>(i, hit_any, best_tri, best_t, best_u, best_v, bt, hits, occluded, id0, id1);
-        if (!ANY && comp_out) comp_out[i] = best_tri != 0xFFFFFFFFu ? best_inst : SGPU_INVALID_ID;
+        // the triangles found in a node come before the next node: leaving an instance changes the ray
+        if (active && pmask == 0 && node == kNext) advance();
+        if (active && pmask == 0 && node == -1) {
+            uint32_t id0 = SGPU_INVALID_ID, id1 = SGPU_INVALID_ID;
+            const WideNode* bw = rw;
+            if (INST && !ANY && best_tri != 0xFFFFFFFFu) {
+                if (best_inst != SGPU_INVALID_ID) {
+                    bw = (MULTI ? table[ray_scene[i]].insts : scene.insts)[best_inst].wide;
+                    if (inst_ids) {
+                        id0 = inst_ids[2 * best_inst];
+                        id1 = inst_ids[2 * best_inst + 1];
+                    }
+                } else {
+                    bw = MULTI ? table[ray_scene[i]].wide : scene.wide;
+                }
+            }
+            write_result<ANY>(i, hit_any, best_tri, best_t, best_u, best_v, reinterpret_cast<const TriRecord*>(bw), hits,
+                              occluded, id0, id1);
+            if (INST && !ANY && comp_out) comp_out[i] = best_tri != 0xFFFFFFFFu ? best_inst : SGPU_INVALID_ID;
+            active = false;
+        }
     }
     if (STATS) {
         atomicAdd(&stats[0], cnt_nodes);
@@ -759,44 +622,39 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) void k_trace8i(const WideNode* __
 
 }  // namespace
 
+namespace {
+
+__global__ void k_zero_work(uint32_t* __restrict w)
+{
+    if (threadIdx.x < kTraceWorkWords) w[threadIdx.x] = 0u;
+}
+
+// Words of a spill buffer for a grid of `threads` lanes: the ray counters, then each lane's stack
+// words past those in LDS.
+size_t spill_words(uint32_t stack_words, size_t threads)
+{
+    const uint32_t deep = stack_words > SGPU_STACK_LDS ? stack_words - SGPU_STACK_LDS : 1;
+    return kTraceWorkWords + deep * threads;
+}
+
+}  // namespace
+
+void sgpu_trace_work_zero(uint32_t* spill, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(kTraceWorkWords), 0, stream, spill);
+}
 
 namespace {
 
-template <bool ANY, bool STATS>
-void launch_trace(bool wide, bool multi, uint32_t blocks, hipStream_t stream, const BvhNode* nodes,
-                  const WideNode* wnodes, uint32_t n_top, const TriRecord* tris, uint32_t n_tris, const TraceScene* table,
-                  const uint32_t* ray_scene, const sgpu_rays_soa& rays, const sgpu_hits_soa& h, uint32_t* occluded,
-                  uint32_t n, const uint32_t* n_ptr, uint32_t* spill, uint32_t cap, unsigned long long* st,
-                  uint32_t* overflow, uint32_t* work)
-{
-    if (wide) {
-        sgpu_trace_work_zero(work, stream);
-        if (multi)
-            hipLaunchKernelGGL((k_trace8<ANY, STATS, true>), dim3(blocks), dim3(SGPU_TRACE_BLOCK), 0, stream, wnodes,
-                               n_top, tris, n_tris, table, ray_scene, rays, h, occluded, n, n_ptr, spill, cap, st, overflow,
-                               work);
-        else
-            hipLaunchKernelGGL((k_trace8<ANY, STATS, false>), dim3(blocks), dim3(SGPU_TRACE_BLOCK), 0, stream, wnodes,
-                               n_top, tris, n_tris, table, ray_scene, rays, h, occluded, n, n_ptr, spill, cap, st, overflow,
-                               work);
-    } else {
-        if (multi)
-            hipLaunchKernelGGL((k_trace<ANY, STATS, true>), dim3(blocks), dim3(SGPU_TRACE_BLOCK), 0, stream, nodes,
-                               tris, n_tris, table, ray_scene, rays, h, occluded, n, n_ptr, spill, cap, st, overflow);
-        else
-            hipLaunchKernelGGL((k_trace<ANY, STATS, false>), dim3(blocks), dim3(SGPU_TRACE_BLOCK), 0, stream, nodes,
-                               tris, n_tris, table, ray_scene, rays, h, occluded, n, n_ptr, spill, cap, st, overflow);
-    }
-}
-
-// One traversal launch over n rays: of one scene (its trees `nodes` / `wnodes`), or (table !=
-// nullptr) of the scenes of a batch, ray i in table[ray_scene[i]]; stack_cap bounds every scene's
-// stack. The context's trace_tree picks the tree kind.
-int trace_launch(sgpu_context ctx, const BvhNode* nodes, const WideNode* wnodes, uint32_t n_wide, const TriRecord* tris,
-                 uint32_t n_tris, uint32_t stack_cap, uint32_t* overflow, const TraceScene* table,
-                 const uint32_t* ray_scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded,
-                 uint32_t n, bool any_hit, uint64_t* d_stats, hipStream_t stream, uint32_t* spill_buf,
-                 const uint32_t* n_ptr, bool instanced = false, uint32_t* comp_out = nullptr, uint32_t cap_blocks = 0)
+// One traversal launch over n rays: of one scene (`scene`, its instances' ids `inst_ids`), or (table
+// != nullptr) of the scenes of a batch, ray i in table[ray_scene[i]]; stack_words bounds every
+// scene's stack. The context's trace_tree picks the tree kind; scenes of instances are walked on the
+// 8-wide one.
+int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, const uint32_t* inst_ids,
+                 uint32_t stack_words, uint32_t* overflow, const TraceScene* table, const uint32_t* ray_scene,
+                 const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded, uint32_t n, bool any_hit,
+                 uint64_t* d_stats, hipStream_t stream, uint32_t* spill_buf, const uint32_t* n_ptr, bool instanced,
+                 uint32_t* comp_out, uint32_t cap_blocks = 0)
 {
     if (n == 0) return SGPU_OK;
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
@@ -808,50 +666,55 @@ int trace_launch(sgpu_context ctx, const BvhNode* nodes, const WideNode* wnodes,
     // stream-ordered scratch for the spilled part of the stacks, private to this call, unless the
     // caller lends a buffer of sgpu_trace_spill_words (sized for the largest grid); its first
     // kTraceWorkWords words are the launch's ray counters (zero between launches)
-    uint32_t* spill = spill_buf;
-    if (!spill)
-        SGPU_HIP_TRY(hipMallocAsync((void**)&spill, sgpu_trace_spill_words(ctx, stack_cap) * sizeof(uint32_t), stream));
-    uint32_t* const buf = spill;
-    uint32_t* const work = spill;
-    spill += kTraceWorkWords;
+    uint32_t* buf = spill_buf;
+    if (!buf)
+        SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
+                                    spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) * sizeof(uint32_t), stream));
+    uint32_t* const work = buf;
+    uint32_t* const spill = buf + kTraceWorkWords;
     sgpu_hits_soa h = {};
     if (hits) h = *hits;
     unsigned long long* st = (unsigned long long*)d_stats;
     const bool multi = table != nullptr;
-    const bool wide = ctx->trace_tree == 1;
-    const uint32_t n_top = std::min(n_wide, std::min(ctx->trace_lds_nodes, kTopNodes));
-    if (multi && instanced) {
-        // a table with instanced scenes: k_trace8i walks both kinds of entry
-        const dim3 g(blocks), b(SGPU_TRACE_BLOCK);
-#define SGPU_LAUNCH_IM(A, S)                                                                                       \
-    hipLaunchKernelGGL((k_trace8i<A, S, true>), g, b, 0, stream, nullptr, nullptr, 0u, 0u, nullptr, nullptr, table, \
-                       ray_scene, *rays, h, occluded, n, n_ptr, spill, stack_cap, st, overflow, comp_out)
+    const dim3 g(blocks), b(SGPU_TRACE_BLOCK);
+    if (ctx->trace_tree == 0 && !instanced) {
+#define SGPU_LAUNCH_2(A, S, M)                                                                                      \
+    hipLaunchKernelGGL((k_trace<A, S, M>), g, b, 0, stream, scene.nodes,                      \
+                       reinterpret_cast<const TriRecord*>(scene.wide), scene.n_tris, table, ray_scene,            \
+                       *rays, h, occluded, n, n_ptr, spill, stack_words, st, overflow)
         if (any_hit) {
-            if (st) SGPU_LAUNCH_IM(true, true);
-            else SGPU_LAUNCH_IM(true, false);
+            if (st) { if (multi) SGPU_LAUNCH_2(true, true, true); else SGPU_LAUNCH_2(true, true, false); }
+            else { if (multi) SGPU_LAUNCH_2(true, false, true); else SGPU_LAUNCH_2(true, false, false); }
         } else {
-            if (st) SGPU_LAUNCH_IM(false, true);
-            else SGPU_LAUNCH_IM(false, false);
+            if (st) { if (multi) SGPU_LAUNCH_2(false, true, true); else SGPU_LAUNCH_2(false, true, false); }
+            else { if (multi) SGPU_LAUNCH_2(false, false, true); else SGPU_LAUNCH_2(false, false, false); }
         }
-#undef SGPU_LAUNCH_IM
-        SGPU_HIP_TRY(hipGetLastError());
-        if (!spill_buf) SGPU_HIP_TRY(hipFreeAsync(buf, stream));
-        return SGPU_OK;
-    }
-    if (any_hit) {
-        if (st)
-            launch_trace<true, true>(wide, multi, blocks, stream, nodes, wnodes, n_top, tris, n_tris, table, ray_scene, *rays,
-                                     h, occluded, n, n_ptr, spill, stack_cap, st, overflow, work);
-        else
-            launch_trace<true, false>(wide, multi, blocks, stream, nodes, wnodes, n_top, tris, n_tris, table, ray_scene, *rays,
-                                      h, occluded, n, n_ptr, spill, stack_cap, st, overflow, work);
+#undef SGPU_LAUNCH_2
     } else {
-        if (st)
-            launch_trace<false, true>(wide, multi, blocks, stream, nodes, wnodes, n_top, tris, n_tris, table, ray_scene, *rays,
-                                      h, occluded, n, n_ptr, spill, stack_cap, st, overflow, work);
-        else
-            launch_trace<false, false>(wide, multi, blocks, stream, nodes, wnodes, n_top, tris, n_tris, table, ray_scene,
-                                       *rays, h, occluded, n, n_ptr, spill, stack_cap, st, overflow, work);
+        // top nodes in LDS: single-scene launches over geometries
+        const uint32_t n_top = multi || instanced ? 0u : std::min(n_wide, std::min(ctx->trace_lds_nodes, kTopNodes));
+        // the launch's ray counter, where the grid does not hold every ray at once
+        if (blocks < (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK) sgpu_trace_work_zero(work, stream);
+#define SGPU_LAUNCH_8(A, S, M, I, T)                                                                               \
+    hipLaunchKernelGGL((k_trace8<A, S, M, I, T>), g, b, 0, stream, scene, inst_ids, table, ray_scene, *rays, h,    \
+                       occluded, n, n_ptr, (uint2*)spill, stack_words / 2, st, overflow, work, comp_out, n_top)
+#define SGPU_LAUNCH_8S(A, S)                                                                                      \
+    do {                                                                                                          \
+        if (multi && instanced) SGPU_LAUNCH_8(A, S, true, true, false);                                           \
+        else if (multi) SGPU_LAUNCH_8(A, S, true, false, false);                                                  \
+        else if (instanced) SGPU_LAUNCH_8(A, S, false, true, false);                                              \
+        else if (n_top) SGPU_LAUNCH_8(A, S, false, false, true);                                                  \
+        else SGPU_LAUNCH_8(A, S, false, false, false);                                                            \
+    } while (0)
+        if (any_hit) {
+            if (st) SGPU_LAUNCH_8S(true, true);
+            else SGPU_LAUNCH_8S(true, false);
+        } else {
+            if (st) SGPU_LAUNCH_8S(false, true);
+            else SGPU_LAUNCH_8S(false, false);
+        }
+#undef SGPU_LAUNCH_8S
+#undef SGPU_LAUNCH_8
     }
     SGPU_HIP_TRY(hipGetLastError());
     if (!spill_buf) SGPU_HIP_TRY(hipFreeAsync(buf, stream));
@@ -860,84 +723,25 @@ int trace_launch(sgpu_context ctx, const BvhNode* nodes, const WideNode* wnodes,
 
 }  // namespace
 
-size_t sgpu_trace_spill_words(sgpu_context ctx, uint32_t stack_cap)
+size_t sgpu_trace_spill_words(sgpu_context ctx, uint32_t stack_words)
 {
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    const uint32_t threads = cus * kMaxTraceBlocksPerCu * SGPU_TRACE_BLOCK;
-    const uint32_t spill_depth = stack_cap > SGPU_STACK_LDS ? stack_cap - SGPU_STACK_LDS : 1;
-    return kTraceWorkWords + (size_t)spill_depth * threads;
-}
-
-namespace {
-__global__ void k_zero_work(uint32_t* __restrict w)
-{
-    if (threadIdx.x < kTraceWorkWords) w[threadIdx.x] = 0u;
-}
-}  // namespace
-
-void sgpu_trace_work_zero(uint32_t* spill, hipStream_t stream)
-{
-    hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(kTraceWorkWords), 0, stream, spill);
+    return spill_words(stack_words, (size_t)cus * kMaxTraceBlocksPerCu * SGPU_TRACE_BLOCK);
 }
 
 size_t sgpu_trace_spill_words(sgpu_scene scene) { return sgpu_trace_spill_words(scene->ctx, scene->stack_cap); }
-
-namespace {
-
-// One traversal launch over the rays of an instanced scene (k_trace8i).
-int trace_launch_instanced(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded,
-                           uint32_t n, bool any_hit, uint64_t* d_stats, hipStream_t stream, uint32_t* overflow,
-                           uint32_t* spill_buf, const uint32_t* n_ptr, uint32_t* comp_out, uint32_t cap_blocks)
-{
-    if (n == 0) return SGPU_OK;
-    sgpu_context ctx = scene->ctx;
-    const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    uint32_t blocks = (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK;
-    uint32_t max_blocks = cus * std::min(ctx->trace_blocks_per_cu, kMaxTraceBlocksPerCu);
-    if (cap_blocks && max_blocks > cap_blocks) max_blocks = cap_blocks;
-    if (blocks > max_blocks) blocks = max_blocks;
-    uint32_t* spill = spill_buf;
-    if (!spill)
-        SGPU_HIP_TRY(hipMallocAsync((void**)&spill, sgpu_trace_spill_words(ctx, scene->stack_cap) * sizeof(uint32_t),
-                                    stream));
-    uint32_t* const buf = spill;
-    spill += kTraceWorkWords;  // the counter words (unused by the instanced traversal) precede the spill
-    sgpu_hits_soa h = {};
-    if (hits) h = *hits;
-    unsigned long long* st = (unsigned long long*)d_stats;
-    const dim3 g(blocks), b(SGPU_TRACE_BLOCK);
-#define SGPU_LAUNCH_I(A, S)                                                                                        \
-    hipLaunchKernelGGL((k_trace8i<A, S, false>), g, b, 0, stream, scene->d_wide, nullptr, 0u, scene->n_inst,      \
-                       scene->d_inst, scene->d_inst_ids, nullptr, nullptr, *rays, h, occluded, n, n_ptr, spill,    \
-                       scene->stack_cap, st, overflow, comp_out)
-    if (any_hit) {
-        if (st) SGPU_LAUNCH_I(true, true);
-        else SGPU_LAUNCH_I(true, false);
-    } else {
-        if (st) SGPU_LAUNCH_I(false, true);
-        else SGPU_LAUNCH_I(false, false);
-    }
-#undef SGPU_LAUNCH_I
-    SGPU_HIP_TRY(hipGetLastError());
-    if (!spill_buf) SGPU_HIP_TRY(hipFreeAsync(buf, stream));
-    return SGPU_OK;
-}
-
-}  // namespace
 
 int sgpu_trace_launch(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded,
                       uint32_t n, bool any_hit, uint64_t* d_stats, hipStream_t stream, uint32_t* spill_buf,
                       const uint32_t* n_ptr, uint32_t* overflow, uint32_t* comp_out, uint32_t max_blocks,
                       uint64_t* curve_stats)
 {
-    int rc;
-    if (!scene->instances.empty())
-        rc = trace_launch_instanced(scene, rays, hits, occluded, n, any_hit, d_stats, stream,
-                                    overflow ? overflow : scene->d_overflow, spill_buf, n_ptr, comp_out, max_blocks);
-    else
-        rc = trace_launch(scene->ctx, scene->d_nodes, scene->d_wide, scene->n_wide, scene->d_tris, scene->n_tris,
-                          scene->stack_cap, overflow ? overflow : scene->d_overflow, nullptr, nullptr, rays, hits,
-                          occluded, n, any_hit, d_stats, stream, spill_buf, n_ptr, false, nullptr, max_blocks);
+    const TraceScene ts{scene->d_nodes, scene->d_wide,   scene->n_tris,   scene->n_inst,
+                        scene->d_inst,  scene->d_cnodes, scene->d_curves, scene->n_curves};
+    const int rc = trace_launch(scene->ctx, ts, scene->n_wide, scene->d_inst_ids, scene->stack_cap,
+                                overflow ? overflow : scene->d_overflow, nullptr, nullptr, rays, hits, occluded, n,
+                                any_hit, d_stats, stream, spill_buf, n_ptr, !scene->instances.empty(), comp_out,
+                                max_blocks);
     if (rc != SGPU_OK || scene->n_curves == 0) return rc;
     return sgpu_curve_launch(scene->d_cnodes, scene->d_curves, scene->n_curves, scene->d_inst, scene->d_inst_ids,
                              nullptr, nullptr, rays, hits, occluded, n, any_hit, n_ptr, comp_out,
@@ -950,8 +754,8 @@ int sgpu_trace_launch_multi(sgpu_context ctx, const TraceScene* table, const uin
                             uint32_t* spill_buf, const uint32_t* n_ptr, bool instanced, uint32_t* comp_out,
                             bool curves)
 {
-    int rc = trace_launch(ctx, nullptr, nullptr, 0, nullptr, 0, stack_cap, overflow, table, ray_scene, rays, hits,
-                          occluded, n, any_hit, d_stats, stream, spill_buf, n_ptr, instanced, comp_out);
+    const int rc = trace_launch(ctx, TraceScene{}, 0, nullptr, stack_cap, overflow, table, ray_scene, rays, hits, occluded,
+                                n, any_hit, d_stats, stream, spill_buf, n_ptr, instanced, comp_out);
     if (rc != SGPU_OK || !curves) return rc;
     return sgpu_curve_launch(nullptr, nullptr, 0, nullptr, nullptr, table, ray_scene, rays, hits, occluded, n, any_hit,
                              n_ptr, comp_out, overflow, stream);

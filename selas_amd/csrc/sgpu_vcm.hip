@@ -1103,7 +1103,7 @@ struct sgpu_vcm_server_s {
     uint32_t* h = nullptr;
     Slice* h_slices = nullptr;
     TraceScene* h_table = nullptr;
-    bool any_instanced = false;  // an instanced scene is in the table (traversal by k_trace8i)
+    bool any_instanced = false;  // an instanced scene is in the table (traversed by the instanced kernels)
     bool any_curves = false;     // a scene of the table has curves (the curve pass follows traversal)
     // the scenes of the admitted jobs (traversal table, rebuilt at every step) and their unique
     // ids, jobs in admission order
@@ -1337,9 +1337,9 @@ int server_upload_table(sgpu_vcm_server sv, hipStream_t stream)
         SGPU_HIP_TRY(hipHostMalloc((void**)&sv->h_table, sizeof(TraceScene) * sv->table_cap, hipHostMallocDefault));
     }
     for (uint32_t k = 0; k < n; ++k)
-        sv->h_table[k] = TraceScene{sv->scenes[k]->d_nodes,  sv->scenes[k]->d_wide,   sv->scenes[k]->d_tris,
-                                    sv->scenes[k]->n_tris,   sv->scenes[k]->n_inst,   sv->scenes[k]->d_inst,
-                                    sv->scenes[k]->d_cnodes, sv->scenes[k]->d_curves, sv->scenes[k]->n_curves};
+        sv->h_table[k] = TraceScene{sv->scenes[k]->d_nodes, sv->scenes[k]->d_wide, sv->scenes[k]->n_tris,
+                                    sv->scenes[k]->n_inst,  sv->scenes[k]->d_inst, sv->scenes[k]->d_cnodes,
+                                    sv->scenes[k]->d_curves, sv->scenes[k]->n_curves};
     SGPU_HIP_TRY(hipMemcpyAsync(sv->d_table, sv->h_table, sizeof(TraceScene) * n, hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     sv->table_dirty = false;
