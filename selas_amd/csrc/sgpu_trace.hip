@@ -19,8 +19,9 @@
 
 namespace {
 
-__device__ __forceinline__ bool tri_test(const TriRecord& r, const f3& o, const f3& d, float tnear, float& t,
-                                         float& u, float& v)
+// The test but for the barycentrics' divisions: u = U / a, v = V / a of the hit kept in the end.
+__device__ __forceinline__ bool tri_hit(const TriRecord& r, const f3& o, const f3& d, float tnear, float& t, float& U,
+                                        float& V, float& a)
 {
     f3 v0 = mk3(r.a.x, r.a.y, r.a.z);
     f3 e1 = mk3(r.b.x, r.b.y, r.b.z);
@@ -28,9 +29,9 @@ __device__ __forceinline__ bool tri_test(const TriRecord& r, const f3& o, const 
     f3 pvec = cross_fma(d, e2);
     float det = dot_fma(e1, pvec);
     f3 tvec = o - v0;
-    float U = dot_fma(tvec, pvec);
+    U = dot_fma(tvec, pvec);
     f3 qvec = cross_fma(tvec, e1);
-    float V = dot_fma(d, qvec);
+    V = dot_fma(d, qvec);
     float T = dot_fma(e2, qvec);
     if (det == 0.0f) return false;
     if (det < 0.0f) {
@@ -38,10 +39,17 @@ __device__ __forceinline__ bool tri_test(const TriRecord& r, const f3& o, const 
         V = -V;
         T = -T;
     }
-    float a = fabsf(det);
+    a = fabsf(det);
     if (!(U >= 0.0f && V >= 0.0f && U + V <= a)) return false;
     t = T / a;
-    if (!(t > tnear)) return false;
+    return t > tnear;
+}
+
+__device__ __forceinline__ bool tri_test(const TriRecord& r, const f3& o, const f3& d, float tnear, float& t,
+                                         float& u, float& v)
+{
+    float U, V, a;
+    if (!tri_hit(r, o, d, tnear, t, U, V, a)) return false;
     u = U / a;
     v = V / a;
     return true;
@@ -252,6 +260,11 @@ __device__ __forceinline__ void cswap(int& a, int& b)
 // nearly every ray. Measured on MI355X they hit in L1/L2 anyway, and the LDS branch costs 1-3 %.
 constexpr uint32_t kTopNodes = 9;
 constexpr uint32_t kTraceChunk = 64;  // rays a wave takes from the launch's counter at a time
+// Finished lanes for which a wave stops to write results and take rays (16M closest-hit rays in 2M
+// triangles: 12.1 ms at 1, 10.9 at 4, 10.6 at 8, 10.3 at 16 and 24; 4M any-hit rays 1.83, 1.72, 1.69,
+// 1.71, 1.78 ms).
+template <bool ANY>
+constexpr int kRefill = ANY ? 8 : 16;
 constexpr int kNext = -2;             // a lane that takes its next node once its triangles are tested
 
 // 8-wide traversal of the collapsed tree (WideNode), one ray per lane. In a trip of the wave's loop
@@ -284,11 +297,11 @@ constexpr int kNext = -2;             // a lane that takes its next node once it
 // chunk at once, so lanes do not wait for the wave's longest ray; a wave whose chunk is used up
 // takes the next from a counter, so waves do not wait for the launch's longest chunk.
 //
-// Bound by vector instructions now (81 % of the issue cycles on the traversal workload, address unit
-// 69 %); 32 KB of LDS a block allow 5 waves per SIMD. Against the version that read nodes and triangles
-// lane by lane, sorted (distance, child) pairs and kept a stack of children: 16M rays in 2M triangles
-// 15.3 -> 12.1 ms, 4M shadow rays in 1M triangles 2.67 -> 1.83 ms, 250K rays 0.62 -> 0.44 ms, 4M rays
-// through 256 instances (which had no refill) 10.1 -> 3.74 ms; hits the same bits.
+// Bound by vector instructions (81 % of the issue cycles on the traversal workload with kRefill = 1,
+// address unit 69 %); 32 KB of LDS a block allow 5 waves per SIMD. Against the version that read nodes
+// and triangles lane by lane, sorted (distance, child) pairs and kept a stack of children: 16M rays in
+// 2M triangles 15.2 -> 10.4 ms, 4M shadow rays in 1M triangles 2.66 -> 1.71 ms, 250K rays 0.62 -> 0.40
+// ms, 4M rays through 256 instances (which had no refill) 9.8 -> 3.14 ms; hits the same bits.
 template <bool ANY, bool STATS, bool MULTI, bool INST, bool TOP>
 __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace8(
     TraceScene scene, const uint32_t* __restrict inst_ids, const TraceScene* __restrict table,
@@ -327,7 +340,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
     float tnear = 0.0f;
     float best_t = 0.0f;  // the any-hit query's tfar
     uint32_t best_key = 0xFFFFFFFFu, best_tri = 0xFFFFFFFFu, best_inst = SGPU_INVALID_ID;
-    float best_u = 0.0f, best_v = 0.0f;
+    float best_u = 0.0f, best_v = 0.0f, best_a = 1.0f;  // u and v times the hit's |det|, and that
     bool hit_any = false;
     const WideNode* rw = scene.wide;
     uint32_t cur = SGPU_INVALID_ID;  // INST: the instance being walked (none: the top tree)
@@ -396,57 +409,83 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
     };
 
     for (;;) {
-        // lanes without a ray take the next rays of the chunk (a new chunk when it is used up)
-        const unsigned long long idle = __ballot(!active);
-        if (idle && next >= end && !drained) {
-            if (grid_rays >= n) {
-                drained = true;  // the first chunks held every ray
-            } else {
-                uint32_t base = 0;
-                if ((threadIdx.x & 63u) == 0) base = grid_rays + atomicAdd(&work[0], kTraceChunk);
-                base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-                if (base >= n) {
-                    drained = true;
+        // Finished rays are written and their lanes take the next rays of the chunk (a new chunk when it
+        // is used up) kRefill at a time: the work of that is a hundred instructions of the wave, and
+        // nearly every trip has a lane or two that are done.
+        const bool done = pmask == 0 && node == -1;
+        const unsigned long long finished = __ballot(active && done), free_lanes = __ballot(done);
+        if (free_lanes == ~0ull || __popcll(drained ? finished : free_lanes) >= kRefill<ANY>) {
+            if (active && done) {
+                uint32_t id0 = SGPU_INVALID_ID, id1 = SGPU_INVALID_ID;
+                const WideNode* bw = rw;
+                if (INST && !ANY && best_tri != 0xFFFFFFFFu) {
+                    if (best_inst != SGPU_INVALID_ID) {
+                        bw = (MULTI ? table[ray_scene[i]].insts : scene.insts)[best_inst].wide;
+                        if (inst_ids) {
+                            id0 = inst_ids[2 * best_inst];
+                            id1 = inst_ids[2 * best_inst + 1];
+                        }
+                    } else {
+                        bw = MULTI ? table[ray_scene[i]].wide : scene.wide;
+                    }
+                }
+                write_result<ANY>(i, hit_any, best_tri, best_t, best_u / best_a, best_v / best_a,
+                                  reinterpret_cast<const TriRecord*>(bw), hits, occluded, id0, id1);
+                if (INST && !ANY && comp_out) comp_out[i] = best_tri != 0xFFFFFFFFu ? best_inst : SGPU_INVALID_ID;
+                active = false;
+            }
+            const unsigned long long idle = free_lanes;
+            if (next >= end && !drained) {
+                if (grid_rays >= n) {
+                    drained = true;  // the first chunks held every ray
                 } else {
-                    next = base;
-                    end = min(n, base + kTraceChunk);
+                    uint32_t base = 0;
+                    if ((threadIdx.x & 63u) == 0) base = grid_rays + atomicAdd(&work[0], kTraceChunk);
+                    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                    if (base >= n) {
+                        drained = true;
+                    } else {
+                        next = base;
+                        end = min(n, base + kTraceChunk);
+                    }
                 }
             }
-        }
-        if (idle && next < end) {
-            const uint32_t r = next + (uint32_t)__popcll(idle & below);
-            if (!active && r < end) {
-                i = r;
-                active = true;
-                load_ray(true);
-                set_slopes();
-                bool walk;
-                if (MULTI) {
-                    const TraceScene ts = table[ray_scene[i]];
-                    rw = ts.wide;
-                    walk = ts.n_tris > 0 || (INST && ts.n_inst > 0);
-                } else {
-                    rw = scene.wide;
-                    walk = scene.n_tris > 0 || (INST && scene.n_inst > 0);
+            if (next < end) {
+                const uint32_t r = next + (uint32_t)__popcll(idle & below);
+                if (!active && r < end) {
+                    i = r;
+                    active = true;
+                    load_ray(true);
+                    set_slopes();
+                    bool walk;
+                    if (MULTI) {
+                        const TraceScene ts = table[ray_scene[i]];
+                        rw = ts.wide;
+                        walk = ts.n_tris > 0 || (INST && ts.n_inst > 0);
+                    } else {
+                        rw = scene.wide;
+                        walk = scene.n_tris > 0 || (INST && scene.n_inst > 0);
+                    }
+                    best_key = 0xFFFFFFFFu;
+                    best_tri = 0xFFFFFFFFu;
+                    best_inst = SGPU_INVALID_ID;
+                    best_u = 0.0f;
+                    best_v = 0.0f;
+                    best_a = 1.0f;
+                    hit_any = false;
+                    sp = 0;
+                    glist = 0;
+                    pmask = 0;
+                    cur = SGPU_INVALID_ID;
+                    node = walk ? 0 : -1;
                 }
-                best_key = 0xFFFFFFFFu;
-                best_tri = 0xFFFFFFFFu;
-                best_inst = SGPU_INVALID_ID;
-                best_u = 0.0f;
-                best_v = 0.0f;
-                hit_any = false;
-                sp = 0;
-                glist = 0;
-                pmask = 0;
-                cur = SGPU_INVALID_ID;
-                node = walk ? 0 : -1;
+                next = min(end, next + (uint32_t)__popcll(idle));
             }
-            next = min(end, next + (uint32_t)__popcll(idle));
+            if (__ballot(active) == 0) break;
         }
-        if (__ballot(active) == 0) break;
 
-        const bool test = active && pmask != 0;
-        const bool visit = active && pmask == 0 && node >= 0;
+        const bool test = pmask != 0;
+        const bool visit = pmask == 0 && node >= 0;
         int slot = visit ? node : -1;
         if (test) {
             const uint32_t k = (uint32_t)__builtin_ctz(pmask);
@@ -492,8 +531,8 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
             r.b = make_float4(__uint_as_float(w1.x), __uint_as_float(w1.y), __uint_as_float(w1.z), __uint_as_float(w1.w));
             r.c = make_float4(__uint_as_float(w2.x), __uint_as_float(w2.y), __uint_as_float(w2.z), __uint_as_float(w2.w));
             if (STATS) ++cnt_tris;
-            float t, u, v;
-            if (tri_test(r, o, d, tnear, t, u, v)) {
+            float t, U, V, a;
+            if (tri_hit(r, o, d, tnear, t, U, V, a)) {
                 if (ANY) {
                     if (t <= best_t) {
                         hit_any = true;
@@ -508,8 +547,9 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
                         best_key = key;
                         best_tri = (uint32_t)slot;
                         if (INST) best_inst = cur;
-                        best_u = u;
-                        best_v = v;
+                        best_u = U;
+                        best_v = V;
+                        best_a = a;
                     }
                 }
             }
@@ -550,7 +590,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
                 int key[8];
                 uint32_t hit = 0;
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
+                for (int c = 7; c >= 0; --c) {
                     const int sh = 8 * (c & 3), wi = c >> 2;
                     const float t0x = fmaf((float)((nx[wi] >> sh) & 0xFFu), ax, bx);
                     const float t0y = fmaf((float)((ny[wi] >> sh) & 0xFFu), ay, by);
@@ -561,7 +601,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
                     const float tmin = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tnear));
                     const float tmax = fminf(fminf(t1x, t1y), fminf(t1z, best_t));
                     const bool in = tmin <= tmax;
-                    hit |= in ? 1u << c : 0u;
+                    hit = hit + hit + (in ? 1u : 0u);
                     // internal children: entry distance as the sort key, the slot (and 8) in its low bits
                     if (!ANY) key[c] = in && (uint32_t)c < ni ? (__float_as_int(tmin) & ~15) | (8 | c) : 0x7FFFFFF0;
                 }
@@ -593,26 +633,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
             }
         }
         // the triangles found in a node come before the next node: leaving an instance changes the ray
-        if (active && pmask == 0 && node == kNext) advance();
-        if (active && pmask == 0 && node == -1) {
-            uint32_t id0 = SGPU_INVALID_ID, id1 = SGPU_INVALID_ID;
-            const WideNode* bw = rw;
-            if (INST && !ANY && best_tri != 0xFFFFFFFFu) {
-                if (best_inst != SGPU_INVALID_ID) {
-                    bw = (MULTI ? table[ray_scene[i]].insts : scene.insts)[best_inst].wide;
-                    if (inst_ids) {
-                        id0 = inst_ids[2 * best_inst];
-                        id1 = inst_ids[2 * best_inst + 1];
-                    }
-                } else {
-                    bw = MULTI ? table[ray_scene[i]].wide : scene.wide;
-                }
-            }
-            write_result<ANY>(i, hit_any, best_tri, best_t, best_u, best_v, reinterpret_cast<const TriRecord*>(bw), hits,
-                              occluded, id0, id1);
-            if (INST && !ANY && comp_out) comp_out[i] = best_tri != 0xFFFFFFFFu ? best_inst : SGPU_INVALID_ID;
-            active = false;
-        }
+        if (pmask == 0 && node == kNext) advance();
     }
     if (STATS) {
         atomicAdd(&stats[0], cnt_nodes);
