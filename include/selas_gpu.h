@@ -99,8 +99,10 @@ const char* sgpu_last_error(void);
 
 /* ---- context (replaces rtcNewDevice / rtcReleaseDevice, Source/Applications/Selas/Source/main.cpp:99)
  * A context keeps device memory between calls: the stream-ordered pool of its device holds freed
- * memory for reuse, and the VCM wavefront buffers of the last sgpu_render_vcm(_batch) call stay
- * allocated until a call needs larger ones or the context is destroyed. */
+ * memory for reuse, the VCM wavefront buffers of the last sgpu_render_vcm(_batch) call stay
+ * allocated until a call needs larger ones or the context is destroyed, and up to 2 GiB of idle
+ * scratch blocks of commits and path-traced renders stay until the context is destroyed (or
+ * sgpu_malloc needs the memory). */
 int sgpu_context_create(int device, sgpu_context* out);
 int sgpu_context_destroy(sgpu_context ctx);
 

@@ -459,8 +459,7 @@ __global__ __launch_bounds__(kBlock) void k_depth(int n, const int* __restrict p
 // of largest surface area (the first such child on ties) until it has 8 children or only leaves.
 // A task is a binary node and the slot its wide node goes to. k_wide_expand writes each task's
 // children (binary refs and boxes) and the counts of its internal children and of the slots its
-// children take; an exclusive scan of those counts numbers the next level's tasks and slots in task
-// order, so the numbering (and the tree) is deterministic and a node's children are contiguous;
+// children take; a scan of those counts numbers the next level's tasks and slots in task order, so the numbering (and the tree) is deterministic and a node's children are contiguous;
 // k_wide_emit quantizes the boxes and writes the node's first slot (internal children first), the
 // next level's tasks and the leaves' slots. In the top tree of an instanced scene leaves are nodes
 // too: a task ~k stands for leaf k, whose node is its instance's (InstNode). A node has 8 children
@@ -571,7 +570,8 @@ struct NodeSlot {
 template <bool TOP>
 __global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t level_base, uint32_t slot_base,
                                                       const WideTask* __restrict tasks,
-                                                      const uint64_t* __restrict offsets, const int* __restrict cref,
+                                                      const uint64_t* __restrict ends, const uint64_t* __restrict counts,
+                                                      const int* __restrict cref,
                                                       const float* __restrict cbox, const uint32_t* __restrict nchild,
                                                       NodeSlot* __restrict out, uint32_t* __restrict out_slot,
                                                       WideTask* __restrict next_tasks,
@@ -600,7 +600,8 @@ __global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t
             lo[a] = fminf(lo[a], B[6 * k + a]);
             hi[a] = fmaxf(hi[a], B[6 * k + 3 + a]);
         }
-    const uint32_t base = slot_base + (uint32_t)(offsets[t] >> 32);
+    const uint64_t offset = ends[t] - counts[t];
+    const uint32_t base = slot_base + (uint32_t)(offset >> 32);
     uint32_t meta = ni << 24 | m << 28;
     for (int a = 0; a < 3; ++a) {
         const float og = origin_floor(lo[a]);
@@ -632,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t
         }
     }
     w.w[3] = meta;
-    const uint32_t task_off = (uint32_t)(offsets[t] & 0xFFFFFFFFull);
+    const uint32_t task_off = (uint32_t)(offset & 0xFFFFFFFFull);
     for (uint32_t k = 0; k < m; ++k) {
         const int r = cref[8 * (size_t)t + k];
         if (k < ni)
@@ -675,20 +676,27 @@ __global__ __launch_bounds__(kBlock) void k_relabel(BvhNode* __restrict nodes, u
     nodes[i].child = c;
 }
 
+// An array in the build's scratch.
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
-    hipError_t alloc(size_t count) { return hipMalloc((void**)&p, count * sizeof(T) + 16); }
-    ~DevBuf()
+    hipError_t alloc(sgpu_scratch& s, size_t count)
     {
-        if (p) (void)hipFree(p);
+        p = s.get<T>(count);
+        return s.err;
     }
 };
+
+// Scratch bytes a build over n primitives takes: per primitive the records (64 for triangles, 80 for
+// curves), boxes and centroid (48), positions (40), codes and order (28), parents (8), the box pyramid
+// (64), the 8-wide tree's tasks (4/7 nodes of 348) and the sorts' own; in a top tree or with PLOC more,
+// taken as needed.
+size_t build_scratch(size_t n) { return 500 * n + ((size_t)1 << 20); }
 
 // Collapses the binary tree (nodes, root 0, over n leaves) into the scene's 8-wide tree, with the
 // triangle records rec[order[j]] of its leaves j. The top tree of an instanced scene passes its
 // instance records instead of triangles (order[j]: the instance of leaf j): its leaves become nodes.
-int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
+int build_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
                const TriRecord* rec, const InstRecord* insts)
 {
     const bool top = insts != nullptr;
@@ -701,21 +709,21 @@ int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream,
     DevBuf<uint64_t> d_cnt, d_off;
     DevBuf<NodeSlot> d_all;
     DevBuf<uint8_t> d_tmp;
-    SGPU_HIP_TRY(d_tasks.alloc(max_nodes));
-    SGPU_HIP_TRY(d_next.alloc(max_nodes));
-    SGPU_HIP_TRY(d_cref.alloc(8 * max_nodes));
-    SGPU_HIP_TRY(d_cbox.alloc(48 * max_nodes));
-    SGPU_HIP_TRY(d_nch.alloc(max_nodes));
-    SGPU_HIP_TRY(d_cnt.alloc(max_nodes));
-    SGPU_HIP_TRY(d_off.alloc(max_nodes));
-    SGPU_HIP_TRY(d_bad.alloc(1));
-    SGPU_HIP_TRY(d_all.alloc(max_nodes));
-    SGPU_HIP_TRY(d_slot.alloc(max_nodes));
-    SGPU_HIP_TRY(d_leaf_slot.alloc(n_leaves));
+    SGPU_HIP_TRY(d_tasks.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_next.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_cref.alloc(S, 8 * max_nodes));
+    SGPU_HIP_TRY(d_cbox.alloc(S, 48 * max_nodes));
+    SGPU_HIP_TRY(d_nch.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_cnt.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_off.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_bad.alloc(S, 1));
+    SGPU_HIP_TRY(d_all.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_slot.alloc(S, max_nodes));
+    SGPU_HIP_TRY(d_leaf_slot.alloc(S, n_leaves));
     size_t tmp_bytes = 0;
-    SGPU_HIP_TRY(rocprim::exclusive_scan(nullptr, tmp_bytes, d_cnt.p, d_off.p, (uint64_t)0, max_nodes,
-                                         rocprim::plus<uint64_t>(), stream));
-    SGPU_HIP_TRY(d_tmp.alloc(tmp_bytes));
+    SGPU_HIP_TRY(rocprim::inclusive_scan(nullptr, tmp_bytes, d_cnt.p, d_off.p, max_nodes, rocprim::plus<uint64_t>(),
+                                         stream));
+    SGPU_HIP_TRY(d_tmp.alloc(S, tmp_bytes));
     const WideTask root{0, 0};
     SGPU_HIP_TRY(hipMemcpyAsync(d_tasks.p, &root, sizeof(root), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemsetAsync(d_bad.p, 0, sizeof(uint32_t), stream));
@@ -730,24 +738,22 @@ int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream,
             hipLaunchKernelGGL(k_wide_expand<false>, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes,
                                d_cref.p, d_cbox.p, d_nch.p, d_cnt.p);
         SGPU_HIP_TRY(hipGetLastError());
-        SGPU_HIP_TRY(rocprim::exclusive_scan(d_tmp.p, tmp_bytes, d_cnt.p, d_off.p, (uint64_t)0, (size_t)n_tasks,
+        SGPU_HIP_TRY(rocprim::inclusive_scan(d_tmp.p, tmp_bytes, d_cnt.p, d_off.p, (size_t)n_tasks,
                                              rocprim::plus<uint64_t>(), stream));
-        uint64_t last[2] = {0, 0};
-        SGPU_HIP_TRY(hipMemcpyAsync(&last[0], d_off.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-        SGPU_HIP_TRY(hipMemcpyAsync(&last[1], d_cnt.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_off.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
         SGPU_HIP_TRY(hipStreamSynchronize(stream));
-        const uint64_t total = last[0] + last[1];
+        const uint64_t total = S.pinned()[0];
         const uint32_t n_next = (uint32_t)(total & 0xFFFFFFFFull), n_new = (uint32_t)(total >> 32);
         if ((uint64_t)level_base + n_tasks + n_next > max_nodes)
             return sgpu_fail(SGPU_E_STATE, "wide tree larger than its bound");
         if (slot_base + n_new > 0x7FFFFFFFull) return sgpu_fail(SGPU_E_RANGE, "wide tree takes more than 2^31 slots");
         if (top)
             hipLaunchKernelGGL(k_wide_emit<true>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
-                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
+                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
                                d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
         else
             hipLaunchKernelGGL(k_wide_emit<false>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
-                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
+                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
                                d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
         SGPU_HIP_TRY(hipGetLastError());
         std::swap(d_tasks.p, d_next.p);
@@ -756,10 +762,9 @@ int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream,
         n_tasks = n_next;
         ++depth;
     }
-    uint32_t bad = 0;
-    SGPU_HIP_TRY(hipMemcpyAsync(&bad, d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+    SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
-    if (bad) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
+    if (*(const uint32_t*)S.pinned()) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
     SGPU_HIP_TRY(hipMalloc((void**)&scene->d_wide, slot_base * kSlotBytes));
     scene->n_slots = (uint32_t)slot_base;
     scene->n_wide = level_base;
@@ -782,9 +787,10 @@ int build_wide(sgpu_scene scene, BvhNode* nodes, uint32_t n, hipStream_t stream,
     return SGPU_OK;
 }
 
-// Words of traversal stack a scene's trees can need: the binary one a word per level, the 8-wide one
-// an entry of two words per level.
-uint32_t tree_stack_words(uint32_t depth, uint32_t wide_depth) { return std::max(depth + 1, 2 * (wide_depth + 1)); }
+// Words of traversal stack an 8-wide tree of `levels` levels can need: an entry of two words for every
+// node above the walked one's parent (whose group is in registers) but the root's level and the last,
+// whose nodes have no nodes below.
+uint32_t wide_stack_words(uint32_t levels) { return levels > 2 ? 2 * (levels - 2) : 0; }
 
 }  // namespace
 
@@ -809,7 +815,7 @@ uint32_t host_f2ord(float f)
 // leaves them): Morton codes, radix sort, Karras hierarchy, bottom-up fit. On success *nodes_out
 // holds max(n - 1, 1) nodes, d_order the primitive of each leaf in leaf order and *depth the
 // deepest leaf.
-int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const float4* d_cent, const uint32_t* d_bounds,
+int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4* d_bhi, const float4* d_cent, const uint32_t* d_bounds,
                  hipStream_t stream, BvhNode** nodes_out, DevBuf<uint32_t>& d_order, uint32_t* depth_out,
                  uint32_t builder)
 {
@@ -825,7 +831,7 @@ int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const flo
         hipError_t _e = (expr);                                                               \
         if (_e != hipSuccess) return fail_free(SGPU_E_HIP, std::string(#expr) + ": " + hipGetErrorString(_e)); \
     } while (0)
-    SGPU_BUILD_TRY(d_order.alloc(n));
+    SGPU_BUILD_TRY(d_order.alloc(S, n));
     if (n == 1) {
         hipLaunchKernelGGL(k_single, dim3(1), dim3(1), 0, stream, d_blo, d_bhi, d_bounds, nodes);
         SGPU_BUILD_TRY(hipGetLastError());
@@ -839,12 +845,12 @@ int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const flo
     DevBuf<uint64_t> d_keys, d_keys2;
     DevBuf<int> d_pint, d_pleaf;
     DevBuf<uint8_t> d_tmp;
-    SGPU_BUILD_TRY(d_keys.alloc(n));
-    SGPU_BUILD_TRY(d_keys2.alloc(n));
-    SGPU_BUILD_TRY(d_vals.alloc(n));
-    SGPU_BUILD_TRY(d_pint.alloc(n_int));
-    SGPU_BUILD_TRY(d_pleaf.alloc(n));
-    SGPU_BUILD_TRY(d_depth.alloc(1));
+    SGPU_BUILD_TRY(d_keys.alloc(S, n));
+    SGPU_BUILD_TRY(d_keys2.alloc(S, n));
+    SGPU_BUILD_TRY(d_vals.alloc(S, n));
+    SGPU_BUILD_TRY(d_pint.alloc(S, n_int));
+    SGPU_BUILD_TRY(d_pleaf.alloc(S, n));
+    SGPU_BUILD_TRY(d_depth.alloc(S, 1));
     SGPU_BUILD_TRY(hipMemsetAsync(d_pint.p, 0xFF, (size_t)n_int * sizeof(int), stream));
     SGPU_BUILD_TRY(hipMemsetAsync(d_pleaf.p, 0xFF, (size_t)n * sizeof(int), stream));
     SGPU_BUILD_TRY(hipMemsetAsync(d_depth.p, 0, sizeof(uint32_t), stream));
@@ -855,7 +861,7 @@ int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const flo
     size_t tmp_bytes = 0;
     SGPU_BUILD_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
                                              (size_t)n, 0, 63, stream));
-    SGPU_BUILD_TRY(d_tmp.alloc(tmp_bytes));
+    SGPU_BUILD_TRY(d_tmp.alloc(S, tmp_bytes));
     SGPU_BUILD_TRY(rocprim::radix_sort_pairs(d_tmp.p, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
                                              (size_t)n, 0, 63, stream));
     if (builder == 1) {
@@ -863,21 +869,21 @@ int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const flo
         DevBuf<int> cid[2];
         DevBuf<float4> clo[2], chi[2];
         DevBuf<uint32_t> hgt[2], nn;
-        DevBuf<uint64_t> flags, prefix, last;
+        DevBuf<uint64_t> flags, prefix;
         for (int b = 0; b < 2; ++b) {
-            SGPU_BUILD_TRY(cid[b].alloc(n));
-            SGPU_BUILD_TRY(clo[b].alloc(n));
-            SGPU_BUILD_TRY(chi[b].alloc(n));
-            SGPU_BUILD_TRY(hgt[b].alloc(n));
+            SGPU_BUILD_TRY(cid[b].alloc(S, n));
+            SGPU_BUILD_TRY(clo[b].alloc(S, n));
+            SGPU_BUILD_TRY(chi[b].alloc(S, n));
+            SGPU_BUILD_TRY(hgt[b].alloc(S, n));
         }
-        SGPU_BUILD_TRY(nn.alloc(n));
-        SGPU_BUILD_TRY(flags.alloc(n));
-        SGPU_BUILD_TRY(prefix.alloc(n));
+        SGPU_BUILD_TRY(nn.alloc(S, n));
+        SGPU_BUILD_TRY(flags.alloc(S, n));
+        SGPU_BUILD_TRY(prefix.alloc(S, n));
         size_t scan_bytes = 0;
         SGPU_BUILD_TRY(rocprim::exclusive_scan(nullptr, scan_bytes, flags.p, prefix.p, (uint64_t)0, (size_t)n,
                                                rocprim::plus<uint64_t>(), stream));
         DevBuf<uint8_t> d_scan;
-        SGPU_BUILD_TRY(d_scan.alloc(scan_bytes));
+        SGPU_BUILD_TRY(d_scan.alloc(S, scan_bytes));
         hipLaunchKernelGGL(k_ploc_init, dim3(grid), dim3(kBlock), 0, stream, n, d_blo, d_bhi, d_order.p, d_bounds,
                            cid[0].p, clo[0].p, chi[0].p, hgt[0].p);
         SGPU_BUILD_TRY(hipGetLastError());
@@ -915,7 +921,7 @@ int build_binary(uint32_t n, const float4* d_blo, const float4* d_bhi, const flo
     }
     // the pyramid's levels one after another: level k has ceil(n / 2^k) boxes
     DevBuf<LeafBox> d_boxes;
-    SGPU_BUILD_TRY(d_boxes.alloc(2 * (size_t)n + 2 * kMaxBoxLevels));
+    SGPU_BUILD_TRY(d_boxes.alloc(S, 2 * (size_t)n + 2 * kMaxBoxLevels));
     LeafBox* level[kMaxBoxLevels + kBoxStep];
     uint32_t size[kMaxBoxLevels + kBoxStep];
     size_t used = 0;
@@ -1028,14 +1034,15 @@ int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::
         rec[s].inst = inst[s];
         rec[s].pad = 0;
     }
+    sgpu_scratch S(scene->ctx, stream, build_scratch(n));
     DevBuf<CurveRecord> d_rec;
     DevBuf<float4> d_blo, d_bhi, d_cent;
     DevBuf<uint32_t> d_bounds, d_order;
-    SGPU_HIP_TRY(d_rec.alloc(n));
-    SGPU_HIP_TRY(d_blo.alloc(n));
-    SGPU_HIP_TRY(d_bhi.alloc(n));
-    SGPU_HIP_TRY(d_cent.alloc(n));
-    SGPU_HIP_TRY(d_bounds.alloc(12));
+    SGPU_HIP_TRY(d_rec.alloc(S, n));
+    SGPU_HIP_TRY(d_blo.alloc(S, n));
+    SGPU_HIP_TRY(d_bhi.alloc(S, n));
+    SGPU_HIP_TRY(d_cent.alloc(S, n));
+    SGPU_HIP_TRY(d_bounds.alloc(S, 12));
     SGPU_HIP_TRY(hipMemcpyAsync(d_rec.p, rec.data(), n * sizeof(CurveRecord), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
     const uint32_t grid = (n + kBlock - 1) / kBlock;
@@ -1046,7 +1053,7 @@ int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::
     SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
     BvhNode* nodes = nullptr;
     uint32_t depth = 0;
-    int rc = build_binary(n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth, 0);
+    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth, 0);
     if (rc != SGPU_OK) return rc;
     if (depth + 1 > kCurveStack) {
         (void)hipFree(nodes);
@@ -1090,18 +1097,19 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
     if (n == 0) return SGPU_OK;
     if (n > (1u << 30)) return sgpu_fail(SGPU_E_RANGE, "scene has more than 2^30 triangles");
 
+    sgpu_scratch S(scene->ctx, stream, build_scratch(n));
     DevBuf<float> d_pos;
     DevBuf<uint32_t> d_geom, d_first, d_bounds, d_order;
     DevBuf<TriRecord> d_rec;
     DevBuf<float4> d_blo, d_bhi, d_cent;
-    SGPU_HIP_TRY(d_pos.alloc((size_t)n * 9));
-    SGPU_HIP_TRY(d_geom.alloc(n));
-    SGPU_HIP_TRY(d_first.alloc(scene->geom_first.size()));
-    SGPU_HIP_TRY(d_bounds.alloc(12));
-    SGPU_HIP_TRY(d_rec.alloc(n));
-    SGPU_HIP_TRY(d_blo.alloc(n));
-    SGPU_HIP_TRY(d_bhi.alloc(n));
-    SGPU_HIP_TRY(d_cent.alloc(n));
+    SGPU_HIP_TRY(d_pos.alloc(S, (size_t)n * 9));
+    SGPU_HIP_TRY(d_geom.alloc(S, n));
+    SGPU_HIP_TRY(d_first.alloc(S, scene->geom_first.size()));
+    SGPU_HIP_TRY(d_bounds.alloc(S, 12));
+    SGPU_HIP_TRY(d_rec.alloc(S, n));
+    SGPU_HIP_TRY(d_blo.alloc(S, n));
+    SGPU_HIP_TRY(d_bhi.alloc(S, n));
+    SGPU_HIP_TRY(d_cent.alloc(S, n));
 
     SGPU_HIP_TRY(hipMemcpyAsync(d_pos.p, scene->tri_pos.data(), (size_t)n * 9 * sizeof(float), hipMemcpyHostToDevice,
                                 stream));
@@ -1123,7 +1131,7 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
 
     BvhNode* nodes = nullptr;
     uint32_t depth = 0;
-    int rc = build_binary(n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
+    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
                           scene->ctx->bvh_builder);
     if (rc != SGPU_OK) return rc;
     for (int k = 0; k < 3; ++k) {
@@ -1133,8 +1141,10 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
     scene->d_nodes = nodes;
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
-    rc = build_wide(scene, nodes, n, stream, d_order.p, d_rec.p, nullptr);
-    scene->stack_cap = tree_stack_words(scene->max_depth, scene->wide_depth);
+    rc = build_wide(scene, S, nodes, n, stream, d_order.p, d_rec.p, nullptr);
+    scene->wide_stack = wide_stack_words(scene->wide_depth);
+    // the binary tree's stack: a word per level
+    scene->stack_cap = std::max(scene->max_depth + 1, scene->wide_stack);
     return rc;
 }
 
@@ -1303,6 +1313,7 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
             e = hipMemcpy(scene->d_inst_ids, xids.data(), xids.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
         if (e != hipSuccess) return sgpu_fail(SGPU_E_HIP, std::string("instance records: ") + hipGetErrorString(e));
         scene->n_inst = 0;
+        scene->wide_stack = 0;
         scene->stack_cap = 1;
         return bake_instance_curves(scene, composed(), stream);
     }
@@ -1397,7 +1408,7 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
             for (int c = 0; c < 3; ++c) scene->comp_l2w.push_back((float)f.l2w[4 * r + c]);
         ids[2 * k] = f.id0;
         ids[2 * k + 1] = f.id1;
-        blas_cap = std::max(blas_cap, f.blas->stack_cap);
+        blas_cap = std::max(blas_cap, f.blas->wide_stack);
     }
     push_extra_shading();
     rec.insert(rec.end(), xrec.begin(), xrec.end());
@@ -1411,19 +1422,20 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
         scene->box[r] = slo[r];
         scene->box[3 + r] = shi[r];
     }
+    sgpu_scratch S(scene->ctx, stream, build_scratch(n));
     DevBuf<float4> d_blo, d_bhi, d_cent;
     DevBuf<uint32_t> d_bounds, d_order;
-    SGPU_HIP_TRY(d_blo.alloc(n));
-    SGPU_HIP_TRY(d_bhi.alloc(n));
-    SGPU_HIP_TRY(d_cent.alloc(n));
-    SGPU_HIP_TRY(d_bounds.alloc(12));
+    SGPU_HIP_TRY(d_blo.alloc(S, n));
+    SGPU_HIP_TRY(d_bhi.alloc(S, n));
+    SGPU_HIP_TRY(d_cent.alloc(S, n));
+    SGPU_HIP_TRY(d_bounds.alloc(S, 12));
     SGPU_HIP_TRY(hipMemcpyAsync(d_blo.p, blo.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemcpyAsync(d_bhi.p, bhi.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemcpyAsync(d_cent.p, cent.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemcpyAsync(d_bounds.p, hb, sizeof(hb), hipMemcpyHostToDevice, stream));
     BvhNode* nodes = nullptr;
     uint32_t depth = 0;
-    int rc = build_binary(n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
+    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
                           scene->ctx->bvh_builder);
     if (rc != SGPU_OK) return rc;
     InstRecord* d_inst = nullptr;
@@ -1447,9 +1459,11 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     scene->blas_stack_cap = blas_cap;
     // instance nodes name composed instances by their composition index (instance i, then its instance
     // j), so the closest-hit tie rule follows (inst_id0, inst_id1)
-    rc = build_wide(scene, nodes, n, stream, d_order.p, nullptr, d_inst);
-    // the top tree's stack, the exit entry, and the deepest placed tree's stack
-    scene->stack_cap = tree_stack_words(scene->max_depth, scene->wide_depth) + 2 + blas_cap;
+    rc = build_wide(scene, S, nodes, n, stream, d_order.p, nullptr, d_inst);
+    // the top tree's groups above an instance's node (its last level), the exit entry and the deepest
+    // placed tree's stack; the binary top tree is not walked
+    scene->wide_stack = 2 * scene->wide_depth + blas_cap;
+    scene->stack_cap = scene->wide_stack;
     if (rc != SGPU_OK) return rc;
     return bake_instance_curves(scene, composed(), stream);
 }

@@ -42,6 +42,81 @@ int sgpu_fail(int code, const std::string& msg)
     return code;
 }
 
+hipError_t sgpu_scratch_take(sgpu_context ctx, size_t bytes, ScratchBlock& out)
+{
+    {
+        std::lock_guard<std::mutex> lock(ctx->scratch_mu);
+        size_t best = ctx->scratch_idle.size();
+        for (size_t k = 0; k < ctx->scratch_idle.size(); ++k)
+            if (ctx->scratch_idle[k].bytes >= bytes &&
+                (best == ctx->scratch_idle.size() || ctx->scratch_idle[k].bytes < ctx->scratch_idle[best].bytes))
+                best = k;
+        if (best < ctx->scratch_idle.size()) {
+            out = ctx->scratch_idle[best];
+            ctx->scratch_idle.erase(ctx->scratch_idle.begin() + (ptrdiff_t)best);
+            return hipSuccess;
+        }
+    }
+    out.bytes = (bytes + bytes / 8 + ((size_t)1 << 20)) & ~(((size_t)1 << 20) - 1);
+    hipError_t e = hipMalloc((void**)&out.dev, out.bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        sgpu_scratch_trim(ctx);
+        out.bytes = bytes;
+        e = hipMalloc((void**)&out.dev, out.bytes);
+    }
+    if (e != hipSuccess) return e;
+    e = hipHostMalloc((void**)&out.pinned, kScratchPinned * sizeof(uint64_t), hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipFree(out.dev);
+    return e;
+}
+
+namespace {
+void scratch_free(const ScratchBlock& b)
+{
+    (void)hipFree(b.dev);
+    (void)hipHostFree(b.pinned);
+}
+}  // namespace
+
+void sgpu_scratch_give(sgpu_context ctx, const ScratchBlock& b)
+{
+    // the smallest idle blocks go first when the context would keep too much
+    std::vector<ScratchBlock> drop;
+    try {
+        std::lock_guard<std::mutex> lock(ctx->scratch_mu);
+        std::vector<ScratchBlock>& idle = ctx->scratch_idle;
+        drop.reserve(idle.size() + 1);
+        idle.push_back(b);
+        size_t total = 0;
+        for (const ScratchBlock& k : idle) total += k.bytes;
+        while (total > kScratchKeep) {
+            const auto it = b.bytes > kScratchKeep ? idle.end() - 1
+                                                   : std::min_element(idle.begin(), idle.end(),
+                                                                      [](const ScratchBlock& x, const ScratchBlock& y) {
+                                                                          return x.bytes < y.bytes;
+                                                                      });
+            drop.push_back(*it);
+            total -= it->bytes;
+            idle.erase(it);
+        }
+    } catch (...) {
+        scratch_free(b);
+        return;
+    }
+    for (const ScratchBlock& k : drop) scratch_free(k);
+}
+
+void sgpu_scratch_trim(sgpu_context ctx)
+{
+    std::vector<ScratchBlock> drop;
+    {
+        std::lock_guard<std::mutex> lock(ctx->scratch_mu);
+        drop.swap(ctx->scratch_idle);
+    }
+    for (const ScratchBlock& k : drop) scratch_free(k);
+}
+
 extern "C" {
 
 const char* sgpu_last_error(void) { return g_last_error.c_str(); }
@@ -82,6 +157,7 @@ int sgpu_context_destroy(sgpu_context ctx)
 {
     if (!ctx) return SGPU_OK;
     sgpu_vcm_release_cached(ctx);
+    sgpu_scratch_trim(ctx);
     delete ctx;
     return SGPU_OK;
 }
@@ -147,6 +223,11 @@ int sgpu_malloc(sgpu_context ctx, size_t bytes, void** dptr)
     *dptr = nullptr;
     if (bytes == 0) bytes = 1;
     hipError_t e = hipMalloc(dptr, bytes);
+    if (e == hipErrorOutOfMemory) {  // the context's idle scratch goes first
+        (void)hipGetLastError();
+        sgpu_scratch_trim(ctx);
+        e = hipMalloc(dptr, bytes);
+    }
     if (e != hipSuccess) return sgpu_fail(SGPU_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return SGPU_OK;
 }
@@ -658,12 +739,15 @@ int sgpu_scene_commit(sgpu_scene scene, void* stream)
     std::vector<std::vector<float>>().swap(scene->geom_xform);
     // the sphere around the triangles' (and curves') bounding box (the IBL emits from its disc)
     if (!scene->tri_pos.empty() || scene->n_curves > 0) {
+        // the build's box is that box; vertices that are not numbers (which it takes in) are left out
         float lo[3], hi[3];
+        bool finite = true;
+        for (int k = 0; k < 6; ++k) finite &= std::isfinite(scene->box[k]);
         for (int k = 0; k < 3; ++k) {
-            lo[k] = scene->tri_pos.empty() ? scene->box[k] : scene->tri_pos[k];
-            hi[k] = scene->tri_pos.empty() ? scene->box[3 + k] : scene->tri_pos[k];
+            lo[k] = finite || scene->tri_pos.empty() ? scene->box[k] : scene->tri_pos[k];
+            hi[k] = finite || scene->tri_pos.empty() ? scene->box[3 + k] : scene->tri_pos[k];
         }
-        for (size_t i = 0; i < scene->tri_pos.size(); i += 3)
+        for (size_t i = 0; !finite && i < scene->tri_pos.size(); i += 3)
             for (int k = 0; k < 3; ++k) {
                 lo[k] = std::min(lo[k], scene->tri_pos[i + k]);
                 hi[k] = std::max(hi[k], scene->tri_pos[i + k]);

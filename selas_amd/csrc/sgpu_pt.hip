@@ -468,36 +468,19 @@ __global__ __launch_bounds__(kBlock) void k_scale(float* __restrict fb, size_t n
     if (i < n) fb[i] = fb[i] * s;
 }
 
-struct Arena {
-    std::vector<void*> ptrs;
-    hipStream_t stream;
-    hipError_t err = hipSuccess;
-    template <typename T>
-    T* get(size_t count)
-    {
-        void* p = nullptr;
-        if (err == hipSuccess) err = hipMallocAsync(&p, count * sizeof(T) + 64, stream);
-        if (err == hipSuccess) ptrs.push_back(p);
-        return (T*)p;
-    }
-    RayBuf rays(size_t n)
-    {
-        RayBuf r;
-        r.ox = get<float>(n);
-        r.oy = get<float>(n);
-        r.oz = get<float>(n);
-        r.dx = get<float>(n);
-        r.dy = get<float>(n);
-        r.dz = get<float>(n);
-        r.tnear = get<float>(n);
-        r.tfar = get<float>(n);
-        return r;
-    }
-    ~Arena()
-    {
-        for (void* p : ptrs) (void)hipFreeAsync(p, stream);
-    }
-};
+RayBuf ray_buf(sgpu_scratch& S, size_t n)
+{
+    RayBuf r;
+    r.ox = S.get<float>(n);
+    r.oy = S.get<float>(n);
+    r.oz = S.get<float>(n);
+    r.dx = S.get<float>(n);
+    r.dy = S.get<float>(n);
+    r.dz = S.get<float>(n);
+    r.tnear = S.get<float>(n);
+    r.tfar = S.get<float>(n);
+    return r;
+}
 
 sgpu_rays_soa as_soa(const RayBuf& r) { return sgpu_rays_soa{r.ox, r.oy, r.oz, r.dx, r.dy, r.dz, r.tnear, r.tfar}; }
 
@@ -536,8 +519,10 @@ int render_paths(sgpu_scene scene, const PathJob& job, float* fb, hipStream_t st
                                    mk3(job.camera.up[0], job.camera.up[1], job.camera.up[2]),
                                    job.camera.fov_degrees, W, H);
 
-    Arena A;
-    A.stream = stream;
+    // per path: state 52 (56), rays and queues 72 (108 with the ray sort), hits 36, light samples 52 and
+    // sky samples 52, sort keys 16 and 24; the sorts' own comes on top
+    const size_t per_path = 52 + 72 + 36 + 52 + (job.dpt ? 56 : 0) + (job.sort_rays ? 52 : 0) + (job.sort_hits ? 24 : 0);
+    sgpu_scratch A(scene->ctx, stream, per_path * cap + sgpu_trace_spill_words(scene) * sizeof(uint32_t) + (1u << 18));
     PathState ps;
     ps.thr = A.get<float>(3 * (size_t)cap);
     ps.ld0 = job.dpt ? nullptr : A.get<float>(3 * (size_t)cap);
@@ -545,10 +530,10 @@ int render_paths(sgpu_scene scene, const PathJob& job, float* fb, hipStream_t st
     ps.rng = A.get<uint64_t>(cap);
     ps.flags = A.get<uint32_t>(cap);
     ps.pdf = job.dpt ? A.get<float>(cap) : nullptr;
-    RayBuf rays[3] = {A.rays(cap), A.rays(cap), RayBuf{}};
+    RayBuf rays[3] = {ray_buf(A, cap), ray_buf(A, cap), RayBuf{}};
     uint32_t* queue[3] = {A.get<uint32_t>(cap), A.get<uint32_t>(cap), nullptr};
     if (job.sort_rays) {
-        rays[2] = A.rays(cap);
+        rays[2] = ray_buf(A, cap);
         queue[2] = A.get<uint32_t>(cap);
     }
     HitBuf hb;
@@ -563,7 +548,7 @@ int render_paths(sgpu_scene scene, const PathJob& job, float* fb, hipStream_t st
     hb.inst = A.get<uint32_t>(cap);
     auto shadow_buf = [&]() {
         ShadowBuf b;
-        b.ray = A.rays(cap);
+        b.ray = ray_buf(A, cap);
         b.path = A.get<uint32_t>(cap);
         b.c = A.get<float>(3 * (size_t)cap);
         b.occluded = A.get<uint32_t>(cap);
@@ -636,13 +621,8 @@ int render_paths(sgpu_scene scene, const PathJob& job, float* fb, hipStream_t st
                                                end_bit, stream));
         sort_tmp = A.get<uint8_t>(sort_bytes);
     }
-    uint32_t* h_counters = nullptr;
     if (A.err != hipSuccess) return sgpu_fail(SGPU_E_NOMEM, "sgpu_render: device allocation failed");
-    SGPU_HIP_TRY(hipHostMalloc((void**)&h_counters, 4 * sizeof(uint32_t), hipHostMallocDefault));
-    struct HostFree {
-        uint32_t* p;
-        ~HostFree() { (void)hipHostFree(p); }
-    } hf{h_counters};
+    uint32_t* const h_counters = (uint32_t*)A.pinned();
 
     SGPU_HIP_TRY(hipMemsetAsync(fb, 0, layers * 3 * n_pixels * sizeof(float), stream));
     if (d_trav) SGPU_HIP_TRY(hipMemsetAsync(d_trav, 0, 2 * sizeof(uint64_t), stream));

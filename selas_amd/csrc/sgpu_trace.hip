@@ -686,19 +686,23 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
 
     // stream-ordered scratch for the spilled part of the stacks, private to this call, unless the
     // caller lends a buffer of sgpu_trace_spill_words (sized for the largest grid); its first
-    // kTraceWorkWords words are the launch's ray counters (zero between launches)
+    // kTraceWorkWords words are the launch's ray counters. A launch whose rays the grid holds at once
+    // and whose stacks fit LDS touches neither (a stream-ordered free makes the host wait for the
+    // kernel: 150 us of a small query).
+    const bool binary = ctx->trace_tree == 0 && !instanced;
+    const bool counts = !binary && blocks < (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK;
     uint32_t* buf = spill_buf;
-    if (!buf)
+    if (!buf && (counts || stack_words > SGPU_STACK_LDS))
         SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
                                     spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) * sizeof(uint32_t), stream));
     uint32_t* const work = buf;
-    uint32_t* const spill = buf + kTraceWorkWords;
+    uint32_t* const spill = buf ? buf + kTraceWorkWords : nullptr;
     sgpu_hits_soa h = {};
     if (hits) h = *hits;
     unsigned long long* st = (unsigned long long*)d_stats;
     const bool multi = table != nullptr;
     const dim3 g(blocks), b(SGPU_TRACE_BLOCK);
-    if (ctx->trace_tree == 0 && !instanced) {
+    if (binary) {
 #define SGPU_LAUNCH_2(A, S, M)                                                                                      \
     hipLaunchKernelGGL((k_trace<A, S, M>), g, b, 0, stream, scene.nodes,                      \
                        reinterpret_cast<const TriRecord*>(scene.wide), scene.n_tris, table, ray_scene,            \
@@ -714,11 +718,10 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
     } else {
         // top nodes in LDS: single-scene launches over geometries
         const uint32_t n_top = multi || instanced ? 0u : std::min(n_wide, std::min(ctx->trace_lds_nodes, kTopNodes));
-        // the launch's ray counter, where the grid does not hold every ray at once
-        if (blocks < (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK) sgpu_trace_work_zero(work, stream);
+        if (counts) sgpu_trace_work_zero(work, stream);
 #define SGPU_LAUNCH_8(A, S, M, I, T)                                                                               \
     hipLaunchKernelGGL((k_trace8<A, S, M, I, T>), g, b, 0, stream, scene, inst_ids, table, ray_scene, *rays, h,    \
-                       occluded, n, n_ptr, (uint2*)spill, stack_words / 2, st, overflow, work, comp_out, n_top)
+                       occluded, n, n_ptr, (uint2*)spill, std::max(stack_words / 2, kWideStackLds), st, overflow, work, comp_out, n_top)
 #define SGPU_LAUNCH_8S(A, S)                                                                                      \
     do {                                                                                                          \
         if (multi && instanced) SGPU_LAUNCH_8(A, S, true, true, false);                                           \
@@ -738,7 +741,7 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
 #undef SGPU_LAUNCH_8
     }
     SGPU_HIP_TRY(hipGetLastError());
-    if (!spill_buf) SGPU_HIP_TRY(hipFreeAsync(buf, stream));
+    if (buf && !spill_buf) SGPU_HIP_TRY(hipFreeAsync(buf, stream));
     return SGPU_OK;
 }
 
@@ -759,7 +762,8 @@ int sgpu_trace_launch(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hi
 {
     const TraceScene ts{scene->d_nodes, scene->d_wide,   scene->n_tris,   scene->n_inst,
                         scene->d_inst,  scene->d_cnodes, scene->d_curves, scene->n_curves};
-    const int rc = trace_launch(scene->ctx, ts, scene->n_wide, scene->d_inst_ids, scene->stack_cap,
+    const int rc = trace_launch(scene->ctx, ts, scene->n_wide, scene->d_inst_ids,
+                                scene->ctx->trace_tree == 1 ? scene->wide_stack : scene->stack_cap,
                                 overflow ? overflow : scene->d_overflow, nullptr, nullptr, rays, hits, occluded, n,
                                 any_hit, d_stats, stream, spill_buf, n_ptr, !scene->instances.empty(), comp_out,
                                 max_blocks);
