@@ -1079,7 +1079,7 @@ def bench_curves(args):
         "build_ms": round(build_ms, 1),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "closest hit: k_trace8 over the ground, then k_curves<false,false,false>",
+                     "kernel": "closest hit: k_trace8 over the ground, then k_curves",
                      "bytes_per_ray": round(bytes_per_ray, 1)},
         "cpu_baseline": None,
     }

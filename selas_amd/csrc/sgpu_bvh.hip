@@ -693,11 +693,17 @@ struct DevBuf {
 // taken as needed.
 size_t build_scratch(size_t n) { return 500 * n + ((size_t)1 << 20); }
 
-// Collapses the binary tree (nodes, root 0, over n leaves) into the scene's 8-wide tree, with the
-// triangle records rec[order[j]] of its leaves j. The top tree of an instanced scene passes its
-// instance records instead of triangles (order[j]: the instance of leaf j): its leaves become nodes.
-int build_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
-               const TriRecord* rec, const InstRecord* insts)
+struct WideTree {
+    WideNode* wide = nullptr;
+    uint32_t n_slots = 0, n_wide = 0, depth = 0;
+};
+
+// Collapses the binary tree (nodes, root 0, over n leaves) into an 8-wide tree, with the records (64
+// bytes, triangles or curve segments) rec[order[j]] of its leaves j; d_leaf_slot: their slots. The top
+// tree of an instanced scene passes its instance records instead (order[j]: the instance of leaf j):
+// its leaves become nodes.
+int build_wide(sgpu_scratch& S, const BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
+               const TriRecord* rec, const InstRecord* insts, WideTree& tree, DevBuf<uint32_t>& d_leaf_slot)
 {
     const bool top = insts != nullptr;
     const uint32_t n_leaves = std::max(n, 2u);  // a tree of one leaf has a root with two children, the leaf twice
@@ -705,7 +711,7 @@ int build_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t n, hi
     DevBuf<WideTask> d_tasks, d_next;
     DevBuf<int> d_cref;
     DevBuf<float> d_cbox;
-    DevBuf<uint32_t> d_nch, d_bad, d_slot, d_leaf_slot;
+    DevBuf<uint32_t> d_nch, d_bad, d_slot;
     DevBuf<uint64_t> d_cnt, d_off;
     DevBuf<NodeSlot> d_all;
     DevBuf<uint8_t> d_tmp;
@@ -765,24 +771,40 @@ int build_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t n, hi
     SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     if (*(const uint32_t*)S.pinned()) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_wide, slot_base * kSlotBytes));
-    scene->n_slots = (uint32_t)slot_base;
-    scene->n_wide = level_base;
-    scene->wide_depth = depth;
-    NodeSlot* const slots = reinterpret_cast<NodeSlot*>(scene->d_wide);
+    SGPU_HIP_TRY(hipMalloc((void**)&tree.wide, slot_base * kSlotBytes));
+    tree.n_slots = (uint32_t)slot_base;
+    tree.n_wide = level_base;
+    tree.depth = depth;
+    NodeSlot* const slots = reinterpret_cast<NodeSlot*>(tree.wide);
     auto grid4 = [](size_t k) { return dim3((uint32_t)((4 * k + kBlock - 1) / kBlock)); };
     hipLaunchKernelGGL(k_place_nodes, grid4(level_base), dim3(kBlock), 0, stream, d_all.p, d_slot.p, level_base, slots);
     SGPU_HIP_TRY(hipGetLastError());
     if (!top) {
-        // (of the two slots of a single triangle one stays empty: zeros, which no ray hits)
-        if (n == 1) SGPU_HIP_TRY(hipMemsetAsync(slots + 1, 0, (slot_base - 1) * kSlotBytes, stream));
         hipLaunchKernelGGL(k_place_tris, grid4(n), dim3(kBlock), 0, stream, rec, order, d_leaf_slot.p, n, slots);
         SGPU_HIP_TRY(hipGetLastError());
-        const uint32_t n_int = n > 1 ? n - 1 : 1;
-        hipLaunchKernelGGL(k_relabel, dim3((n_int + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, nodes, n_int,
-                           d_leaf_slot.p);
-        SGPU_HIP_TRY(hipGetLastError());
+        if (n == 1)  // a single leaf is both children of the root: slots 1 and 2
+            for (int k = 1; k <= 2; ++k)
+                SGPU_HIP_TRY(hipMemcpyAsync(slots + k, rec, kSlotBytes, hipMemcpyDeviceToDevice, stream));
     }
+    SGPU_HIP_TRY(hipStreamSynchronize(stream));
+    return SGPU_OK;
+}
+
+// build_wide as the scene's own tree (of triangles, or of instances).
+int build_scene_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t n, hipStream_t stream,
+                     const uint32_t* order, const TriRecord* rec, const InstRecord* insts)
+{
+    WideTree t;
+    DevBuf<uint32_t> leaf_slot;
+    const int rc = build_wide(S, nodes, n, stream, order, rec, insts, t, leaf_slot);
+    scene->d_wide = t.wide;
+    scene->n_slots = t.n_slots;
+    scene->n_wide = t.n_wide;
+    scene->wide_depth = t.depth;
+    if (rc != SGPU_OK || insts) return rc;
+    const uint32_t n_int = n > 1 ? n - 1 : 1;
+    hipLaunchKernelGGL(k_relabel, dim3((n_int + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, nodes, n_int, leaf_slot.p);
+    SGPU_HIP_TRY(hipGetLastError());
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     return SGPU_OK;
 }
@@ -963,7 +985,10 @@ namespace {
 
 // Box of each curve segment (its control points' box grown by the largest radius: the B-spline
 // basis weights are non-negative and sum to one, so the swept balls stay inside), centroid, and the
-// ordered-uint bounds k_prep computes.
+// ordered-uint bounds k_prep computes. TIGHT: the box and centroid of the same cubic's Bezier points,
+// which span the segment alone and not its neighbours' two thirds of the control polygon (a third of
+// the length along a blade of grass); the bounds' scene box stays that of the control points.
+template <bool TIGHT>
 __global__ __launch_bounds__(kBlock) void k_curve_prep(const CurveRecord* __restrict rec, uint32_t n,
                                                        float4* __restrict blo, float4* __restrict bhi,
                                                        float4* __restrict cent, uint32_t* __restrict bounds)
@@ -983,12 +1008,24 @@ __global__ __launch_bounds__(kBlock) void k_curve_prep(const CurveRecord* __rest
         }
         lo = mk3(lo.x - rmax, lo.y - rmax, lo.z - rmax);
         hi = mk3(hi.x + rmax, hi.y + rmax, hi.z + rmax);
+        v[0] = f2ord(lo.x); v[1] = f2ord(lo.y); v[2] = f2ord(lo.z);
+        v[3] = ~f2ord(hi.x); v[4] = ~f2ord(hi.y); v[5] = ~f2ord(hi.z);
+        if (TIGHT) {
+            const float4 p0 = r.p[0], p1 = r.p[1], p2 = r.p[2], p3 = r.p[3];
+            auto bezier = [&](float a, float b, float c, float e, float& l, float& h) {
+                const float q0 = (a + 4.0f * b + c) * (1.0f / 6.0f), q1 = (2.0f * b + c) * (1.0f / 3.0f);
+                const float q2 = (b + 2.0f * c) * (1.0f / 3.0f), q3 = (b + 4.0f * c + e) * (1.0f / 6.0f);
+                l = fminf(fminf(q0, q1), fminf(q2, q3)) - rmax;
+                h = fmaxf(fmaxf(q0, q1), fmaxf(q2, q3)) + rmax;
+            };
+            bezier(p0.x, p1.x, p2.x, p3.x, lo.x, hi.x);
+            bezier(p0.y, p1.y, p2.y, p3.y, lo.y, hi.y);
+            bezier(p0.z, p1.z, p2.z, p3.z, lo.z, hi.z);
+        }
         const f3 c = mk3(0.5f * (lo.x + hi.x), 0.5f * (lo.y + hi.y), 0.5f * (lo.z + hi.z));
         blo[i] = make_float4(lo.x, lo.y, lo.z, 0.0f);
         bhi[i] = make_float4(hi.x, hi.y, hi.z, 0.0f);
         cent[i] = make_float4(c.x, c.y, c.z, 0.0f);
-        v[0] = f2ord(lo.x); v[1] = f2ord(lo.y); v[2] = f2ord(lo.z);
-        v[3] = ~f2ord(hi.x); v[4] = ~f2ord(hi.y); v[5] = ~f2ord(hi.z);
         v[6] = f2ord(c.x); v[7] = f2ord(c.y); v[8] = f2ord(c.z);
         v[9] = ~f2ord(c.x); v[10] = ~f2ord(c.y); v[11] = ~f2ord(c.z);
     }
@@ -1008,12 +1045,35 @@ __global__ __launch_bounds__(kBlock) void k_curve_prep(const CurveRecord* __rest
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_curve_reorder(const CurveRecord* __restrict in,
-                                                          const uint32_t* __restrict order, uint32_t n,
-                                                          CurveRecord* __restrict out)
+// The control points alone, as leaf records.
+__global__ __launch_bounds__(kBlock) void k_curve_points(const CurveRecord* __restrict in, uint32_t n,
+                                                         CurvePoints* __restrict out)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) out[i] = in[order[i]];
+    if (i >= n) return;
+    for (int j = 0; j < 4; ++j) out[i].p[j] = in[i].p[j];
+}
+
+// Each segment's place in the leaf order `order`.
+__global__ __launch_bounds__(kBlock) void k_curve_places(const uint32_t* __restrict order, uint32_t n,
+                                                         uint32_t* __restrict place)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) place[order[i]] = i;
+}
+
+// The ids of the segment in each leaf's slot (a single segment is in slots 1 and 2).
+__global__ __launch_bounds__(kBlock) void k_curve_ids(const CurveRecord* __restrict rec, const uint32_t* __restrict order,
+                                                      const uint32_t* __restrict leaf_slot,
+                                                      const uint32_t* __restrict place, uint32_t n,
+                                                      uint4* __restrict ids)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t k = order[i];
+    const uint4 v = make_uint4(rec[k].geom, rec[k].prim, rec[k].inst, place[k]);
+    ids[leaf_slot[i]] = v;
+    if (n == 1) ids[1] = ids[2] = v;
 }
 
 }  // namespace
@@ -1046,34 +1106,49 @@ int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::
     SGPU_HIP_TRY(hipMemcpyAsync(d_rec.p, rec.data(), n * sizeof(CurveRecord), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
     const uint32_t grid = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_curve_prep, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p, d_cent.p,
+    hipLaunchKernelGGL(k_curve_prep<false>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p, d_cent.p,
                        d_bounds.p);
     SGPU_HIP_TRY(hipGetLastError());
     uint32_t hb[12];
     SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
-    BvhNode* nodes = nullptr;
+    // the tree that orders hits at equal distance
     uint32_t depth = 0;
-    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth, 0);
+    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &scene->d_cnodes, d_order, &depth, 0);
     if (rc != SGPU_OK) return rc;
-    if (depth + 1 > kCurveStack) {
-        (void)hipFree(nodes);
+    if (depth + 1 > kCurveStack)
         return sgpu_fail(SGPU_E_RANGE, "curve tree deeper than the curve traversal's stack");
-    }
-    CurveRecord* out = nullptr;
-    hipError_t e = hipMalloc((void**)&out, (size_t)n * sizeof(CurveRecord));
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_curve_reorder, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order.p, n, out);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) {
-        (void)hipFree(nodes);
-        if (out) (void)hipFree(out);
-        return sgpu_fail(SGPU_E_HIP, std::string("curve records: ") + hipGetErrorString(e));
-    }
-    scene->d_cnodes = nodes;
-    scene->d_curves = out;
+    DevBuf<uint32_t> d_place, d_order2, d_leaf_slot;
+    DevBuf<CurvePoints> d_points;
+    SGPU_HIP_TRY(d_place.alloc(S, n));
+    SGPU_HIP_TRY(d_points.alloc(S, n));
+    hipLaunchKernelGGL(k_curve_places, dim3(grid), dim3(kBlock), 0, stream, d_order.p, n, d_place.p);
+    hipLaunchKernelGGL(k_curve_points, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_points.p);
+    SGPU_HIP_TRY(hipGetLastError());
+    // the tree that is walked, over the tight boxes
+    SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
+    hipLaunchKernelGGL(k_curve_prep<true>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p, d_cent.p,
+                       d_bounds.p);
+    SGPU_HIP_TRY(hipGetLastError());
+    struct Nodes {
+        BvhNode* p = nullptr;
+        ~Nodes() { (void)hipFree(p); }
+    } walked;
+    rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &walked.p, d_order2, &depth, 0);
+    WideTree tree;
+    if (rc == SGPU_OK)
+        rc = build_wide(S, walked.p, n, stream, d_order2.p, reinterpret_cast<const TriRecord*>(d_points.p), nullptr, tree,
+                        d_leaf_slot);
+    scene->d_cwide = tree.wide;
+    scene->n_cslots = tree.n_slots;
+    if (rc != SGPU_OK) return rc;
+    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_cids, (size_t)tree.n_slots * sizeof(uint4)));
+    hipLaunchKernelGGL(k_curve_ids, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order2.p, d_leaf_slot.p, d_place.p, n,
+                       scene->d_cids);
+    SGPU_HIP_TRY(hipGetLastError());
+    SGPU_HIP_TRY(hipStreamSynchronize(stream));
     scene->n_curves = n;
+    scene->wide_stack = std::max(scene->wide_stack, wide_stack_words(tree.depth));
+    scene->stack_cap = std::max(scene->stack_cap, scene->wide_stack);
     // the scene's box takes in the curves
     for (int k = 0; k < 3; ++k) {
         const float lo = host_ord2f(hb[k]), hi = host_ord2f(~hb[3 + k]);
@@ -1141,7 +1216,7 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
     scene->d_nodes = nodes;
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
-    rc = build_wide(scene, S, nodes, n, stream, d_order.p, d_rec.p, nullptr);
+    rc = build_scene_wide(scene, S, nodes, n, stream, d_order.p, d_rec.p, nullptr);
     scene->wide_stack = wide_stack_words(scene->wide_depth);
     // the binary tree's stack: a word per level
     scene->stack_cap = std::max(scene->max_depth + 1, scene->wide_stack);
@@ -1459,7 +1534,7 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     scene->blas_stack_cap = blas_cap;
     // instance nodes name composed instances by their composition index (instance i, then its instance
     // j), so the closest-hit tie rule follows (inst_id0, inst_id1)
-    rc = build_wide(scene, S, nodes, n, stream, d_order.p, nullptr, d_inst);
+    rc = build_scene_wide(scene, S, nodes, n, stream, d_order.p, nullptr, d_inst);
     // the top tree's groups above an instance's node (its last level), the exit entry and the deepest
     // placed tree's stack; the binary top tree is not walked
     scene->wide_stack = 2 * scene->wide_depth + blas_cap;

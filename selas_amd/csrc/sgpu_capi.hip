@@ -793,7 +793,8 @@ int sgpu_scene_release(sgpu_scene scene)
     if (scene->d_nodes) (void)hipFree(scene->d_nodes);
     if (scene->d_wide) (void)hipFree(scene->d_wide);
     if (scene->d_cnodes) (void)hipFree(scene->d_cnodes);
-    if (scene->d_curves) (void)hipFree(scene->d_curves);
+    if (scene->d_cwide) (void)hipFree(scene->d_cwide);
+    if (scene->d_cids) (void)hipFree(scene->d_cids);
     if (scene->d_overflow) (void)hipFree(scene->d_overflow);
     if (scene->d_materials) (void)hipFree(scene->d_materials);
     if (scene->d_geom_material) (void)hipFree(scene->d_geom_material);
@@ -1252,7 +1253,7 @@ int sgpu_scene_device_bytes(sgpu_scene scene, uint64_t* bytes)
                  (uint64_t)scene->n_geom_tex * sizeof(sgpu::PtexTex) +
                  (uint64_t)scene->ibl_w * scene->ibl_h * 4 * sizeof(float) + (uint64_t)scene->ibl_h * sizeof(float) +
                  (uint64_t)scene->n_inst * (sizeof(InstRecord) + 2 * sizeof(uint32_t)) +
-                 (uint64_t)scene->n_curves * (sizeof(CurveRecord) + sizeof(BvhNode));
+                 (uint64_t)scene->n_cslots * (kSlotBytes + sizeof(uint4)) + (uint64_t)scene->n_curves * sizeof(BvhNode);
     for (const sgpu::PtexTex& t : scene->tex_host)
         if (t.texels) b += (uint64_t)t.nfaces * (3ull << (2 * t.res_log2)) + (uint64_t)t.nfaces * 8 * sizeof(int32_t);
     for (const auto& a : scene->attr_allocs) b += a.second;

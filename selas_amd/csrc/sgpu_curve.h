@@ -148,19 +148,27 @@ SGPU_HD float curve_golden(const CurveSeg& s, const CurveRay& ray, float lo, flo
     return 0.5f * (lo + hi);
 }
 
-// First entry of the ray into the segment with t in [tnear, tfar]; ANY: the first found.
-template <bool ANY>
-SGPU_HD bool curve_intersect(const CurveSeg& s, f3 o, f3 d, float tnear, float tfar, float& t_out, float& u_out,
-                             f3& ng)
+// The search's steps, for a caller that runs them one at a time (the device's traversal, whose waves do
+// each step for many lanes at once). Over one segment: curve_start, then for the pieces k that
+// curve_piece_candidate passes with the closest entry so far, in ascending order, curve_piece_search and,
+// where the line crosses a ball, curve_piece_entry.
+
+SGPU_HD CurveRay curve_ray(f3 o, f3 d, float& a)
 {
     CurveRay ray;
     ray.o = o;
     ray.d = d;
-    const float a = dot3(d, d);
+    a = dot3(d, d);
     ray.inv_a = 1.0f / a;
     ray.inv_len = 1.0f / sqrtf(a);
-    const float h = 1.0f / kCurvePieces;
-    float m2 = 0.0f, m2r = 0.0f;
+    return ray;
+}
+
+// Bounds of the segment's second differences: position m2, radius m2r.
+SGPU_HD void curve_bounds(const CurveSeg& s, float& m2, float& m2r)
+{
+    m2 = 0.0f;
+    m2r = 0.0f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const f3 e = mk3(s.p[j].x - 2.0f * s.p[j + 1].x + s.p[j + 2].x, s.p[j].y - 2.0f * s.p[j + 1].y + s.p[j + 2].y,
@@ -168,95 +176,104 @@ SGPU_HD bool curve_intersect(const CurveSeg& s, f3 o, f3 d, float tnear, float t
         m2 = fmaxf(m2, length3(e));
         m2r = fmaxf(m2r, fabsf(s.p[j].w - 2.0f * s.p[j + 1].w + s.p[j + 2].w));
     }
-    const float dev = h * h * 0.125f * (m2 + m2r);
-    float best = tfar, bu = 0.0f;
-    bool found = false;
-    f3 A;
-    float ra;
+}
+
+// Whether the capsule of radius R around chord AB can hold an entry in [tnear, best]: the closest
+// approach of the ray's line and the chord, then the entry bound of its bounding sphere.
+SGPU_HD bool capsule_may_hit(const CurveRay& ray, float a, f3 A, f3 B, float R, float tnear, float best)
+{
+    const f3 e = B - A, w0 = ray.o - A;
+    const float b = dot3(ray.d, e), c = dot3(e, e), dd = dot3(ray.d, w0), ee = dot3(e, w0);
+    const float den = a * c - b * b;
+    float sc = den > 0.0f ? (a * ee - b * dd) / den : 0.0f;
+    sc = fminf(fmaxf(sc, 0.0f), 1.0f);
+    const float tc = (sc * b - dd) * ray.inv_a;
+    const f3 x = (ray.o + ray.d * tc) - (A + e * sc);
+    const float reach = (R + sqrtf(c)) * ray.inv_len;
+    if (!(dot3(x, x) <= R * R * 1.0001f && tc + reach >= tnear && tc - reach <= best)) return false;
+    float tl;
+    return capsule_entry_bound(ray, A, B, R * 1.0001f, tl) && tl <= best;
+}
+
+// The whole segment first: its balls lie in the capsule around the chord P(0) P(1) whose radius is the
+// larger end radius plus (position and radius second-difference bounds) / 8.
+SGPU_HD bool curve_start(const CurveSeg& s, const CurveRay& ray, float a, float m2, float m2r, float tnear, float best)
+{
+    f3 A, B;
+    float ra, rb;
     curve_eval(s, 0.0f, A, ra);
-    {
-        // the whole segment first: its balls lie in the capsule around the chord P(0) P(1) whose radius
-        // is the larger end radius plus (position and radius second-difference bounds) / 8
-        f3 B;
-        float rb;
-        curve_eval(s, 1.0f, B, rb);
-        const float R = fmaxf(ra, rb) + 0.125f * (m2 + m2r);
-        const f3 e = B - A, w0 = o - A;
-        const float b = dot3(d, e), c = dot3(e, e), dd = dot3(d, w0), ee = dot3(e, w0);
-        const float den = a * c - b * b;
-        float sc = den > 0.0f ? (a * ee - b * dd) / den : 0.0f;
-        sc = fminf(fmaxf(sc, 0.0f), 1.0f);
-        const float tc = (sc * b - dd) * ray.inv_a;
-        const f3 x = (o + d * tc) - (A + e * sc);
-        const float reach = (R + sqrtf(c)) * ray.inv_len;
-        if (!(dot3(x, x) <= R * R * 1.0001f && tc + reach >= tnear && tc - reach <= best)) return false;
-        float tl;
-        if (!capsule_entry_bound(ray, A, B, R * 1.0001f, tl) || tl > best) return false;
-    }
-    for (int k = 0; k < kCurvePieces; ++k) {
-        f3 B;
-        float rb;
-        curve_eval(s, (float)(k + 1) * h, B, rb);
-        const float R = fmaxf(ra, rb) + dev;
-        // closest approach of the ray's line and the chord AB
-        const f3 e = B - A, w0 = o - A;
-        const float b = dot3(d, e), c = dot3(e, e), dd = dot3(d, w0), ee = dot3(e, w0);
-        const float den = a * c - b * b;
-        float sc = den > 0.0f ? (a * ee - b * dd) / den : 0.0f;
-        sc = fminf(fmaxf(sc, 0.0f), 1.0f);
-        const float tc = (sc * b - dd) * ray.inv_a;
-        const f3 x = (o + d * tc) - (A + e * sc);
-        const float reach = (R + sqrtf(c)) * ray.inv_len;
-        float tl;
-        if (dot3(x, x) <= R * R * 1.0001f && tc + reach >= tnear && tc - reach <= best &&
-            capsule_entry_bound(ray, A, B, R * 1.0001f, tl) && tl <= best) {
-            const float lo = fmaxf((float)k * h - 0.5f * h, 0.0f);
-            const float hi = fminf((float)(k + 1) * h + 0.5f * h, 1.0f);
-            const float ug = curve_golden(s, ray, lo, hi, false);
-            float tg;
-            if (curve_ball(s, ray, ug, tg) <= 0.0f) {
-                // the run of crossed balls around ug within [lo, hi]
-                float l = lo, r = hi, t;
-                if (curve_ball(s, ray, l, t) > 0.0f) {
-                    float p = l, q = ug;
-                    for (int i = 0; i < kCurveIters; ++i) {
-                        const float m = 0.5f * (p + q);
-                        if (curve_ball(s, ray, m, t) <= 0.0f) q = m;
-                        else p = m;
-                    }
-                    l = q;
-                }
-                if (curve_ball(s, ray, r, t) > 0.0f) {
-                    float p = ug, q = r;
-                    for (int i = 0; i < kCurveIters; ++i) {
-                        const float m = 0.5f * (p + q);
-                        if (curve_ball(s, ray, m, t) <= 0.0f) p = m;
-                        else q = m;
-                    }
-                    r = p;
-                }
-                const float u = curve_golden(s, ray, l, r, true);
-                if (curve_ball(s, ray, u, t) <= 0.0f && t >= tnear && t <= best) {
-                    best = t;
-                    bu = u;
-                    found = true;
-                    if (ANY) break;
-                }
-            }
+    curve_eval(s, 1.0f, B, rb);
+    return capsule_may_hit(ray, a, A, B, fmaxf(ra, rb) + 0.125f * (m2 + m2r), tnear, best);
+}
+
+SGPU_HD float curve_deviation(float m2, float m2r)
+{
+    const float h = 1.0f / kCurvePieces;
+    return h * h * 0.125f * (m2 + m2r);
+}
+
+// Piece k with its ends' balls (A, ra), (B, rb) at parameters k h and (k + 1) h.
+SGPU_HD bool curve_piece_candidate(const CurveRay& ray, float a, f3 A, float ra, f3 B, float rb, float dev, float tnear,
+                                   float best)
+{
+    return capsule_may_hit(ray, a, A, B, fmaxf(ra, rb) + dev, tnear, best);
+}
+
+// The range searched for piece k: the piece widened by half a piece each side.
+SGPU_HD void curve_piece_range(int k, float& lo, float& hi)
+{
+    const float h = 1.0f / kCurvePieces;
+    lo = fmaxf((float)k * h - 0.5f * h, 0.0f);
+    hi = fminf((float)(k + 1) * h + 0.5f * h, 1.0f);
+}
+
+// The ball of piece k's range nearest the line: true when the line crosses it.
+SGPU_HD bool curve_piece_search(const CurveSeg& s, const CurveRay& ray, int k, float& ug)
+{
+    float lo, hi, t;
+    curve_piece_range(k, lo, hi);
+    ug = curve_golden(s, ray, lo, hi, false);
+    return curve_ball(s, ray, ug, t) <= 0.0f;
+}
+
+// The least entry over the run of crossed balls around ug within piece k's range: true when it lies in
+// [tnear, best].
+SGPU_HD bool curve_piece_entry(const CurveSeg& s, const CurveRay& ray, int k, float ug, float tnear, float best, float& t,
+                               float& u)
+{
+    float l, r;
+    curve_piece_range(k, l, r);
+    if (curve_ball(s, ray, l, t) > 0.0f) {
+        float p = l, q = ug;
+        for (int i = 0; i < kCurveIters; ++i) {
+            const float m = 0.5f * (p + q);
+            if (curve_ball(s, ray, m, t) <= 0.0f) q = m;
+            else p = m;
         }
-        A = B;
-        ra = rb;
+        l = q;
     }
-    if (!found) return false;
-    const f3 X = o + d * best;
-    bu = curve_contact(s, X, bu);
-    t_out = best;
-    u_out = bu;
+    if (curve_ball(s, ray, r, t) > 0.0f) {
+        float p = ug, q = r;
+        for (int i = 0; i < kCurveIters; ++i) {
+            const float m = 0.5f * (p + q);
+            if (curve_ball(s, ray, m, t) <= 0.0f) p = m;
+            else q = m;
+        }
+        r = p;
+    }
+    u = curve_golden(s, ray, l, r, true);
+    return curve_ball(s, ray, u, t) <= 0.0f && t >= tnear && t <= best;
+}
+
+// The hit at entry t of ball u: the contact parameter of the hit point and the normal.
+SGPU_HD void curve_finish(const CurveSeg& s, f3 o, f3 d, float t, float u, float& u_out, f3& ng)
+{
+    const f3 X = o + d * t;
+    u_out = curve_contact(s, X, u);
     f3 P;
     float r;
-    curve_eval(s, bu, P, r);
+    curve_eval(s, u_out, P, r);
     ng = X - P;
-    return true;
 }
 
 }  // namespace sgpu

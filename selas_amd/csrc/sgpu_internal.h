@@ -7,6 +7,7 @@
 #include "sgpu_surface.h"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <string>
@@ -80,17 +81,21 @@ struct InstNode {
     float4 w2l[3];
 };
 static_assert(sizeof(InstNode) == kSlotBytes, "an instance node takes a node's first slot");
-// Round B-spline curve segment, 80 B, in curve-tree leaf order: the four control points (xyz,
-// radius; in world space, also for the curves of an instanced scene's placed scenes, which are
-// carried into world space at its commit), the geometry id (in the placed scene for an instanced
-// scene), the segment's index within its geometry and the composed instance (SGPU_INVALID_ID in a
-// scene of geometries).
+// Round B-spline curve segment as a build takes it: the four control points (xyz, radius; in world
+// space, also for the curves of an instanced scene's placed scenes, which are carried into world space
+// at its commit), the geometry id (in the placed scene for an instanced scene), the segment's index
+// within its geometry and the composed instance (SGPU_INVALID_ID in a scene of geometries).
 struct CurveRecord {
     float4 p[4];
     uint32_t geom, prim, inst, pad;
 };
 static_assert(sizeof(CurveRecord) == 80, "CurveRecord must be 80 bytes");
-// Stack entries of the curve tree's traversal (a binary tree: its depth must stay below this).
+// A segment's control points as a slot of the curve tree's array (its leaf records).
+struct CurvePoints {
+    float4 p[4];
+};
+static_assert(sizeof(CurvePoints) == kSlotBytes, "CurvePoints must be a slot");
+// The depth a curve's binary tree must stay below.
 constexpr uint32_t kCurveStack = 96;
 
 // 32-bit words of the LDS part of the per-lane traversal stack; deeper entries spill to global memory.
@@ -149,10 +154,13 @@ struct sgpu_scene_s {
     // its geometry and index within it; kept after commit for the scenes that place this one
     std::vector<float> curve_cp;
     std::vector<uint32_t> curve_geom, curve_prim;
-    // the curve tree (binary, over the segments, or over the placed scenes' curves carried into world
-    // space for an instanced scene) and its records in leaf order
+    // the curve tree (8-wide, over the segments, or over the placed scenes' curves carried into world
+    // space for an instanced scene), the ids of its segments by slot (geom, prim, inst, place in the
+    // order of d_cnodes's leaves), and the binary tree that orders hits at equal distance
+    WideNode* d_cwide = nullptr;
+    uint4* d_cids = nullptr;
+    uint32_t n_cslots = 0;
     BvhNode* d_cnodes = nullptr;
-    CurveRecord* d_curves = nullptr;
     uint32_t n_curves = 0;
     bool committed = false;
     uint32_t n_tris = 0;
@@ -317,7 +325,7 @@ struct sgpu_scratch {
     {
         const size_t bytes = (count * sizeof(T) + 511) & ~(size_t)255;
         if (err != hipSuccess) return nullptr;
-        if (used + bytes > blocks.back().bytes && !grow(bytes)) return nullptr;
+        if (used + bytes > blocks.back().bytes && !grow(std::max(bytes, blocks.back().bytes / 2))) return nullptr;
         T* p = (T*)(blocks.back().dev + used);
         used += bytes;
         return p;
@@ -435,10 +443,15 @@ struct TraceScene {
     uint32_t n_tris;
     uint32_t n_inst;           // > 0: an instanced scene (wide = its top tree over `insts`)
     const InstRecord* insts;
-    const BvhNode* cnodes;     // curve tree (n_curves == 0: none)
-    const CurveRecord* curves;
+    const WideNode* cwide;     // curve tree (n_curves == 0: none), its segments' ids and their order
+    const uint4* cids;
+    const BvhNode* cnodes;
     uint32_t n_curves;
 };
+inline TraceScene sgpu_trace_scene(const sgpu_scene_s* s)
+{
+    return TraceScene{s->d_nodes, s->d_wide, s->n_tris, s->n_inst, s->d_inst, s->d_cwide, s->d_cids, s->d_cnodes, s->n_curves};
+}
 // One launch over rays of several scenes: ray i traverses table[ray_scene[i]] (device arrays);
 // stack_cap is the largest stack_cap of the table's scenes.
 // instanced: some entries are instanced scenes (then comp_out, if not NULL, receives each closest
@@ -451,13 +464,16 @@ int sgpu_trace_launch_multi(sgpu_context ctx, const TraceScene* table, const uin
                             uint32_t* comp_out = nullptr, bool curves = false);
 // The curve pass (sgpu_curve.hip): after a triangle pass over the same rays, the curve tree's hits
 // closer than the ray's current hit (hits->t, which the triangle pass wrote: its hit or tfar)
-// replace it; for any-hit queries, rays not yet occluded are tested. One scene (nodes, curves,
-// n_curves; insts / inst_ids of an instanced scene, or NULL) or a table (then ray_scene).
-int sgpu_curve_launch(const BvhNode* nodes, const CurveRecord* curves, uint32_t n_curves, const InstRecord* insts,
-                      const uint32_t* inst_ids, const TraceScene* table, const uint32_t* ray_scene,
-                      const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded, uint32_t n,
-                      bool any_hit, const uint32_t* n_ptr, uint32_t* comp_out, uint32_t* overflow,
-                      hipStream_t stream, uint64_t* stats = nullptr);
+// replace it; for any-hit queries, rays not yet occluded are tested. One scene (inst_ids of an instanced
+// one, or NULL) or a table (then ray_scene); stack_words bounds the stacks. `spill`: the buffer lent to
+// the triangle pass (used again; max_blocks caps the grid where it holds no more), or NULL.
+int sgpu_curve_launch(sgpu_context ctx, const TraceScene& scene, const uint32_t* inst_ids, uint32_t stack_words,
+                      const TraceScene* table, const uint32_t* ray_scene, const sgpu_rays_soa* rays,
+                      const sgpu_hits_soa* hits, uint32_t* occluded, uint32_t n, bool any_hit, const uint32_t* n_ptr,
+                      uint32_t* comp_out, uint32_t* overflow, hipStream_t stream, uint32_t* spill,
+                      uint32_t max_blocks = 0, uint64_t* stats = nullptr);
+// Words of a spill buffer for a traversal grid of `threads` lanes (sgpu_trace.hip).
+size_t sgpu_trace_spill_words(uint32_t stack_words, size_t threads);
 // Builds the curve tree of a scene of geometries from its segments, or of an instanced scene from
 // the curves of its composed instances (sgpu_bvh.hip; called by the builds above).
 int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::vector<uint32_t>& geom,

@@ -13,11 +13,13 @@
 //   barycentric accept: U >= 0 && V >= 0 && U + V <= a
 //   t = T / a, u = U / a, v = V / a (IEEE division); accept tnear < t <= tfar.
 // Closest hit: smallest t, ties to the smaller global triangle index (= smaller (geomID, primID)).
-#include "sgpu_internal.h"
+#include "sgpu_wide.h"
 
 #include <algorithm>
 
 namespace {
+
+using sgpu::safe_rcp;
 
 // The test but for the barycentrics' divisions: u = U / a, v = V / a of the hit kept in the end.
 __device__ __forceinline__ bool tri_hit(const TriRecord& r, const f3& o, const f3& d, float tnear, float& t, float& U,
@@ -54,14 +56,6 @@ __device__ __forceinline__ bool tri_test(const TriRecord& r, const f3& o, const 
     v = V / a;
     return true;
 }
-
-__device__ __forceinline__ float safe_rcp(float x)
-{
-    float ax = fabsf(x);
-    float y = ax < 1e-20f ? copysignf(1e-20f, x) : x;
-    return __builtin_amdgcn_rcpf(y);
-}
-
 
 // The query's result: occlusion flag, or Embree's hit fields (quad hits reported as the quad and its
 // own (u, v): triangle 2q + h of quad q, second triangle (1 - u, 1 - v)).
@@ -247,14 +241,6 @@ __device__ __forceinline__ f3 inst_vector(const float4* w, f3 v)
 }
 
 
-// Compare-exchange of sort keys, ascending.
-__device__ __forceinline__ void cswap(int& a, int& b)
-{
-    const int lo = min(a, b);
-    b = max(a, b);
-    a = lo;
-}
-
 // Wide nodes of a single-scene launch that may be kept in LDS (sgpu_tuning.trace_lds_nodes): the root
 // and the next breadth-first nodes (the root's children when it has 8 internal ones), visited by
 // nearly every ray. Measured on MI355X they hit in L1/L2 anyway, and the LDS branch costs 1-3 %.
@@ -271,20 +257,13 @@ constexpr int kNext = -2;             // a lane that takes its next node once it
 // every lane has at most one 64-byte slot to read: a triangle to test, or else a node to visit.
 // (Letting the lanes with triangles wait until 4, 8 or 16 of a wave have one cost 1-25 %.)
 //
-// Slots are fetched by the wave together: lane l asks for 16 bytes of the slot of lane 16 k + l / 4
-// in the k-th of four loads, straight into LDS, and each lane reads its own slot from there. A
-// divergent 16-byte load costs the address unit two cycles a lane whatever it hits; read lane by lane
-// (5 loads a node, 3 a triangle) the traversal workload kept that unit busy 84 % of the time.
-// The 16-byte pieces of a slot are permuted by bits 2-3 of its lane, so that the reads' banks differ.
-//
-// Node visit: the 8 quantized child boxes are slab-tested in registers, near and far planes picked
-// by the direction's signs, each plane one fused multiply-add t = q (2^e / d) + (origin - o) / d.
-// Leaf children hit become the lane's triangles to test (a slot base and a mask). Internal children
-// hit become a group: the base of the node's children and a list of their numbers, 4 bits each
-// (closest hit: by entry distance, a min/max network over keys that carry the number in their low
-// bits; any hit: the mask, in order). The group being walked is in registers, the groups above it on
-// the stack, so a visit pushes or pops one 8-byte entry at most and the stack is as deep as the tree.
-// Hits are the triangle test's, independent of the tree and of the visiting order.
+// Slots are fetched by the wave together (WaveFetch). A node visit (wide_boxes) turns leaf children hit
+// into the lane's triangles to test (a slot base and a mask) and internal children hit into a group:
+// the base of the node's children and a list of their numbers, 4 bits each (closest hit: by entry
+// distance, a min/max network over keys that carry the number in their low bits; any hit: the mask, in
+// order). The group being walked is in registers, the groups above it on the stack, so a visit pushes
+// or pops one 8-byte entry at most and the stack is as deep as the tree. Hits are the triangle test's,
+// independent of the tree and of the visiting order.
 //
 // INST: scenes of instances. Leaves of the top tree are nodes (InstNode); visiting one saves the
 // group, pushes an exit entry (an empty group), moves the ray into the instance's space (t keeps its
@@ -349,11 +328,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
     uint32_t pfirst = 0, pbase = 0, pmask = 0;  // triangles to test: slot of leaf 0, base of the others, mask
     uint32_t sp = 0;
 
-    // this wave's part of lds_slots and the lane's place in the fetches
-    const uint32_t wl = threadIdx.x & 63u;
-    uint4* const wave_slots = lds_slots + 4 * 64 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t piece = (wl & 3u) ^ ((wl >> 4) & 3u);
-    const uint32_t own = 4 * wl, swz = (wl >> 2) & 3u;
+    const sgpu::WaveFetch wf(lds_slots);
 
     auto load_ray = [&](bool with_range) {
         o = mk3(rays.org_x[i], rays.org_y[i], rays.org_z[i]);
@@ -397,15 +372,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
                 cur = SGPU_INVALID_ID;
             }
         }
-        if (glist == 0) {
-            node = -1;
-        } else if (ANY) {
-            node = (int)(gbase + 2u * (uint32_t)__builtin_ctz(glist));
-            glist &= glist - 1;
-        } else {
-            node = (int)(gbase + 2u * (glist & 7u));
-            glist >>= 4;
-        }
+        node = glist ? sgpu::wide_take<ANY>(gbase, glist) : -1;
     };
 
     for (;;) {
@@ -492,37 +459,14 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
             slot = (int)(k == 0 ? pfirst : pbase + k);
             pmask &= pmask - 1;
         }
-        // ---- the slots, fetched together ----
-        {
-            const bool in_top = TOP && (uint32_t)slot < 2 * n_top && visit;
-            const int ask = in_top ? -1 : slot;
-            unsigned long long from[4];
-            int s[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int src = 4 * (16 * k + (int)(wl >> 2));
-                const unsigned long long at = (unsigned long long)rw;
-                s[k] = __builtin_amdgcn_ds_bpermute(src, ask);
-                from[k] = at;
-                if (MULTI || INST)
-                    from[k] = (unsigned long long)(uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)at) |
-                              (unsigned long long)(uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)(at >> 32)) << 32;
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (s[k] >= 0)
-                    __builtin_amdgcn_global_load_lds(
-                        (const __attribute__((address_space(1))) uint32_t*)(from[k] + (unsigned long long)(uint32_t)s[k] * kSlotBytes + 16 * piece),
-                        (__attribute__((address_space(3))) uint32_t*)(wave_slots + 64 * k), 16, 0, 0);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
+        const bool in_top = TOP && visit && (uint32_t)slot < 2 * n_top;
+        wf.fetch<MULTI || INST>(in_top ? -1 : slot, rw);
         uint4 w0, w1, w2, w3;
-        if (TOP && visit && (uint32_t)slot < 2 * n_top) {
+        if (in_top) {
             const uint4* t = lds_top + 2 * slot;
             w0 = t[0], w1 = t[1], w2 = t[2], w3 = t[3];
         } else {
-            w0 = wave_slots[own + (0 ^ swz)], w1 = wave_slots[own + (1 ^ swz)];
-            w2 = wave_slots[own + (2 ^ swz)], w3 = wave_slots[own + (3 ^ swz)];
+            w0 = wf.read(0), w1 = wf.read(1), w2 = wf.read(2), w3 = wf.read(3);
         }
         if (test) {
             // ---- one triangle test ----
@@ -556,8 +500,7 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
         }
         if (visit) {
             // ---- one node visit ----
-            const uint32_t meta = w0.w;
-            if (INST && (meta >> 28) == 0) {
+            if (INST && (w0.w >> 28) == 0) {
                 // an instance: into its space, at its root
                 if (glist) push(gbase, glist);
                 push(0, 0);
@@ -574,60 +517,14 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
                 glist = 0;
             } else {
                 if (STATS) ++cnt_nodes;
-                const uint32_t ni = (meta >> 24) & 15u, nch = meta >> 28;
-                // per axis: slope a (per quantization step) and intercept b of the planes' distances
-                const float ax = __builtin_amdgcn_ldexpf(inv.x, (int)(meta << 24) >> 24);
-                const float ay = __builtin_amdgcn_ldexpf(inv.y, (int)(meta << 16) >> 24);
-                const float az = __builtin_amdgcn_ldexpf(inv.z, (int)(meta << 8) >> 24);
-                const float bx = fmaf(__uint_as_float(w0.x & kOriginMask), inv.x, -oinv.x);
-                const float by = fmaf(__uint_as_float(w0.y & kOriginMask), inv.y, -oinv.y);
-                const float bz = fmaf(__uint_as_float(w0.z & kOriginMask), inv.z, -oinv.z);
-                const uint32_t base = (w0.x & ~kOriginMask) | (w0.y & ~kOriginMask) << 11 | w0.z << 22;
-                const bool sx = __float_as_int(inv.x) < 0, sy = __float_as_int(inv.y) < 0, sz = __float_as_int(inv.z) < 0;
-                const uint32_t nx[2] = {sx ? w2.z : w1.x, sx ? w2.w : w1.y}, fx[2] = {sx ? w1.x : w2.z, sx ? w1.y : w2.w};
-                const uint32_t ny[2] = {sy ? w3.x : w1.z, sy ? w3.y : w1.w}, fy[2] = {sy ? w1.z : w3.x, sy ? w1.w : w3.y};
-                const uint32_t nz[2] = {sz ? w3.z : w2.x, sz ? w3.w : w2.y}, fz[2] = {sz ? w2.x : w3.z, sz ? w2.y : w3.w};
-                int key[8];
-                uint32_t hit = 0;
-#pragma unroll
-                for (int c = 7; c >= 0; --c) {
-                    const int sh = 8 * (c & 3), wi = c >> 2;
-                    const float t0x = fmaf((float)((nx[wi] >> sh) & 0xFFu), ax, bx);
-                    const float t0y = fmaf((float)((ny[wi] >> sh) & 0xFFu), ay, by);
-                    const float t0z = fmaf((float)((nz[wi] >> sh) & 0xFFu), az, bz);
-                    const float t1x = fmaf((float)((fx[wi] >> sh) & 0xFFu), ax, bx);
-                    const float t1y = fmaf((float)((fy[wi] >> sh) & 0xFFu), ay, by);
-                    const float t1z = fmaf((float)((fz[wi] >> sh) & 0xFFu), az, bz);
-                    const float tmin = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tnear));
-                    const float tmax = fminf(fminf(t1x, t1y), fminf(t1z, best_t));
-                    const bool in = tmin <= tmax;
-                    hit = hit + hit + (in ? 1u : 0u);
-                    // internal children: entry distance as the sort key, the slot (and 8) in its low bits
-                    if (!ANY) key[c] = in && (uint32_t)c < ni ? (__float_as_int(tmin) & ~15) | (8 | c) : 0x7FFFFFF0;
-                }
-                pmask = __builtin_amdgcn_ubfe(hit, ni, nch - ni);
+                const sgpu::WideHits h = sgpu::wide_boxes<ANY>(w0, w1, w2, w3, inv, oinv, tnear, best_t);
+                pmask = h.leaves;
                 pfirst = (uint32_t)node + 1;
-                pbase = base + 2 * ni - 1;
-                uint32_t list;
-                if (ANY) {
-                    list = __builtin_amdgcn_ubfe(hit, 0, ni);
-                } else {
-                    // Batcher's odd-even merge sort network for 8 keys
-                    cswap(key[0], key[1]); cswap(key[2], key[3]); cswap(key[4], key[5]); cswap(key[6], key[7]);
-                    cswap(key[0], key[2]); cswap(key[1], key[3]); cswap(key[4], key[6]); cswap(key[5], key[7]);
-                    cswap(key[1], key[2]); cswap(key[5], key[6]);
-                    cswap(key[0], key[4]); cswap(key[1], key[5]); cswap(key[2], key[6]); cswap(key[3], key[7]);
-                    cswap(key[2], key[4]); cswap(key[3], key[5]);
-                    cswap(key[1], key[2]); cswap(key[3], key[4]); cswap(key[5], key[6]);
-                    // the low 4 bits of each key, the nearest lowest
-                    list = 0;
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) list = __builtin_amdgcn_alignbit((uint32_t)key[c], list, 4);
-                }
-                if (list) {
+                pbase = h.leaf_base;
+                if (h.list) {
                     if (glist) push(gbase, glist);
-                    gbase = base;
-                    glist = list;
+                    gbase = h.base;
+                    glist = h.list;
                 }
                 node = kNext;
             }
@@ -650,15 +547,14 @@ __global__ void k_zero_work(uint32_t* __restrict w)
     if (threadIdx.x < kTraceWorkWords) w[threadIdx.x] = 0u;
 }
 
-// Words of a spill buffer for a grid of `threads` lanes: the ray counters, then each lane's stack
-// words past those in LDS.
-size_t spill_words(uint32_t stack_words, size_t threads)
+}  // namespace
+
+// The ray counters, then each lane's stack words past those in LDS.
+size_t sgpu_trace_spill_words(uint32_t stack_words, size_t threads)
 {
     const uint32_t deep = stack_words > SGPU_STACK_LDS ? stack_words - SGPU_STACK_LDS : 1;
     return kTraceWorkWords + deep * threads;
 }
-
-}  // namespace
 
 void sgpu_trace_work_zero(uint32_t* spill, hipStream_t stream)
 {
@@ -694,7 +590,9 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
     uint32_t* buf = spill_buf;
     if (!buf && (counts || stack_words > SGPU_STACK_LDS))
         SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
-                                    spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) * sizeof(uint32_t), stream));
+                                    sgpu_trace_spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) *
+                                        sizeof(uint32_t),
+                                    stream));
     uint32_t* const work = buf;
     uint32_t* const spill = buf ? buf + kTraceWorkWords : nullptr;
     sgpu_hits_soa h = {};
@@ -750,7 +648,7 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
 size_t sgpu_trace_spill_words(sgpu_context ctx, uint32_t stack_words)
 {
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    return spill_words(stack_words, (size_t)cus * kMaxTraceBlocksPerCu * SGPU_TRACE_BLOCK);
+    return sgpu_trace_spill_words(stack_words, (size_t)cus * kMaxTraceBlocksPerCu * SGPU_TRACE_BLOCK);
 }
 
 size_t sgpu_trace_spill_words(sgpu_scene scene) { return sgpu_trace_spill_words(scene->ctx, scene->stack_cap); }
@@ -760,17 +658,15 @@ int sgpu_trace_launch(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hi
                       const uint32_t* n_ptr, uint32_t* overflow, uint32_t* comp_out, uint32_t max_blocks,
                       uint64_t* curve_stats)
 {
-    const TraceScene ts{scene->d_nodes, scene->d_wide,   scene->n_tris,   scene->n_inst,
-                        scene->d_inst,  scene->d_cnodes, scene->d_curves, scene->n_curves};
+    const TraceScene ts = sgpu_trace_scene(scene);
     const int rc = trace_launch(scene->ctx, ts, scene->n_wide, scene->d_inst_ids,
                                 scene->ctx->trace_tree == 1 ? scene->wide_stack : scene->stack_cap,
                                 overflow ? overflow : scene->d_overflow, nullptr, nullptr, rays, hits, occluded, n,
                                 any_hit, d_stats, stream, spill_buf, n_ptr, !scene->instances.empty(), comp_out,
                                 max_blocks);
     if (rc != SGPU_OK || scene->n_curves == 0) return rc;
-    return sgpu_curve_launch(scene->d_cnodes, scene->d_curves, scene->n_curves, scene->d_inst, scene->d_inst_ids,
-                             nullptr, nullptr, rays, hits, occluded, n, any_hit, n_ptr, comp_out,
-                             overflow ? overflow : scene->d_overflow, stream, curve_stats);
+    return sgpu_curve_launch(scene->ctx, ts, scene->d_inst_ids, scene->wide_stack, nullptr, nullptr, rays, hits, occluded, n, any_hit, n_ptr, comp_out,
+                             overflow ? overflow : scene->d_overflow, stream, spill_buf, max_blocks, curve_stats);
 }
 
 int sgpu_trace_launch_multi(sgpu_context ctx, const TraceScene* table, const uint32_t* ray_scene, uint32_t stack_cap,
@@ -782,6 +678,6 @@ int sgpu_trace_launch_multi(sgpu_context ctx, const TraceScene* table, const uin
     const int rc = trace_launch(ctx, TraceScene{}, 0, nullptr, stack_cap, overflow, table, ray_scene, rays, hits, occluded,
                                 n, any_hit, d_stats, stream, spill_buf, n_ptr, instanced, comp_out);
     if (rc != SGPU_OK || !curves) return rc;
-    return sgpu_curve_launch(nullptr, nullptr, 0, nullptr, nullptr, table, ray_scene, rays, hits, occluded, n, any_hit,
-                             n_ptr, comp_out, overflow, stream);
+    return sgpu_curve_launch(ctx, TraceScene{}, nullptr, stack_cap, table, ray_scene, rays, hits, occluded, n, any_hit,
+                             n_ptr, comp_out, overflow, stream, spill_buf);
 }

@@ -1337,9 +1337,7 @@ int server_upload_table(sgpu_vcm_server sv, hipStream_t stream)
         SGPU_HIP_TRY(hipHostMalloc((void**)&sv->h_table, sizeof(TraceScene) * sv->table_cap, hipHostMallocDefault));
     }
     for (uint32_t k = 0; k < n; ++k)
-        sv->h_table[k] = TraceScene{sv->scenes[k]->d_nodes, sv->scenes[k]->d_wide, sv->scenes[k]->n_tris,
-                                    sv->scenes[k]->n_inst,  sv->scenes[k]->d_inst, sv->scenes[k]->d_cnodes,
-                                    sv->scenes[k]->d_curves, sv->scenes[k]->n_curves};
+        sv->h_table[k] = sgpu_trace_scene(sv->scenes[k]);
     SGPU_HIP_TRY(hipMemcpyAsync(sv->d_table, sv->h_table, sizeof(TraceScene) * n, hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     sv->table_dirty = false;
