@@ -263,39 +263,6 @@ SGPU_HD f3 disney_fresnel(const Surface& s, f3 wo, f3 wm, f3 wi)
     f3 mf = schlick3(r0, dot3(wi, wm));
     return lerp3(mk3(df, df, df), mf, s.metallic);
 }
-SGPU_HD f3 eval_brdf(const Surface& s, f3 wo, f3 wm, f3 wi, float& fpdf, float& rpdf)
-{
-    fpdf = 0.0f;
-    rpdf = 0.0f;
-    float nl = cos_theta(wi), nv = cos_theta(wo);
-    if (nl <= 0.0f || nv <= 0.0f) return mk3(0, 0, 0);
-    float ax, ay;
-    aniso_params(s.roughness, s.anisotropic, ax, ay);
-    float d = d_aniso(wm, ax, ay);
-    float gl = g1_aniso(wi, ax, ay), gv = g1_aniso(wo, ax, ay);
-    f3 f = disney_fresnel(s, wo, wm, wi);
-    vndf_pdf(wi, wm, wo, ax, ay, fpdf, rpdf);
-    fpdf *= (1.0f / (4 * absf_(dot3(wo, wm))));
-    rpdf *= (1.0f / (4 * absf_(dot3(wi, wm))));
-    float k = d * gl * gv;
-    float den = 4.0f * nl * nv;
-    return mk3(k * f.x / den, k * f.y / den, k * f.z / den);
-}
-SGPU_HD f3 eval_spec_trans(const Surface& s, f3 wo, f3 wm, f3 wi, float ax, float ay, bool thin)
-{
-    float rel = s.relative_ior;
-    float n2 = rel * rel;
-    float nl = abs_cos_theta(wi), nv = abs_cos_theta(wo);
-    float hl = dot3(wm, wi), hv = dot3(wm, wo);
-    float ahl = absf_(hl), ahv = absf_(hv);
-    float d = d_aniso(wm, ax, ay);
-    float gl = g1_aniso(wi, ax, ay), gv = g1_aniso(wo, ax, ay);
-    float f = fresnel_dielectric(hv, 1.0f, s.ior);
-    f3 color = thin ? sqrt3(s.base_color) : s.base_color;
-    float c = (ahl * ahv) / (nl * nv);
-    float t = (n2 / sq(hl + rel * hv));
-    return color * c * t * (1.0f - f) * gl * gv * d;
-}
 SGPU_HD float eval_retro(const Surface& s, f3 wo, f3 wi)
 {
     float nl = abs_cos_theta(wi), nv = abs_cos_theta(wo);
@@ -321,56 +288,164 @@ SGPU_HD float eval_diffuse(const Surface& s, f3 wo, f3 wm, f3 wi, bool thin)
     return kInvPi * (retro + sub_approx * (1.0f - 0.5f * fl) * (1.0f - 0.5f * fv));
 }
 
-// EvaluateDisney (Disney.cpp:525-614): returns f * |cos(theta_l)|, forward and reverse pdfs.
-SGPU_HD f3 disney_eval(const Surface& s, f3 v, f3 l, bool thin, float& fwd, float& rev)
+// ---- EvaluateDisney (Disney.cpp:525-614) in two parts ------------------------------------------------
+//
+// What does not depend on the light's direction (the local view direction, the lobes' probabilities,
+// the GGX parameters and the view's masking, the normal-incidence reflectance, colours), computed once
+// for many directions of one surface and view, and the rest. Each operation is the one that evaluating
+// a direction by itself takes, on the same values in the same order, so both ways give the same bits.
+struct DisneyView {
+    f3 t, n, b;   // shading frame
+    f3 wo;        // the view direction in it
+    float nv, fv;  // |cos| of the view and its Schlick weight
+    float ax, ay, ax2, ay2, kd;  // GGX parameters, their squares, pi ax ay
+    float gv;                    // the view's masking
+    float tax, tay, tax2, tay2, tkd, tgv;  // the same of the transmission lobe
+    float p_brdf, p_diff, p_cc, p_trans, diff_w, trans_w;
+    float relative_ior, n2, ior, metallic, r2, flatness, clearcoat, clearcoat_gloss;
+    f3 r0;     // normal-incidence reflectance of the metallic Fresnel term
+    f3 base;   // base colour
+    f3 sheen;  // sheen colour times its weight (zero: none)
+    f3 trans;  // transmission colour
+    uint32_t bits;  // kView*
+};
+enum ViewBits : uint32_t { kViewThin = 1, kViewFront = 2, kViewSheen = 4, kViewSameAlpha = 8, kViewLambert = 16 };
+
+SGPU_HD float d_aniso_at(f3 wm, float ax2, float ay2, float kd)
 {
-    f3 wo = normalize3(to_local(s, v));
-    f3 wi = normalize3(to_local(s, l));
+    float hx2 = sq(wm.x), hy2 = sq(wm.z), c2 = cos2_theta(wm);
+    return 1.0f / (kd * sq(hx2 / ax2 + hy2 / ay2 + c2));
+}
+
+SGPU_HD void disney_view(const Surface& s, f3 v, bool thin, DisneyView& q)
+{
+    q.t = s.t;
+    q.n = s.n;
+    q.b = s.b;
+    q.wo = normalize3(to_local(s, v));
+    q.nv = abs_cos_theta(q.wo);
+    q.fv = schlick_weight(q.nv);
+    lobe_pdfs(s, q.p_brdf, q.p_diff, q.p_cc, q.p_trans);
+    q.diff_w = (1.0f - s.metallic) * (1.0f - s.spec_trans);
+    q.trans_w = (1.0f - s.metallic) * s.spec_trans;
+    aniso_params(s.roughness, s.anisotropic, q.ax, q.ay);
+    q.ax2 = sq(q.ax);
+    q.ay2 = sq(q.ay);
+    q.kd = kPi * q.ax * q.ay;
+    q.gv = g1_aniso(q.wo, q.ax, q.ay);
+    q.tax = q.ax;
+    q.tay = q.ay;
+    q.tax2 = q.ax2;
+    q.tay2 = q.ay2;
+    q.tkd = q.kd;
+    q.tgv = q.gv;
+    q.bits = (thin ? kViewThin : 0u) | (cos_theta(q.wo) > 0.0f ? kViewFront : 0u) | (s.sheen > 0.0f ? kViewSheen : 0u) |
+             kViewSameAlpha;
+    if (thin && q.trans_w > 0.0f) {
+        aniso_params(thin_trans_roughness(s.ior, s.roughness), s.anisotropic, q.tax, q.tay);
+        q.tax2 = sq(q.tax);
+        q.tay2 = sq(q.tay);
+        q.tkd = kPi * q.tax * q.tay;
+        q.tgv = g1_aniso(q.wo, q.tax, q.tay);
+        q.bits &= ~(uint32_t)kViewSameAlpha;
+    }
+    q.relative_ior = s.relative_ior;
+    q.n2 = s.relative_ior * s.relative_ior;
+    q.ior = s.ior;
+    q.metallic = s.metallic;
+    q.r2 = s.roughness * s.roughness;
+    q.flatness = s.flatness;
+    q.clearcoat = s.clearcoat;
+    q.clearcoat_gloss = s.clearcoat_gloss;
+    f3 tint = tint_of(s.base_color);
+    f3 r0 = lerp3(mk3(1, 1, 1), tint, s.specular_tint) * schlick_r0(s.relative_ior);
+    q.r0 = lerp3(r0, s.base_color, s.metallic);
+    q.base = s.base_color;
+    q.sheen = s.sheen > 0.0f ? lerp3(mk3(1, 1, 1), tint, s.sheen_tint) * s.sheen : mk3(0, 0, 0);
+    q.trans = thin ? sqrt3(s.base_color) : s.base_color;
+}
+
+// f * |cos(theta_l)| and the forward and reverse pdfs for the light direction l.
+SGPU_HD f3 disney_eval_view(const DisneyView& q, f3 l, float& fwd, float& rev)
+{
+    const f3 wo = q.wo;
+    f3 wi = normalize3(mk3(dot3(l, q.t), dot3(l, q.n), dot3(l, q.b)));
     f3 wm = normalize3(wo + wi);
-    float nv = cos_theta(wo), nl = cos_theta(wi);
+    const float cl = cos_theta(wi), nl = absf_(cl), nv = q.nv;
+    const float hl = dot3(wm, wi), hv = dot3(wm, wo);
     f3 refl = mk3(0, 0, 0);
     fwd = 0.0f;
     rev = 0.0f;
-    float p_brdf, p_diff, p_cc, p_trans;
-    lobe_pdfs(s, p_brdf, p_diff, p_cc, p_trans);
-    float diff_w = (1.0f - s.metallic) * (1.0f - s.spec_trans);
-    float trans_w = (1.0f - s.metallic) * s.spec_trans;
-    bool upper = nl > 0.0f && nv > 0.0f;
-    if (upper && s.clearcoat > 0.0f) {
+    const bool upper = cl > 0.0f && (q.bits & kViewFront);
+    if (upper && q.clearcoat > 0.0f) {
         float fcc, rcc;
-        float cc = eval_clearcoat(s.clearcoat, s.clearcoat_gloss, wo, wm, wi, fcc, rcc);
+        float cc = eval_clearcoat(q.clearcoat, q.clearcoat_gloss, wo, wm, wi, fcc, rcc);
         refl += mk3(cc, cc, cc);
-        fwd += p_cc * fcc;
-        rev += p_cc * rcc;
+        fwd += q.p_cc * fcc;
+        rev += q.p_cc * rcc;
     }
-    if (diff_w > 0.0f) {
-        float fd = abs_cos_theta(wi), rd = abs_cos_theta(wo);
-        float diffuse = eval_diffuse(s, wo, wm, wi, thin);
-        f3 sheen = eval_sheen(s, wm, wi);
-        refl += (s.base_color * diffuse + sheen) * diff_w;
-        fwd += p_diff * fd;
-        rev += p_diff * rd;
+    if (q.diff_w > 0.0f) {
+        // diffuse with retro-reflection (and the thin surfaces' subsurface approximation), sheen
+        const float fl = schlick_weight(nl);
+        float hk = 0.0f;
+        const bool thin = (q.bits & kViewThin) != 0;
+        if (thin && q.flatness > 0.0f) {
+            float fss90 = hl * hl * q.r2;
+            float fss = lerp_(1.0f, fss90, fl) * lerp_(1.0f, fss90, q.fv);
+            hk = 1.25f * (fss * (1.0f / (nl + nv) - 0.5f) + 0.5f);
+        }
+        float rr = 0.5f + 2.0f * nl * nl * q.r2;
+        float retro = rr * (fl + q.fv + fl * q.fv * (rr - 1.0f));
+        float sub_approx = lerp_(1.0f, hk, thin ? q.flatness : 0.0f);
+        float diffuse = kInvPi * (retro + sub_approx * (1.0f - 0.5f * fl) * (1.0f - 0.5f * q.fv));
+        f3 sheen = mk3(0, 0, 0);
+        if (q.bits & kViewSheen) sheen = q.sheen * schlick_weight(absf_(hl));
+        refl += (q.base * diffuse + sheen) * q.diff_w;
+        fwd += q.p_diff * nl;
+        rev += q.p_diff * nv;
     }
-    if (trans_w > 0.0f) {
-        float rscaled = thin ? thin_trans_roughness(s.ior, s.roughness) : s.roughness;
-        float tax, tay;
-        aniso_params(rscaled, s.anisotropic, tax, tay);
-        f3 tr = eval_spec_trans(s, wo, wm, wi, tax, tay, thin);
-        refl += tr * trans_w;
-        float ft, rt;
-        vndf_pdf(wi, wm, wo, tax, tay, ft, rt);
-        float lh = dot3(wm, wi), vh = dot3(wm, wo);
-        fwd += p_trans * ft / (sq(lh + s.relative_ior * vh));
-        rev += p_trans * rt / (sq(vh + s.relative_ior * lh));
+    // the specular lobes share the distribution, the light's masking (where they share the GGX
+    // parameters: but for thin surfaces) and the dielectric Fresnel term
+    if (upper || q.trans_w > 0.0f) {
+        float d = d_aniso_at(wm, q.ax2, q.ay2, q.kd);
+        float gl = g1_aniso(wi, q.ax, q.ay);
+        const float df = fresnel_dielectric(hv, 1.0f, q.ior);
+        const float ahl = absf_(hl), ahv = absf_(hv);
+        if (q.trans_w > 0.0f) {
+            float td = d, tgl = gl;
+            if (!(q.bits & kViewSameAlpha)) {
+                td = d_aniso_at(wm, q.tax2, q.tay2, q.tkd);
+                tgl = g1_aniso(wi, q.tax, q.tay);
+            }
+            float c = (ahl * ahv) / (nl * nv);
+            float t = (q.n2 / sq(hl + q.relative_ior * hv));
+            f3 tr = q.trans * c * t * (1.0f - df) * tgl * q.tgv * td;
+            refl += tr * q.trans_w;
+            float ft = q.tgv * ahl * td / nl, rt = tgl * ahv * td / nv;
+            fwd += q.p_trans * ft / (sq(hl + q.relative_ior * hv));
+            rev += q.p_trans * rt / (sq(hv + q.relative_ior * hl));
+        }
+        if (upper) {
+            f3 mf = schlick3(q.r0, hl);
+            f3 f = lerp3(mk3(df, df, df), mf, q.metallic);
+            float fm = q.gv * ahl * d / nl, rm = gl * ahv * d / nv;
+            fm *= (1.0f / (4 * ahv));
+            rm *= (1.0f / (4 * ahl));
+            float k = d * gl * q.gv;
+            float den = 4.0f * nl * nv;
+            refl += mk3(k * f.x / den, k * f.y / den, k * f.z / den);
+            fwd += q.p_brdf * fm / (4 * ahv);
+            rev += q.p_brdf * rm / (4 * ahl);
+        }
     }
-    if (upper) {
-        float fm, rm;
-        f3 sp = eval_brdf(s, wo, wm, wi, fm, rm);
-        refl += sp;
-        fwd += p_brdf * fm / (4 * absf_(dot3(wo, wm)));
-        rev += p_brdf * rm / (4 * absf_(dot3(wi, wm)));
-    }
-    return refl * absf_(nl);
+    return refl * nl;
+}
+
+SGPU_HD f3 disney_eval(const Surface& s, f3 v, f3 l, bool thin, float& fwd, float& rev)
+{
+    DisneyView q;
+    disney_view(s, v, thin, q);
+    return disney_eval_view(q, l, fwd, rev);
 }
 
 SGPU_HD f3 extinction_of(f3 a, float sd)
@@ -616,6 +691,30 @@ SGPU_HD f3 bsdf_eval(const Surface& s, f3 v, f3 l, float& fwd, float& rev)
 {
     if (s.shader == kLambert) return lambert_eval(s, v, l, fwd, rev);
     return disney_eval(s, v, l, s.shader == kDisneyThin, fwd, rev);
+}
+
+// The same in two parts (disney_view): the view's of either shader, then a light direction.
+SGPU_HD void bsdf_view(const Surface& s, f3 v, DisneyView& q)
+{
+    if (s.shader == kLambert) {
+        q.n = s.n;
+        q.nv = dot3(s.n, v);
+        q.base = s.base_color;
+        q.bits = kViewLambert;
+        return;
+    }
+    disney_view(s, v, s.shader == kDisneyThin, q);
+}
+SGPU_HD f3 bsdf_eval_view(const DisneyView& q, f3 l, float& fwd, float& rev)
+{
+    if (!(q.bits & kViewLambert)) return disney_eval_view(q, l, fwd, rev);
+    fwd = 0.0f;
+    rev = 0.0f;
+    float nl = dot3(q.n, l);
+    if (nl <= 0.0f || q.nv <= 0.0f) return mk3(0, 0, 0);
+    fwd = nl * kInvPi;
+    rev = q.nv * kInvPi;
+    return q.base * (kInvPi * nl);
 }
 
 template <class U>
