@@ -253,6 +253,214 @@ template <bool ANY>
 constexpr int kRefill = ANY ? 8 : 16;
 constexpr int kNext = -2;             // a lane that takes its next node once its triangles are tested
 
+// Launches of few rays: eight lanes a ray, lane c testing child c of the node and, where that is a leaf,
+// its triangle, so that a visit is one box test long and the node's triangles are tested at once. A wave
+// of one ray per lane is a chain of some 40 trips of 400 instructions whatever it holds; up to kGroupRays
+// rays the chip has waves to spare and that chain is what a launch takes (61 rays: 107 -> 36 us; a 64 x 64
+// image of one vertex-merging iteration, 42 such launches: 2.57 -> 1.57 ms). What is left is a chain of
+// node and triangle fetches. The ray's stack holds (slot, entry distance) pairs in LDS, pushed by the
+// lanes that hit, far to near, and entries beyond the closest hit so far are dropped when popped. Hits
+// are the same bits (the ties of k_trace8).
+// The line: closest hits of random rays through 65 536 triangles take 271 us this way and 335 lane by lane
+// at 131 072 rays, 401 and 376 at 200 000; any hits through a million 220 and 273 at 98 304, 284 and 277
+// at 131 072; 1024 rays 80 and 253, 58 and 176.
+template <bool ANY>
+constexpr uint32_t kGroupRays = ANY ? 98304u : 131072u;
+constexpr uint32_t kGroupStack = 128;  // entries a ray's stack holds
+// The entries a tree can need whose 8-wide stack takes `words` words (two a level but two): a visit takes
+// one entry and leaves eight, on every level but the last, and an instanced ray has an exit entry.
+constexpr uint32_t group_stack(uint32_t words) { return 7 * (words / 2) + 9; }
+constexpr uint32_t kGroupExit = 0xFFFFFFFFu;  // the entry that returns to the top tree
+
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+
+// How many of the group's eight keys are smaller than this lane's (keys differ).
+__device__ __forceinline__ uint32_t group_rank(int k)
+{
+    const int m = dpp<0x141>(k);  // lane ^ 7
+    return (uint32_t)(dpp<0xB1>(k) < k) + (uint32_t)(dpp<0x4E>(k) < k) + (uint32_t)(dpp<0x1B>(k) < k) + (uint32_t)(m < k) +
+           (uint32_t)(dpp<0xB1>(m) < k) + (uint32_t)(dpp<0x4E>(m) < k) + (uint32_t)(dpp<0x1B>(m) < k);
+}
+
+template <bool ANY, bool STATS, bool MULTI, bool INST>
+__device__ void trace_groups(const TraceScene& scene, const uint32_t* __restrict inst_ids,
+                             const TraceScene* __restrict table, const uint32_t* __restrict ray_scene,
+                             const sgpu_rays_soa& rays, sgpu_hits_soa& hits, uint32_t* __restrict occluded, uint32_t n,
+                             unsigned long long* __restrict stats, uint32_t* __restrict comp_out, uint2* lds)
+{
+    const uint32_t gl = threadIdx.x & 7u, shift = threadIdx.x & 56u;
+    const uint32_t group = (blockIdx.x * SGPU_TRACE_BLOCK + threadIdx.x) >> 3, groups = gridDim.x * SGPU_TRACE_BLOCK >> 3;
+    uint2* const stack = lds + kGroupStack * (threadIdx.x >> 3);
+    const float inf = __int_as_float(0x7f800000);
+    unsigned long long cnt_nodes = 0, cnt_tris = 0;
+    for (uint32_t i = group; i < n; i += groups) {
+        f3 o, d, inv, oinv;
+        auto load_ray = [&]() {
+            o = mk3(rays.org_x[i], rays.org_y[i], rays.org_z[i]);
+            d = mk3(rays.dir_x[i], rays.dir_y[i], rays.dir_z[i]);
+        };
+        auto set_slopes = [&]() {
+            inv = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
+            oinv = mk3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+        };
+        load_ray();
+        set_slopes();
+        const float tnear = rays.tnear[i];
+        float best_t = rays.tfar[i];
+        const TraceScene ts = MULTI ? table[ray_scene[i]] : scene;
+        const WideNode* rw = ts.wide;
+        uint32_t best_key = 0xFFFFFFFFu, best_tri = 0xFFFFFFFFu, best_inst = SGPU_INVALID_ID, cur = SGPU_INVALID_ID;
+        float best_u = 0.0f, best_v = 0.0f, best_a = 1.0f;
+        bool hit_any = false;
+        uint32_t sp = 0;
+        int node = ts.n_tris > 0 || (INST && ts.n_inst > 0) ? 0 : -1;
+        // the node's header and this lane's child's box
+        uint4 w0;
+        uint32_t lx, ly, lz, hx, hy, hz;
+        auto fetch = [&]() {
+            const uint8_t* __restrict np = reinterpret_cast<const uint8_t*>(rw) + (size_t)(uint32_t)node * kSlotBytes;
+            w0 = *reinterpret_cast<const uint4*>(np);
+            lx = np[16 + gl], ly = np[24 + gl], lz = np[32 + gl];
+            hx = np[40 + gl], hy = np[48 + gl], hz = np[56 + gl];
+        };
+        if (node >= 0) fetch();
+        while (node >= 0) {
+            if (INST && (w0.w >> 28) == 0) {
+                // an instance: into its space, at its root
+                const InstNode* __restrict in = reinterpret_cast<const InstNode*>(rw) + node;
+                const float4 rows[3] = {in->w2l[0], in->w2l[1], in->w2l[2]};
+                const f3 wo = o, wd = d;
+                o = inst_point(rows, wo);
+                d = inst_vector(rows, wd);
+                set_slopes();
+                cur = w0.x;
+                rw = ts.insts[cur].wide;
+                stack[sp++] = make_uint2(kGroupExit, 0);
+                node = 0;
+                fetch();
+                continue;
+            }
+            if (STATS && gl == 0) ++cnt_nodes;
+            // this lane's child (wide_boxes' arithmetic)
+            const uint32_t meta = w0.w, ni = (meta >> 24) & 15u, nch = meta >> 28;
+            const float ax = __builtin_amdgcn_ldexpf(inv.x, (int)(meta << 24) >> 24);
+            const float ay = __builtin_amdgcn_ldexpf(inv.y, (int)(meta << 16) >> 24);
+            const float az = __builtin_amdgcn_ldexpf(inv.z, (int)(meta << 8) >> 24);
+            const float bx = fmaf(__uint_as_float(w0.x & kOriginMask), inv.x, -oinv.x);
+            const float by = fmaf(__uint_as_float(w0.y & kOriginMask), inv.y, -oinv.y);
+            const float bz = fmaf(__uint_as_float(w0.z & kOriginMask), inv.z, -oinv.z);
+            const uint32_t base = (w0.x & ~kOriginMask) | (w0.y & ~kOriginMask) << 11 | w0.z << 22;
+            const bool sx = __float_as_int(inv.x) < 0, sy = __float_as_int(inv.y) < 0, sz = __float_as_int(inv.z) < 0;
+            const float t0x = fmaf((float)(sx ? hx : lx), ax, bx), t1x = fmaf((float)(sx ? lx : hx), ax, bx);
+            const float t0y = fmaf((float)(sy ? hy : ly), ay, by), t1y = fmaf((float)(sy ? ly : hy), ay, by);
+            const float t0z = fmaf((float)(sz ? hz : lz), az, bz), t1z = fmaf((float)(sz ? lz : hz), az, bz);
+            const float tmin = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tnear));
+            const float tmax = fminf(fminf(t1x, t1y), fminf(t1z, best_t));
+            const bool in = gl < nch && tmin <= tmax;
+            // internal children, far to near (any hit: last to first) onto the stack
+            const bool inner = in && gl < ni, leaf = in && gl >= ni;
+            const uint32_t inners = (uint32_t)(__ballot(inner) >> shift) & 0xFFu;
+            const int k = inner ? (__float_as_int(tmin) & ~7) | (int)gl : 0x7FFFFFF8 | (int)gl;
+            const uint32_t rank = ANY ? (uint32_t)__popc(inners & ((1u << gl) - 1u)) : group_rank(k);
+            const uint32_t cnt = (uint32_t)__popc(inners);
+            if (inner) stack[sp + cnt - 1u - rank] = make_uint2(base + 2u * gl, __float_as_uint(tmin));
+            sp += cnt;
+            asm volatile("" ::: "memory");
+            // leaf children's triangles and, with them in flight, the node on top of the stack (65 536 rays:
+            // 194 -> 167 us). Not over instances: the top entry may leave the one whose triangles these
+            // are, and telling that apart costs more than the wait (494 -> 522 us).
+            const uint32_t slot = gl == ni ? (uint32_t)node + 1u : base + ni + gl - 1u;
+            const TriRecord* __restrict rt = reinterpret_cast<const TriRecord*>(rw);
+            TriRecord r;
+            if (leaf) r = rt[slot];
+            uint2 e = make_uint2(kGroupExit, 0);
+            const bool ahead = !INST && sp > 0;
+            if (ahead) {
+                e = stack[--sp];
+                node = (int)e.x;
+                fetch();
+            }
+            float t = 0.0f, U = 0.0f, V = 0.0f, a = 1.0f;
+            uint32_t key = 0xFFFFFFFFu;
+            bool closer = false;
+            if (leaf) {
+                if (STATS) ++cnt_tris;
+                if (tri_hit(r, o, d, tnear, t, U, V, a)) {
+                    key = __float_as_uint(r.a.w);
+                    const bool first = INST ? (cur < best_inst || (cur == best_inst && key < best_key)) : key < best_key;
+                    closer = ANY ? t <= best_t : t < best_t || (t == best_t && first);
+                }
+            }
+            if ((uint32_t)(__ballot(closer) >> shift) & 0xFFu) {
+                if (ANY) {
+                    hit_any = true;
+                    break;
+                }
+                // the smallest (t, key) of the lanes that found a closer hit, and its lane
+                float ct = closer ? t : inf;
+                uint32_t ck = closer ? key : 0xFFFFFFFFu, from = gl;
+#pragma unroll
+                for (uint32_t x = 1; x < 8; x <<= 1) {
+                    const float ot = __shfl_xor(ct, x, 8);
+                    const uint32_t ok = (uint32_t)__shfl_xor((int)ck, x, 8), of = (uint32_t)__shfl_xor((int)from, x, 8);
+                    if (ot < ct || (ot == ct && ok < ck)) {
+                        ct = ot;
+                        ck = ok;
+                        from = of;
+                    }
+                }
+                best_t = ct;
+                best_key = ck;
+                best_tri = (uint32_t)__shfl((int)slot, (int)from, 8);
+                best_inst = cur;
+                best_u = __shfl(U, (int)from, 8);
+                best_v = __shfl(V, (int)from, 8);
+                best_a = __shfl(a, (int)from, 8);
+            }
+            if (ahead && (ANY || __uint_as_float(e.y) <= best_t)) continue;
+            node = -1;
+            while (sp > 0) {
+                e = stack[--sp];
+                if (INST && e.x == kGroupExit) {
+                    load_ray();
+                    set_slopes();
+                    rw = ts.wide;
+                    cur = SGPU_INVALID_ID;
+                    continue;
+                }
+                if (ANY || __uint_as_float(e.y) <= best_t) {
+                    node = (int)e.x;
+                    fetch();
+                    break;
+                }
+            }
+            asm volatile("" ::: "memory");
+        }
+        if (gl == 0) {
+            uint32_t id0 = SGPU_INVALID_ID, id1 = SGPU_INVALID_ID;
+            const WideNode* bw = ts.wide;
+            if (INST && !ANY && best_tri != 0xFFFFFFFFu && best_inst != SGPU_INVALID_ID) {
+                bw = ts.insts[best_inst].wide;
+                if (inst_ids) {
+                    id0 = inst_ids[2 * best_inst];
+                    id1 = inst_ids[2 * best_inst + 1];
+                }
+            }
+            write_result<ANY>(i, hit_any, best_tri, best_t, best_u / best_a, best_v / best_a,
+                              reinterpret_cast<const TriRecord*>(bw), hits, occluded, id0, id1);
+            if (INST && !ANY && comp_out) comp_out[i] = best_tri != 0xFFFFFFFFu ? best_inst : SGPU_INVALID_ID;
+        }
+    }
+    if (STATS) {
+        atomicAdd(&stats[0], cnt_nodes);
+        atomicAdd(&stats[1], cnt_tris);
+    }
+}
+
 // 8-wide traversal of the collapsed tree (WideNode), one ray per lane. In a trip of the wave's loop
 // every lane has at most one 64-byte slot to read: a triangle to test, or else a node to visit.
 // (Letting the lanes with triangles wait until 4, 8 or 16 of a wave have one cost 1-25 %.)
@@ -287,16 +495,24 @@ __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_e
     const uint32_t* __restrict ray_scene, sgpu_rays_soa rays, sgpu_hits_soa hits, uint32_t* __restrict occluded,
     uint32_t n, const uint32_t* __restrict n_ptr, uint2* __restrict spill, uint32_t stack_cap,
     unsigned long long* __restrict stats, uint32_t* __restrict overflow, uint32_t* __restrict work,
-    uint32_t* __restrict comp_out, uint32_t n_top)
+    uint32_t* __restrict comp_out, uint32_t n_top, uint32_t group_max)
 {
-    __shared__ uint2 lds_stack[kWideStackLds][SGPU_TRACE_BLOCK];
-    __shared__ uint4 lds_slots[4 * SGPU_TRACE_BLOCK];  // each lane's fetched slot, 4 KB a wave
+    // each lane's fetched slot (4 KB a wave) and the stacks; or the stacks of 32 groups
+    __shared__ uint4 lds_all[4 * SGPU_TRACE_BLOCK + kWideStackLds * SGPU_TRACE_BLOCK / 2];
+    static_assert(sizeof(uint2) * kGroupStack * (SGPU_TRACE_BLOCK / 8) <= sizeof(lds_all), "the groups' stacks");
+    uint4* const lds_slots = lds_all;
+    uint2(*const lds_stack)[SGPU_TRACE_BLOCK] = reinterpret_cast<uint2(*)[SGPU_TRACE_BLOCK]>(lds_all + 4 * SGPU_TRACE_BLOCK);
     __shared__ uint4 lds_top[TOP ? 4 * kTopNodes : 1];
     const uint32_t lane = threadIdx.x;
     const uint32_t gtid = blockIdx.x * SGPU_TRACE_BLOCK + threadIdx.x;
     const uint32_t stride = gridDim.x * SGPU_TRACE_BLOCK;
     unsigned long long cnt_nodes = 0, cnt_tris = 0;
     if (n_ptr) n = *n_ptr;  // the count written on the device by the kernel that queued the rays
+    if (!TOP && n <= group_max) {
+        trace_groups<ANY, STATS, MULTI, INST>(scene, inst_ids, table, ray_scene, rays, hits, occluded, n, stats, comp_out,
+                                              reinterpret_cast<uint2*>(lds_all));
+        return;
+    }
     if (TOP) {
         for (uint32_t k = threadIdx.x; k < 4 * n_top; k += SGPU_TRACE_BLOCK)
             lds_top[k] = reinterpret_cast<const uint4*>(scene.wide + k / 4)[k % 4];
@@ -575,7 +791,14 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
 {
     if (n == 0) return SGPU_OK;
     const uint32_t cus = (uint32_t)ctx->props.multiProcessorCount;
-    uint32_t blocks = (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK;
+    const bool binary = ctx->trace_tree == 0 && !instanced;
+    const bool multi = table != nullptr;
+    // top nodes in LDS: single-scene launches over geometries
+    const uint32_t n_top = binary || multi || instanced ? 0u : std::min(n_wide, std::min(ctx->trace_lds_nodes, kTopNodes));
+    // launches of few rays go eight lanes a ray, where the trees' depth lets their stacks be in LDS
+    const uint32_t group_max = binary || n_top || group_stack(stack_words) > kGroupStack ? 0u : any_hit ? kGroupRays<true> : kGroupRays<false>;
+    const uint32_t lanes = n <= group_max ? 8u : 1u;
+    uint32_t blocks = (uint32_t)(((uint64_t)n * lanes + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK);
     uint32_t max_blocks = cus * std::min(ctx->trace_blocks_per_cu, kMaxTraceBlocksPerCu);
     if (cap_blocks && max_blocks > cap_blocks) max_blocks = cap_blocks;
     if (blocks > max_blocks) blocks = max_blocks;
@@ -585,10 +808,9 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
     // kTraceWorkWords words are the launch's ray counters. A launch whose rays the grid holds at once
     // and whose stacks fit LDS touches neither (a stream-ordered free makes the host wait for the
     // kernel: 150 us of a small query).
-    const bool binary = ctx->trace_tree == 0 && !instanced;
     const bool counts = !binary && blocks < (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK;
     uint32_t* buf = spill_buf;
-    if (!buf && (counts || stack_words > SGPU_STACK_LDS))
+    if (!buf && (counts || (n > group_max && stack_words > SGPU_STACK_LDS)))
         SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
                                     sgpu_trace_spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) *
                                         sizeof(uint32_t),
@@ -598,7 +820,6 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
     sgpu_hits_soa h = {};
     if (hits) h = *hits;
     unsigned long long* st = (unsigned long long*)d_stats;
-    const bool multi = table != nullptr;
     const dim3 g(blocks), b(SGPU_TRACE_BLOCK);
     if (binary) {
 #define SGPU_LAUNCH_2(A, S, M)                                                                                      \
@@ -614,12 +835,10 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
         }
 #undef SGPU_LAUNCH_2
     } else {
-        // top nodes in LDS: single-scene launches over geometries
-        const uint32_t n_top = multi || instanced ? 0u : std::min(n_wide, std::min(ctx->trace_lds_nodes, kTopNodes));
         if (counts) sgpu_trace_work_zero(work, stream);
 #define SGPU_LAUNCH_8(A, S, M, I, T)                                                                               \
     hipLaunchKernelGGL((k_trace8<A, S, M, I, T>), g, b, 0, stream, scene, inst_ids, table, ray_scene, *rays, h,    \
-                       occluded, n, n_ptr, (uint2*)spill, std::max(stack_words / 2, kWideStackLds), st, overflow, work, comp_out, n_top)
+                       occluded, n, n_ptr, (uint2*)spill, std::max(stack_words / 2, kWideStackLds), st, overflow, work, comp_out, n_top, group_max)
 #define SGPU_LAUNCH_8S(A, S)                                                                                      \
     do {                                                                                                          \
         if (multi && instanced) SGPU_LAUNCH_8(A, S, true, true, false);                                           \

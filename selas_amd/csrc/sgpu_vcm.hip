@@ -1299,7 +1299,7 @@ void server_sync_scenes(sgpu_vcm_server sv)
             uids.push_back(j.scene->uid);
             inst |= !j.scene->instances.empty();
             curves |= j.scene->n_curves > 0;
-            stack = std::max(stack, j.scene->stack_cap);
+            stack = std::max(stack, sv->ctx->trace_tree == 1 ? j.scene->wide_stack : j.scene->stack_cap);
         }
         j.base.scene = k;
     }
