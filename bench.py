@@ -11,7 +11,7 @@ stream time the kernels. The roofline object describes the vertex-merging kernel
 largest kernel of the render): its algorithmic bytes are counted over an untimed run of the same
 job (camera vertices read, range searches, photons visited, photons within the radius; see
 merge_bytes); roofline_closest_hit does the same for the closest-hit traversal (48 B of ray/hit
-traffic + nodes visited x node bytes + triangles tested x 48 B per ray). cpu_baseline renders the
+traffic + nodes visited x 64 B + triangles tested x 64 B per ray: what a visit and a test read). cpu_baseline renders the
 same job with the oracle on the host's cores and compares the images pixel by pixel.
 
 The default run adds two legs to the same line (skip them with --no-batch / --no-serve):
@@ -130,6 +130,11 @@ def cpu_baseline_vcm(sc, width, iterations, threads, seed=1):
 # The VCM workload's job: 512 x 512, 32 iterations (one step of the vcm workload).
 C3_ITERATIONS = 32
 
+# Bytes a node visit and a triangle test read, on both trees (an 8-wide node's second 64 B are its first
+# triangle's record, read when that is tested).
+NODE_READ = 64
+TRI_READ = 64
+
 # Algorithmic bytes of the vertex-merging kernel (k_cam_merge): per camera vertex read 80 B (its
 # CamVertex record); per range search 4 B (its path's slice) + 8 cells x 8 B (two cell ends) + 16 B
 # (the contribution slot and its flag); per photon visited 16 B (its position); per photon within
@@ -169,12 +174,11 @@ def bench_vcm(args):
     # work counters of the same job (untimed): traversal of every closest-hit ray and the vertex
     # merging's range searches, on the tree in use
     _, cnt = job(N.VCM_COUNT_TRAVERSAL | N.VCM_COUNT_MERGE, stats=True)
-    node_bytes = 128 if ctx.tuning()["trace_tree"] == 1 else 64
     nodes_per_ray = cnt["nodes_visited"] / cnt["closest_rays"]
     tris_per_ray = cnt["tris_tested"] / cnt["closest_rays"]
-    bytes_per_ray = 48 + nodes_per_ray * node_bytes + tris_per_ray * 48
+    bytes_per_ray = 48 + nodes_per_ray * NODE_READ + tris_per_ray * TRI_READ
     m_bytes_job = merge_bytes(cnt)
-    log(f"closest hit in VCM: {nodes_per_ray:.2f} nodes/ray ({node_bytes} B), {tris_per_ray:.2f} tris/ray, "
+    log(f"closest hit in VCM: {nodes_per_ray:.2f} nodes/ray ({NODE_READ} B), {tris_per_ray:.2f} tris/ray, "
         f"{bytes_per_ray:.1f} B/ray")
     log(f"merging: {cnt['merge_entries']} camera vertices, {cnt['merge_queries']} range searches, "
         f"{cnt['merge_visited']} photons visited, {cnt['merge_near']} within the radius, "
@@ -308,8 +312,8 @@ def bench_vcm(args):
             "frac": round(achieved_closest / HBM_PEAK_GBS, 4),
             "traffic": load_traffic("traffic_bvh_intersect_vcm_1Mtri.json"),
             "kernel": ("k_trace8 (closest hit, 8-wide nodes, all launches of the timed jobs)"
-                       if node_bytes == 128 else "k_trace<false,false,false> (closest hit, all launches)"),
-            "node_bytes": node_bytes,
+                       if ctx.tuning()["trace_tree"] == 1 else "k_trace<false,false,false> (closest hit, all launches)"),
+            "node_bytes": NODE_READ,
             "launches": st["closest_launches"],
             "avg_launch_ms": round(closest_ms / max(1, st["closest_launches"]), 4),
             "bytes_per_ray": round(bytes_per_ray, 1),
@@ -776,10 +780,9 @@ def bench_pt(args):
         return N.render_pt(scene, cam, w, w, spp, L, seed, flags=flags, return_stats=stats, framebuffer=fb)
 
     _, cnt = image(N.PT_COUNT_TRAVERSAL)
-    node_bytes = 128 if ctx.tuning()["trace_tree"] == 1 else 64
     nodes_per_ray = cnt["nodes_visited"] / cnt["closest_rays"]
     tris_per_ray = cnt["tris_tested"] / cnt["closest_rays"]
-    bytes_per_ray = 48 + nodes_per_ray * node_bytes + tris_per_ray * 48
+    bytes_per_ray = 48 + nodes_per_ray * NODE_READ + tris_per_ray * TRI_READ
     cont = cnt["closest_rays"] - w * w * spp
     shade_bytes = (cnt["closest_rays"] * PT_B_RAY + cnt["hits"] * PT_B_HIT + cnt["shadow_rays"] * PT_B_SHADOW +
                    cont * PT_B_CONT + (cnt["closest_rays"] - cnt["hits"]) * PT_B_MISS)
@@ -899,7 +902,7 @@ def bench_traversal(args):
     stats = scene.intersect_stats(dr)
     nodes_per_ray = stats["nodes_visited"] / n
     tris_per_ray = stats["tris_tested"] / n
-    bytes_per_ray = 48 + nodes_per_ray * stats["bytes_node"] + tris_per_ray * stats["bytes_tri"]
+    bytes_per_ray = 48 + nodes_per_ray * NODE_READ + tris_per_ray * TRI_READ
     log(f"closest hit: {nodes_per_ray:.2f} nodes/ray, {tris_per_ray:.2f} tris/ray, {bytes_per_ray:.1f} B/ray")
 
     for _ in range(args.warmup):
@@ -950,8 +953,8 @@ def bench_traversal(args):
             "triangles": int(t9.shape[0]),
             "rays": n,
             "passes": "closest hit + any hit",
-            "bvh": ("device LBVH collapsed to 8-wide compressed nodes (128 B), triangles as children (48 B)"
-                    if wide else "device LBVH, binary nodes (64 B), 1 triangle per leaf (48 B)"),
+            "bvh": ("device LBVH collapsed to 8-wide compressed nodes (64 B and a first triangle), triangles as children (64 B)"
+                    if wide else "device LBVH, binary nodes (64 B), 1 triangle per leaf (64 B)"),
         },
         "closest_hit_mrays_s": round(n / (avg_isect / 1e3) / 1e6, 2),
         "any_hit_mrays_s": round(n / (avg_occ / 1e3) / 1e6, 2),
@@ -965,7 +968,7 @@ def bench_traversal(args):
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": load_traffic(),
-            "kernel": "k_trace8<false,false,false> (closest hit)" if wide else "k_trace<false,false,false> (closest hit)",
+            "kernel": "k_trace8<false,false,false,false,false> (closest hit)" if wide else "k_trace<false,false,false> (closest hit)",
             "bytes_per_ray": round(bytes_per_ray, 1),
             "nodes_per_ray": round(nodes_per_ray, 3),
             "tris_per_ray": round(tris_per_ray, 3),
@@ -1168,7 +1171,7 @@ def bench_instances(args):
         log(f"{name}: {res[name]}")
         occ.free()
     r = res["instanced"]
-    bytes_per_ray = 48 + r["nodes_per_ray"] * 128 + r["tris_per_ray"] * 48
+    bytes_per_ray = 48 + r["nodes_per_ray"] * NODE_READ + r["tris_per_ray"] * TRI_READ
     ms_i = 1e3 * n / (r["closest_hit_mrays_s"] * 1e6)
     achieved = n * bytes_per_ray / (ms_i / 1e3) / 1e9
     out = {
