@@ -101,8 +101,9 @@ const char* sgpu_last_error(void);
  * A context keeps device memory between calls: the stream-ordered pool of its device holds freed
  * memory for reuse, the VCM wavefront buffers of the last sgpu_render_vcm(_batch) call stay
  * allocated until a call needs larger ones or the context is destroyed, and up to 2 GiB of idle
- * scratch blocks of commits and path-traced renders stay until the context is destroyed (or
- * sgpu_malloc needs the memory). */
+ * scratch blocks of commits and path-traced renders stay until the context is destroyed or an
+ * allocation of any context on the device finds no memory left (which also takes back what the pool
+ * holds freed). */
 int sgpu_context_create(int device, sgpu_context* out);
 int sgpu_context_destroy(sgpu_context ctx);
 

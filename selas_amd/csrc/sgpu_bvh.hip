@@ -771,7 +771,7 @@ int build_wide(sgpu_scratch& S, const BvhNode* nodes, uint32_t n, hipStream_t st
     SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     if (*(const uint32_t*)S.pinned()) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
-    SGPU_HIP_TRY(hipMalloc((void**)&tree.wide, slot_base * kSlotBytes));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&tree.wide, slot_base * kSlotBytes));
     tree.n_slots = (uint32_t)slot_base;
     tree.n_wide = level_base;
     tree.depth = depth;
@@ -843,7 +843,7 @@ int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4*
 {
     const uint32_t n_int = n > 1 ? n - 1 : 1;
     BvhNode* nodes = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&nodes, (size_t)n_int * sizeof(BvhNode)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&nodes, (size_t)n_int * sizeof(BvhNode)));
     auto fail_free = [&](int code, const std::string& msg) {
         (void)hipFree(nodes);
         return sgpu_fail(code, msg);
@@ -1141,7 +1141,7 @@ int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::
     scene->d_cwide = tree.wide;
     scene->n_cslots = tree.n_slots;
     if (rc != SGPU_OK) return rc;
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_cids, (size_t)tree.n_slots * sizeof(uint4)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_cids, (size_t)tree.n_slots * sizeof(uint4)));
     hipLaunchKernelGGL(k_curve_ids, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order2.p, d_leaf_slot.p, d_place.p, n,
                        scene->d_cids);
     SGPU_HIP_TRY(hipGetLastError());
@@ -1381,8 +1381,8 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
         if (extra.empty()) return SGPU_OK;
         // only curves: no top tree; the composed instances' records for the curve pass and shading
         push_extra_shading();
-        hipError_t e = hipMalloc((void**)&scene->d_inst, xrec.size() * sizeof(InstRecord));
-        if (e == hipSuccess) e = hipMalloc((void**)&scene->d_inst_ids, xids.size() * sizeof(uint32_t));
+        hipError_t e = sgpu_device_malloc((void**)&scene->d_inst, xrec.size() * sizeof(InstRecord));
+        if (e == hipSuccess) e = sgpu_device_malloc((void**)&scene->d_inst_ids, xids.size() * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMemcpy(scene->d_inst, xrec.data(), xrec.size() * sizeof(InstRecord), hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(scene->d_inst_ids, xids.data(), xids.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -1515,8 +1515,8 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     if (rc != SGPU_OK) return rc;
     InstRecord* d_inst = nullptr;
     uint32_t* d_ids = nullptr;
-    hipError_t e = hipMalloc((void**)&d_inst, rec.size() * sizeof(InstRecord));
-    if (e == hipSuccess) e = hipMalloc((void**)&d_ids, ids.size() * sizeof(uint32_t));
+    hipError_t e = sgpu_device_malloc((void**)&d_inst, rec.size() * sizeof(InstRecord));
+    if (e == hipSuccess) e = sgpu_device_malloc((void**)&d_ids, ids.size() * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemcpy(d_inst, rec.data(), rec.size() * sizeof(InstRecord), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_ids, ids.data(), ids.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (e != hipSuccess) {

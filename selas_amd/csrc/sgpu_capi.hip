@@ -42,6 +42,45 @@ int sgpu_fail(int code, const std::string& msg)
     return code;
 }
 
+namespace {
+// The contexts there are, so that an allocation that finds the device full can have what they hold idle.
+std::mutex g_contexts_mu;
+std::vector<sgpu_context> g_contexts;
+
+// Gives the current device's memory that nobody uses back: the contexts' idle scratch blocks and what
+// its stream-ordered pool holds freed.
+void give_idle_memory_back()
+{
+    (void)hipGetLastError();
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return;
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        for (sgpu_context c : g_contexts)
+            if (c->device == device) sgpu_scratch_trim(c);
+    }
+    hipMemPool_t pool = nullptr;
+    if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess && pool) (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+}
+}  // namespace
+
+hipError_t sgpu_device_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    give_idle_memory_back();
+    return hipMalloc(p, bytes);
+}
+
+hipError_t sgpu_device_malloc_async(void** p, size_t bytes, hipStream_t stream)
+{
+    hipError_t e = hipMallocAsync(p, bytes, stream);
+    if (e != hipErrorOutOfMemory) return e;
+    give_idle_memory_back();
+    return hipMallocAsync(p, bytes, stream);
+}
+
 hipError_t sgpu_scratch_take(sgpu_context ctx, size_t bytes, ScratchBlock& out)
 {
     {
@@ -61,9 +100,8 @@ hipError_t sgpu_scratch_take(sgpu_context ctx, size_t bytes, ScratchBlock& out)
     hipError_t e = hipMalloc((void**)&out.dev, out.bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        sgpu_scratch_trim(ctx);
         out.bytes = bytes;
-        e = hipMalloc((void**)&out.dev, out.bytes);
+        e = sgpu_device_malloc((void**)&out.dev, out.bytes);
     }
     if (e != hipSuccess) return e;
     e = hipHostMalloc((void**)&out.pinned, kScratchPinned * sizeof(uint64_t), hipHostMallocDefault);
@@ -149,6 +187,13 @@ int sgpu_context_create(int device, sgpu_context* out)
         delete ctx;
         return rc;
     }
+    try {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        g_contexts.push_back(ctx);
+    } catch (const std::bad_alloc&) {
+        delete ctx;
+        return sgpu_fail(SGPU_E_NOMEM, "sgpu_context_create: out of host memory");
+    }
     *out = ctx;
     return SGPU_OK;
 }
@@ -156,6 +201,10 @@ int sgpu_context_create(int device, sgpu_context* out)
 int sgpu_context_destroy(sgpu_context ctx)
 {
     if (!ctx) return SGPU_OK;
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        g_contexts.erase(std::remove(g_contexts.begin(), g_contexts.end(), ctx), g_contexts.end());
+    }
     sgpu_vcm_release_cached(ctx);
     sgpu_scratch_trim(ctx);
     delete ctx;
@@ -222,12 +271,7 @@ int sgpu_malloc(sgpu_context ctx, size_t bytes, void** dptr)
     if (!ctx || !dptr) return sgpu_fail(SGPU_E_INVALID, "sgpu_malloc: NULL argument");
     *dptr = nullptr;
     if (bytes == 0) bytes = 1;
-    hipError_t e = hipMalloc(dptr, bytes);
-    if (e == hipErrorOutOfMemory) {  // the context's idle scratch goes first
-        (void)hipGetLastError();
-        sgpu_scratch_trim(ctx);
-        e = hipMalloc(dptr, bytes);
-    }
+    const hipError_t e = sgpu_device_malloc(dptr, bytes);
     if (e != hipSuccess) return sgpu_fail(SGPU_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return SGPU_OK;
 }
@@ -576,7 +620,7 @@ int sgpu_scene_set_vertex_attributes(sgpu_scene scene, uint32_t geom_id, const f
                 for (int r = 0; r < 3; ++r) o[r] = m[0 * 4 + r] * a[0] + m[1 * 4 + r] * a[1] + m[2 * 4 + r] * a[2];
         }
         void* d = nullptr;
-        SGPU_HIP_TRY(hipMalloc(&d, std::max<size_t>(c.size(), 1) * sizeof(float)));
+        SGPU_HIP_TRY(sgpu_device_malloc(&d, std::max<size_t>(c.size(), 1) * sizeof(float)));
         scene->attr_allocs.emplace_back(d, c.size() * sizeof(float));
         SGPU_HIP_TRY(hipMemcpy(d, c.data(), c.size() * sizeof(float), hipMemcpyHostToDevice));
         *out = (const float*)d;
@@ -674,23 +718,23 @@ static int gather_instance_shading(sgpu_scene scene)
         }
     }
     if (any_attr) {
-        SGPU_HIP_TRY(hipMalloc((void**)&scene->d_g_geom_attr, sizeof(sgpu::GeomAttr) * (size_t)n_geoms));
+        SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_g_geom_attr, sizeof(sgpu::GeomAttr) * (size_t)n_geoms));
         SGPU_HIP_TRY(hipMemcpy(scene->d_g_geom_attr, gattr.data(), sizeof(sgpu::GeomAttr) * n_geoms,
                                hipMemcpyHostToDevice));
     }
     std::vector<uint32_t> base(model_of.size());
     for (size_t k = 0; k < base.size(); ++k) base[k] = g0[model_of[k]];
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_g_materials, 22 * sizeof(float) * (size_t)std::max<uint64_t>(n_mats, 1)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_g_materials, 22 * sizeof(float) * (size_t)std::max<uint64_t>(n_mats, 1)));
     for (size_t j = 0; j < models.size(); ++j)
         SGPU_HIP_TRY(hipMemcpy(scene->d_g_materials + 22 * (size_t)m0[j], models[j]->d_materials,
                                22 * sizeof(float) * (size_t)models[j]->n_materials, hipMemcpyDeviceToDevice));
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_g_geom_material, sizeof(uint32_t) * (size_t)std::max<uint64_t>(n_geoms, 1)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_g_geom_material, sizeof(uint32_t) * (size_t)std::max<uint64_t>(n_geoms, 1)));
     SGPU_HIP_TRY(hipMemcpy(scene->d_g_geom_material, gmat.data(), sizeof(uint32_t) * n_geoms, hipMemcpyHostToDevice));
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_g_geom_tex, sizeof(sgpu::PtexTex) * (size_t)std::max<uint64_t>(n_geoms, 1)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_g_geom_tex, sizeof(sgpu::PtexTex) * (size_t)std::max<uint64_t>(n_geoms, 1)));
     SGPU_HIP_TRY(hipMemcpy(scene->d_g_geom_tex, gtex.data(), sizeof(sgpu::PtexTex) * n_geoms, hipMemcpyHostToDevice));
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_inst_geom_base, sizeof(uint32_t) * std::max<size_t>(base.size(), 1)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_inst_geom_base, sizeof(uint32_t) * std::max<size_t>(base.size(), 1)));
     SGPU_HIP_TRY(hipMemcpy(scene->d_inst_geom_base, base.data(), sizeof(uint32_t) * base.size(), hipMemcpyHostToDevice));
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_inst_l2w, sizeof(float) * std::max<size_t>(scene->comp_l2w.size(), 1)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_inst_l2w, sizeof(float) * std::max<size_t>(scene->comp_l2w.size(), 1)));
     SGPU_HIP_TRY(hipMemcpy(scene->d_inst_l2w, scene->comp_l2w.data(), sizeof(float) * scene->comp_l2w.size(),
                            hipMemcpyHostToDevice));
     scene->n_g_geoms = (uint32_t)n_geoms;
@@ -703,7 +747,7 @@ int sgpu_scene_commit(sgpu_scene scene, void* stream)
     std::lock_guard<std::mutex> lock(scene->mu);
     if (scene->committed) return sgpu_fail(SGPU_E_STATE, "sgpu_scene_commit: scene already committed");
     SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_overflow, sizeof(uint32_t)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_overflow, sizeof(uint32_t)));
     SGPU_HIP_TRY(hipMemset(scene->d_overflow, 0, sizeof(uint32_t)));
     if (!scene->instances.empty()) {
         int rc = sgpu_bvh_build_instances(scene, as_stream(stream));
@@ -731,7 +775,7 @@ int sgpu_scene_commit(sgpu_scene scene, void* stream)
     }
     if (any_attr) {
         scene->attr_host.resize(scene->geom_first.size(), sgpu::GeomAttr{nullptr, nullptr, nullptr, 0, 0});
-        SGPU_HIP_TRY(hipMalloc((void**)&scene->d_geom_attr, sizeof(sgpu::GeomAttr) * scene->attr_host.size()));
+        SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_geom_attr, sizeof(sgpu::GeomAttr) * scene->attr_host.size()));
         SGPU_HIP_TRY(hipMemcpy(scene->d_geom_attr, scene->attr_host.data(),
                                sizeof(sgpu::GeomAttr) * scene->attr_host.size(), hipMemcpyHostToDevice));
     }
@@ -825,8 +869,8 @@ int sgpu_scene_set_materials(sgpu_scene scene, const float* materials, uint32_t 
     SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
     float* dm = nullptr;
     uint32_t* dg = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&dm, 22 * sizeof(float) * (size_t)n_materials));
-    hipError_t e = hipMalloc((void**)&dg, sizeof(uint32_t) * (size_t)n_geoms);
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&dm, 22 * sizeof(float) * (size_t)n_materials));
+    hipError_t e = sgpu_device_malloc((void**)&dg, sizeof(uint32_t) * (size_t)n_geoms);
     if (e != hipSuccess) {
         (void)hipFree(dm);
         return sgpu_fail(SGPU_E_NOMEM, "sgpu_scene_set_materials: hipMalloc failed");
@@ -860,7 +904,7 @@ int sgpu_scene_set_lights(sgpu_scene scene, const sgpu_light* lights, uint32_t n
     SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
     void* dl = nullptr;
     if (n_lights > 0) {
-        SGPU_HIP_TRY(hipMalloc(&dl, sizeof(sgpu_light) * (size_t)n_lights));
+        SGPU_HIP_TRY(sgpu_device_malloc(&dl, sizeof(sgpu_light) * (size_t)n_lights));
         hipError_t e = hipMemcpy(dl, lights, sizeof(sgpu_light) * (size_t)n_lights, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             (void)hipFree(dl);
@@ -944,7 +988,7 @@ int sgpu_scene_set_ibl(sgpu_scene scene, uint32_t width, uint32_t height, const 
     std::memcpy(host.data(), rgb, 3 * n * sizeof(float));
     ibl_build_tables(width, height, rgb, host.data() + 3 * n, host.data() + 3 * n + height);
     float* d = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&d, host.size() * sizeof(float)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&d, host.size() * sizeof(float)));
     hipError_t e = hipMemcpy(d, host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(d);
@@ -1000,9 +1044,9 @@ int sgpu_scene_set_ptex(sgpu_scene scene, uint32_t geom_id, uint32_t res_log2, u
     SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
     uint8_t* dt = nullptr;
     int32_t* da = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&dt, texel_bytes));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&dt, texel_bytes));
     scene->tex_allocs.push_back(dt);
-    SGPU_HIP_TRY(hipMalloc((void**)&da, adj.size() * sizeof(int32_t)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&da, adj.size() * sizeof(int32_t)));
     scene->tex_allocs.push_back(da);
     SGPU_HIP_TRY(hipMemcpy(dt, texels, texel_bytes, hipMemcpyHostToDevice));
     SGPU_HIP_TRY(hipMemcpy(da, adj.data(), adj.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -1012,7 +1056,7 @@ int sgpu_scene_set_ptex(sgpu_scene scene, uint32_t geom_id, uint32_t res_log2, u
     if (scene->d_geom_tex) (void)hipFree(scene->d_geom_tex);
     scene->d_geom_tex = nullptr;
     scene->n_geom_tex = 0;
-    SGPU_HIP_TRY(hipMalloc((void**)&scene->d_geom_tex, n_geoms * sizeof(sgpu::PtexTex)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_geom_tex, n_geoms * sizeof(sgpu::PtexTex)));
     SGPU_HIP_TRY(hipMemcpy(scene->d_geom_tex, scene->tex_host.data(), n_geoms * sizeof(sgpu::PtexTex),
                            hipMemcpyHostToDevice));
     scene->n_geom_tex = (uint32_t)n_geoms;
@@ -1313,10 +1357,10 @@ int sgpu_intersect_stats(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu
     if (!stats) return sgpu_fail(SGPU_E_INVALID, "sgpu_intersect_stats: NULL stats");
     uint64_t* d_stats = nullptr;
     uint32_t* d_occ = nullptr;
-    SGPU_HIP_TRY(hipMalloc((void**)&d_stats, 4 * sizeof(uint64_t)));
+    SGPU_HIP_TRY(sgpu_device_malloc((void**)&d_stats, 4 * sizeof(uint64_t)));
     SGPU_HIP_TRY(hipMemset(d_stats, 0, 4 * sizeof(uint64_t)));
     if (any_hit) {
-        hipError_t e = hipMalloc((void**)&d_occ, (size_t)(n ? n : 1) * sizeof(uint32_t));
+        hipError_t e = sgpu_device_malloc((void**)&d_occ, (size_t)(n ? n : 1) * sizeof(uint32_t));
         if (e != hipSuccess) {
             (void)hipFree(d_stats);
             return sgpu_fail(SGPU_E_NOMEM, "sgpu_intersect_stats: hipMalloc failed");

@@ -406,7 +406,7 @@ int sgpu_curve_launch(sgpu_context ctx, const TraceScene& scene, const uint32_t*
     if (max_blocks) blocks = std::min(blocks, max_blocks);  // a lent buffer's
     uint32_t* buf = spill;
     if (!buf && (blocks < needed || stack_words > SGPU_STACK_LDS))
-        SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
+        SGPU_HIP_TRY(sgpu_device_malloc_async((void**)&buf,
                                     sgpu_trace_spill_words(stack_words, (size_t)blocks * kCurveBlock) * sizeof(uint32_t),
                                     stream));
     if (blocks < needed) sgpu_trace_work_zero(buf, stream);

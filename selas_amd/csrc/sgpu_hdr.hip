@@ -75,7 +75,7 @@ int sgpu_framebuffer_save_hdr(const char* path_prefix, const float* framebuffer,
     hipStream_t st = (hipStream_t)stream;
     const size_t n = (size_t)width * height;
     uint32_t* d = nullptr;
-    SGPU_HIP_TRY(hipMallocAsync((void**)&d, n * sizeof(uint32_t), st));
+    SGPU_HIP_TRY(sgpu_device_malloc_async((void**)&d, n * sizeof(uint32_t), st));
     std::vector<uint32_t> px(n);
     std::vector<uint8_t> line, planes(4 * (size_t)width);
     int rc = SGPU_OK;

@@ -291,6 +291,11 @@ struct sgpu_phase_timer {
     }
 };
 
+// Device memory (sgpu_capi.hip). Every allocation but that of a scratch block goes this way: where the
+// device is full, the memory that contexts keep idle and that its pool holds freed is given back first.
+hipError_t sgpu_device_malloc(void** p, size_t bytes);
+hipError_t sgpu_device_malloc_async(void** p, size_t bytes, hipStream_t stream);
+
 // Scratch blocks of a context (sgpu_capi.hip): an idle block of at least `bytes` or a new one; a block
 // back among the idle ones (or freed, past kScratchKeep bytes of them); all idle ones freed.
 hipError_t sgpu_scratch_take(sgpu_context ctx, size_t bytes, ScratchBlock& out);

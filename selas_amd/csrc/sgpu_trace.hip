@@ -959,7 +959,7 @@ int trace_launch(sgpu_context ctx, const TraceScene& scene, uint32_t n_wide, con
     const bool counts = !binary && blocks < (n + SGPU_TRACE_BLOCK - 1) / SGPU_TRACE_BLOCK;
     uint32_t* buf = spill_buf;
     if (!buf && (counts || (n > group_max && stack_words > SGPU_STACK_LDS)))
-        SGPU_HIP_TRY(hipMallocAsync((void**)&buf,
+        SGPU_HIP_TRY(sgpu_device_malloc_async((void**)&buf,
                                     sgpu_trace_spill_words(stack_words, (size_t)blocks * SGPU_TRACE_BLOCK) *
                                         sizeof(uint32_t),
                                     stream));

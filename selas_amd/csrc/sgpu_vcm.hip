@@ -988,7 +988,7 @@ struct Arena {
         bytes += n;
         if (dry) return reinterpret_cast<T*>((uintptr_t)256);
         void* p = nullptr;
-        if (err == hipSuccess) err = hipMallocAsync(&p, n, stream);
+        if (err == hipSuccess) err = sgpu_device_malloc_async(&p, n, stream);
         if (err == hipSuccess) ptrs.push_back(p);
         return (T*)p;
     }
@@ -1333,7 +1333,7 @@ int server_upload_table(sgpu_vcm_server sv, hipStream_t stream)
         sv->d_table = nullptr;
         sv->h_table = nullptr;
         sv->table_cap = std::max<uint32_t>(16, 2 * n);
-        SGPU_HIP_TRY(hipMalloc((void**)&sv->d_table, sizeof(TraceScene) * sv->table_cap));
+        SGPU_HIP_TRY(sgpu_device_malloc((void**)&sv->d_table, sizeof(TraceScene) * sv->table_cap));
         SGPU_HIP_TRY(hipHostMalloc((void**)&sv->h_table, sizeof(TraceScene) * sv->table_cap, hipHostMallocDefault));
     }
     for (uint32_t k = 0; k < n; ++k)
@@ -1431,7 +1431,7 @@ int sgpu_vcm_server_submit_impl(sgpu_vcm_server sv, sgpu_scene sc, const sgpu_vc
     if (sc->stack_cap > sv->spill_cap) {
         // a deeper tree than the spill buffer holds stacks for: a larger one, stream-ordered
         uint32_t* grown = nullptr;
-        SGPU_HIP_TRY(hipMallocAsync((void**)&grown, sgpu_trace_spill_words(sv->ctx, sc->stack_cap) * sizeof(uint32_t),
+        SGPU_HIP_TRY(sgpu_device_malloc_async((void**)&grown, sgpu_trace_spill_words(sv->ctx, sc->stack_cap) * sizeof(uint32_t),
                                     stream));
         if (sv->spill_grown) SGPU_HIP_TRY(hipFreeAsync(sv->spill_grown, stream));
         sv->spill_grown = grown;
@@ -1442,7 +1442,7 @@ int sgpu_vcm_server_submit_impl(sgpu_vcm_server sv, sgpu_scene sc, const sgpu_vc
         // the tangent arrays: 2 x (paths x vertex slots) for light vertices, paths for camera vertices
         const size_t nv = (size_t)sv->TM * sv->mlv;
         float4* t = nullptr;
-        SGPU_HIP_TRY(hipMallocAsync((void**)&t, (2 * nv + sv->TM) * sizeof(float4), stream));
+        SGPU_HIP_TRY(sgpu_device_malloc_async((void**)&t, (2 * nv + sv->TM) * sizeof(float4), stream));
         sv->vtan = t;
         sv->cvtan = t + nv;
         sv->cam_tan = t + 2 * nv;
