@@ -741,16 +741,39 @@ static int gather_instance_shading(sgpu_scene scene)
     return SGPU_OK;
 }
 
-int sgpu_scene_commit(sgpu_scene scene, void* stream)
+// What a commit puts on the device, freed: at the scene's release, and where a commit failed (it may be
+// tried again).
+static void drop_committed(sgpu_scene scene)
 {
-    if (!scene) return sgpu_fail(SGPU_E_INVALID, "sgpu_scene_commit: NULL scene");
-    std::lock_guard<std::mutex> lock(scene->mu);
-    if (scene->committed) return sgpu_fail(SGPU_E_STATE, "sgpu_scene_commit: scene already committed");
-    SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
+    auto drop = [](auto*& p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    };
+    drop(scene->d_inst);
+    drop(scene->d_inst_ids);
+    drop(scene->d_g_materials);
+    drop(scene->d_g_geom_material);
+    drop(scene->d_g_geom_tex);
+    drop(scene->d_g_geom_attr);
+    drop(scene->d_geom_attr);
+    drop(scene->d_inst_geom_base);
+    drop(scene->d_inst_l2w);
+    drop(scene->d_nodes);
+    drop(scene->d_wide);
+    drop(scene->d_cnodes);
+    drop(scene->d_cwide);
+    drop(scene->d_cids);
+    drop(scene->d_overflow);
+    scene->n_curves = 0;
+    scene->n_inst = 0;
+}
+
+static int commit_scene(sgpu_scene scene, hipStream_t stream)
+{
     SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_overflow, sizeof(uint32_t)));
     SGPU_HIP_TRY(hipMemset(scene->d_overflow, 0, sizeof(uint32_t)));
     if (!scene->instances.empty()) {
-        int rc = sgpu_bvh_build_instances(scene, as_stream(stream));
+        int rc = sgpu_bvh_build_instances(scene, stream);
         if (rc == SGPU_OK) rc = gather_instance_shading(scene);
         if (rc != SGPU_OK) return rc;
         if (scene->n_inst > 0 || scene->n_curves > 0) {
@@ -762,10 +785,10 @@ int sgpu_scene_commit(sgpu_scene scene, void* stream)
         scene->committed = true;
         return SGPU_OK;
     }
-    int rc = sgpu_bvh_build(scene, as_stream(stream));
+    int rc = sgpu_bvh_build(scene, stream);
     if (rc == SGPU_OK && !scene->curve_geom.empty())
         rc = sgpu_curve_build(scene, scene->curve_cp, scene->curve_geom, scene->curve_prim,
-                              std::vector<uint32_t>(scene->curve_geom.size(), SGPU_INVALID_ID), as_stream(stream));
+                              std::vector<uint32_t>(scene->curve_geom.size(), SGPU_INVALID_ID), stream);
     if (rc != SGPU_OK) return rc;
     // the attribute table (one record per geometry) when any geometry has attributes
     bool any_attr = false;
@@ -810,6 +833,17 @@ int sgpu_scene_commit(sgpu_scene scene, void* stream)
     return SGPU_OK;
 }
 
+int sgpu_scene_commit(sgpu_scene scene, void* stream)
+{
+    if (!scene) return sgpu_fail(SGPU_E_INVALID, "sgpu_scene_commit: NULL scene");
+    std::lock_guard<std::mutex> lock(scene->mu);
+    if (scene->committed) return sgpu_fail(SGPU_E_STATE, "sgpu_scene_commit: scene already committed");
+    SGPU_HIP_TRY(hipSetDevice(scene->ctx->device));
+    const int rc = commit_scene(scene, as_stream(stream));
+    if (rc != SGPU_OK) drop_committed(scene);
+    return rc;
+}
+
 int sgpu_scene_release(sgpu_scene scene)
 {
     if (!scene) return SGPU_OK;
@@ -824,22 +858,8 @@ int sgpu_scene_release(sgpu_scene scene)
         std::lock_guard<std::mutex> lock(in.child->mu);
         --in.child->refs;
     }
-    if (scene->d_inst) (void)hipFree(scene->d_inst);
-    if (scene->d_inst_ids) (void)hipFree(scene->d_inst_ids);
-    if (scene->d_g_materials) (void)hipFree(scene->d_g_materials);
-    if (scene->d_g_geom_material) (void)hipFree(scene->d_g_geom_material);
-    if (scene->d_g_geom_tex) (void)hipFree(scene->d_g_geom_tex);
-    if (scene->d_g_geom_attr) (void)hipFree(scene->d_g_geom_attr);
-    if (scene->d_geom_attr) (void)hipFree(scene->d_geom_attr);
+    drop_committed(scene);
     for (const auto& a : scene->attr_allocs) (void)hipFree(a.first);
-    if (scene->d_inst_geom_base) (void)hipFree(scene->d_inst_geom_base);
-    if (scene->d_inst_l2w) (void)hipFree(scene->d_inst_l2w);
-    if (scene->d_nodes) (void)hipFree(scene->d_nodes);
-    if (scene->d_wide) (void)hipFree(scene->d_wide);
-    if (scene->d_cnodes) (void)hipFree(scene->d_cnodes);
-    if (scene->d_cwide) (void)hipFree(scene->d_cwide);
-    if (scene->d_cids) (void)hipFree(scene->d_cids);
-    if (scene->d_overflow) (void)hipFree(scene->d_overflow);
     if (scene->d_materials) (void)hipFree(scene->d_materials);
     if (scene->d_geom_material) (void)hipFree(scene->d_geom_material);
     if (scene->d_lights) (void)hipFree(scene->d_lights);

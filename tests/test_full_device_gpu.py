@@ -39,6 +39,13 @@ def test_call_takes_idle_memory(limit_lib, call):
     _child(limit_lib, call)
 
 
+@pytest.mark.parametrize("kind", ["triangles", "curves", "instances"])
+def test_refused_commit_leaves_nothing(limit_lib, kind):
+    """Whichever of a commit's allocations is refused: an error, nothing left allocated, and the same
+    scene commits once there is memory."""
+    _child(limit_lib, "refused " + kind)
+
+
 # ---- the child ---------------------------------------------------------------------------------------
 
 def _main(so, call):
@@ -66,8 +73,8 @@ def _main(so, call):
         return s
 
     def hits(s):
-        dr, dh = N.DeviceRays(ctx, cam), N.DeviceHits(ctx, cam["org_x"].size)
         lim_off()
+        dr, dh = N.DeviceRays(ctx, cam), N.DeviceHits(ctx, cam["org_x"].size)
         s.intersect(dr, dh)
         N.synchronize()
         return dh.to_host()
@@ -86,6 +93,46 @@ def _main(so, call):
     scene(ctx, 3200000).release()  # 1.8 GB more that stay idle
     job = {"camera": sc["camera"], "width": 32, "height": 32, "iterations": 1, "max_path_length": 5, "base_radius": 0.05,
            "radius_alpha": 0.75, "seed": 3}
+
+    if call.startswith("refused"):
+        def make():
+            s = N.Scene(ctx)
+            if call == "refused instances":
+                for k in range(500):
+                    m = np.eye(4)
+                    m[:3, 3] = (k % 13, k // 13, 0)
+                    s.add_instance(bare if k % 250 else with_curves, m)
+                return s
+            s.release()
+            return scene(ctx, 3200, curves=call == "refused curves", commit=False)
+
+        want_scene = make()
+        want_scene.commit()
+        want = hits(want_scene)
+        s = make()
+
+        def held():  # with the idle blocks given back
+            lim.alloc_limit_set(1)
+            with pytest.raises(N.SgpuError):
+                ctx.empty(1 << 20)
+            return lim.alloc_limit_used()
+
+        before, refusals = held(), 0
+        for slack in range(0, 1 << 24, 24 << 10):
+            lim.alloc_limit_set(before + slack)
+            try:
+                s.commit()
+                break
+            except N.SgpuError as e:
+                assert e.code in (N.SGPU_E_NOMEM, N.SGPU_E_HIP), str(e)
+            refusals += 1
+            assert held() == before, (slack, before, lim.alloc_limit_used())
+        assert refusals > 20
+        got = hits(s)
+        for k in want:
+            assert np.array_equal(got[k].view(np.uint32), want[k].view(np.uint32)), k
+        print(f"{call}: ok after {refusals} refusals", flush=True)
+        return
 
     def vcm():
         N.render_vcm(room, sc["camera"], 32, 32, 1, 5, 0.05, 0.75, 3, framebuffer=frame)
