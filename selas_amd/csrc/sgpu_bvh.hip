@@ -771,7 +771,8 @@ int build_wide(sgpu_scratch& S, const BvhNode* nodes, uint32_t n, hipStream_t st
     SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
     if (*(const uint32_t*)S.pinned()) return sgpu_fail(SGPU_E_RANGE, "wide node quantization could not contain a child box");
-    SGPU_HIP_TRY(sgpu_device_malloc((void**)&tree.wide, slot_base * kSlotBytes));
+    if (sgpu_device_malloc((void**)&tree.wide, slot_base * kSlotBytes) != hipSuccess)
+        return sgpu_fail(SGPU_E_NOMEM, "hipMalloc of triangle records and 8-wide nodes failed");
     tree.n_slots = (uint32_t)slot_base;
     tree.n_wide = level_base;
     tree.depth = depth;

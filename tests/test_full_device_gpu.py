@@ -117,7 +117,7 @@ def _main(so, call):
                 ctx.empty(1 << 20)
             return lim.alloc_limit_used()
 
-        before, refusals = held(), 0
+        before, refusals, codes = held(), 0, set()
         for slack in range(0, 1 << 24, 24 << 10):
             lim.alloc_limit_set(before + slack)
             try:
@@ -125,9 +125,11 @@ def _main(so, call):
                 break
             except N.SgpuError as e:
                 assert e.code in (N.SGPU_E_NOMEM, N.SGPU_E_HIP), str(e)
+                codes.add(e.code)
             refusals += 1
             assert held() == before, (slack, before, lim.alloc_limit_used())
         assert refusals > 20
+        assert N.SGPU_E_NOMEM in codes  # the records' allocation says what it was
         got = hits(s)
         for k in want:
             assert np.array_equal(got[k].view(np.uint32), want[k].view(np.uint32)), k
