@@ -65,20 +65,28 @@ void give_idle_memory_back()
 }
 }  // namespace
 
+// (A refusal is in what these return, and not left as the thread's last error, which the next launch's
+// check would take for its own.)
 hipError_t sgpu_device_malloc(void** p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipErrorOutOfMemory) return e;
-    give_idle_memory_back();
-    return hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        give_idle_memory_back();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 hipError_t sgpu_device_malloc_async(void** p, size_t bytes, hipStream_t stream)
 {
     hipError_t e = hipMallocAsync(p, bytes, stream);
-    if (e != hipErrorOutOfMemory) return e;
-    give_idle_memory_back();
-    return hipMallocAsync(p, bytes, stream);
+    if (e == hipErrorOutOfMemory) {
+        give_idle_memory_back();
+        e = hipMallocAsync(p, bytes, stream);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 hipError_t sgpu_scratch_take(sgpu_context ctx, size_t bytes, ScratchBlock& out)

@@ -1,7 +1,8 @@
 /* The HIP allocation calls with a limit on what they hand out, for a test process: loaded with
  * RTLD_GLOBAL before libselas_gpu, so that the library's calls come here first. Nothing is really
  * exhausted: a request past alloc_limit_set's bytes gets hipErrorOutOfMemory, every other goes on to the
- * runtime. Memory freed to the stream-ordered pool counts until the pool is trimmed. */
+ * runtime. A refusal stays the thread's last error until it is asked for, as the runtime's do. Memory
+ * freed to the stream-ordered pool counts until the pool is trimmed. */
 #define _GNU_SOURCE
 #include <dlfcn.h>
 #include <pthread.h>
@@ -15,6 +16,7 @@ static struct {
     size_t n;
 } block[kMax];
 static size_t count, plain, pooled, pool_size, limit = (size_t)-1, refused;
+static __thread int last;
 
 static void* real(const char* name)
 {
@@ -51,7 +53,7 @@ int hipMalloc(void** p, size_t n)
     pthread_mutex_lock(&mu);
     int e = kOutOfMemory;
     if (plain + pool_size + n > limit)
-        ++refused;
+        ++refused, last = e;
     else if ((e = f(p, n)) == 0) {
         note(*p, n);
         plain += n;
@@ -76,7 +78,7 @@ int hipMallocAsync(void** p, size_t n, void* stream)
     const size_t size = pooled + n > pool_size ? pooled + n : pool_size;
     int e = kOutOfMemory;
     if (plain + size > limit)
-        ++refused;
+        ++refused, last = e;
     else if ((e = f(p, n, stream)) == 0) {
         note(*p, n);
         pooled += n;
@@ -102,4 +104,12 @@ int hipMemPoolTrimTo(void* pool, size_t keep)
     pool_size = pooled > keep ? pooled : keep;
     pthread_mutex_unlock(&mu);
     return f(pool, keep);
+}
+
+int hipGetLastError(void)
+{
+    int (*f)(void) = (int (*)(void))real("hipGetLastError");
+    const int e = f(), mine = last;
+    last = 0;
+    return mine ? mine : e;
 }
