@@ -1706,11 +1706,12 @@ int sgpu_vcm_server_step_impl(sgpu_vcm_server sv, hipStream_t stream, uint64_t* 
                 if (merge_sorted) bin_sort(c_in, n, false, nullptr);
                 // sorted: a multiple of the XCD count, so that the blocks can be numbered xcd-major
                 const uint32_t mlanes = sv->ctx->vcm_merge_lanes;
-                const uint32_t per_block = (64 / mlanes) * kMergeWaves;  // queries per block and stride
+                const uint32_t per_block = (64 / mlanes) * kMergeWaves;  // queries a block takes in a round
                 uint32_t merge_blocks = std::min<uint32_t>((n + per_block - 1) / per_block, 16u * cus);
                 if (merge_sorted) merge_blocks = (merge_blocks + kXcds - 1) / kXcds * kXcds;
                 launch_cam_merge(mlanes, merge_blocks, st, wv, merge_sorted ? sv->bins.n : c_in,
-                                 merge_sorted ? sv->bins.order : nullptr, sv->cam_vm, ps.slice, G, S, d_mstat);
+                                 merge_sorted ? sv->bins.order : nullptr, sv->cam_vm, ps.slice, G, S,
+                                 4 * kMergeWavesPerSimd * cus, d_mstat);
                 SGPU_HIP_TRY(hipGetLastError());
                 SGPU_HIP_TRY(T.end());
             }

@@ -27,7 +27,7 @@ struct QueryCells {
 };
 
 // Vertex merging (SearchHashGrid + MergeVertices, VCMHashGrid.cpp:107-157, VCM.cpp:362-409). A wave takes
-// the queries of a bounce kBatch at a time, grid-stride: a lane each prepares its BSDF and constants in
+// the queries of a bounce up to kBatch at a time, grid-stride: a lane each prepares its BSDF and constants in
 // LDS, eight lanes each look up its cells. Then the wave's groups of GW lanes take a query each, round by
 // round: the lanes of a group scan the photons of its cells as one list (the cells' ranges in the
 // reference's visiting order, strided over the lanes) and append those within the radius to the group's
@@ -40,15 +40,20 @@ struct QueryCells {
 // the query's values in every lane's registers and each group evaluating its own photons (168 VGPRs, 3
 // waves per SIMD, passes half empty, a query's preparation run by 4 queries at a time) the 512 x 512 x 32
 // job's merging took 15.3 ms; the values in LDS (5 waves) 11.0, photons of all groups in one pass 10.6,
-// preparation in batches 8.8 (16 lanes a group; 9.0 with 8, 10.7 with 32). Bound by vector instructions. With `order` (the
+// preparation in batches 8.8 (16 lanes a group; 9.0 with 8, 10.7 with 32). Bound by vector instructions.
+// A batch is as many rounds as it takes for the waves that are resident to hold every query: full batches
+// on a part of the chip took longer than the smaller preparation gains (the merges of a 64 x 64 image of
+// one iteration, ten launches: 90 us, 140 with full batches, 83 before the pooling; 128 x 128 x 4 161, 241
+// and 175; 256 x 256 x 8 494, 580 and 762; with 32 lanes a group 87, 170, 79; 181, 325, 221; 652, 845,
+// 1215). With `order` (the
 // queries of the bounce in spatial order) blocks are numbered xcd-major, so that the queries running at
 // once on one XCD are neighbours in space and read the same photon cells through that XCD's L2.
 template <uint32_t GW>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_cam_merge(Wave w, const uint32_t* __restrict count_ptr,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMergeWavesPerSimd))) void k_cam_merge(Wave w, const uint32_t* __restrict count_ptr,
                                                       const uint32_t* __restrict order,
                                                       const CamVertex* __restrict cam_vm,
                                                       const uint32_t* __restrict path_slice, GridView G, CamSlots S,
-                                                      unsigned long long* __restrict mstat)
+                                                      uint32_t resident, unsigned long long* __restrict mstat)
 {
     static_assert(GW == 8 || GW == 16 || GW == 32, "a group divides the wave");
     constexpr uint32_t kQ = 64 / GW;                   // groups of a wave
@@ -65,7 +70,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     const unsigned long long below = (1ull << lane) - 1ull;
     const unsigned long long group_bits = ((1ull << GW) - 1ull) << (grp * GW);
     if (*G.nv_ptr == 0) return;
-    const uint32_t stride = kBatch * gridDim.x * kMergeWaves;
+    const uint32_t waves = min(gridDim.x * kMergeWaves, resident);
+    const uint32_t batch = min(kBatch, kQ * max(1u, (count + kQ * waves - 1) / (kQ * waves)));
+    const uint32_t stride = batch * gridDim.x * kMergeWaves;
     const uint32_t block = order ? xcd_major_block(blockIdx.x, gridDim.x) : blockIdx.x;
     // work counters of this wave, flushed at the end
     __shared__ uint32_t cnt_lds[kMergeWaves][4];
@@ -98,10 +105,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
         return (f * mk3(lv.thr[0], lv.thr[1], lv.thr[2])) * (mis / cos_l);
     };
 
-    for (uint32_t j0 = kBatch * (block * kMergeWaves + wid); j0 < count; j0 += stride) {
+    for (uint32_t j0 = batch * (block * kMergeWaves + wid); j0 < count; j0 += stride) {
         // ---- the batch's queries, a lane each (none past the end, or without a query, or outside the box) ----
         const uint32_t jj = j0 + lane;
-        const bool in_batch = lane < kBatch && jj < count;
+        const bool in_batch = lane < batch && jj < count;
         const uint32_t j = order && in_batch ? order[jj] : jj;
         bool active = false;
         uint32_t si = 0, cell_base = 0, cell_count = 1;
@@ -152,7 +159,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
         }
         const unsigned long long actives = __ballot(active);
         if (mstat && lane == 0) {
-            atomicAdd(&cnt_lds[wid][0], min(kBatch, count - j0));
+            atomicAdd(&cnt_lds[wid][0], min(batch, count - j0));
             atomicAdd(&cnt_lds[wid][1], (uint32_t)__popcll(actives));
         }
         if (actives == 0) continue;
@@ -181,7 +188,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
         }
         __builtin_amdgcn_wave_barrier();
 
-        for (uint32_t round = 0; round < kBatch / kQ; ++round) {
+        for (uint32_t round = 0; round < batch / kQ; ++round) {
             const uint32_t b = round * kQ + grp;  // this group's query
             const QueryCells& cells = cell_lds[wid][b];
             const QueryView& mine = view_lds[wid][b];
@@ -275,17 +282,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
 
 void launch_cam_merge(uint32_t lanes, uint32_t blocks, hipStream_t stream, const Wave& w, const uint32_t* count_ptr,
                       const uint32_t* order, const CamVertex* cam_vm, const uint32_t* path_slice, const GridView& G,
-                      const CamSlots& S, unsigned long long* mstat)
+                      const CamSlots& S, uint32_t resident, unsigned long long* mstat)
 {
     if (lanes == 32)
         hipLaunchKernelGGL(k_cam_merge<32>, dim3(blocks), dim3(kBlock), 0, stream, w, count_ptr, order, cam_vm,
-                           path_slice, G, S, mstat);
+                           path_slice, G, S, resident, mstat);
     else if (lanes == 8)
         hipLaunchKernelGGL(k_cam_merge<8>, dim3(blocks), dim3(kBlock), 0, stream, w, count_ptr, order, cam_vm,
-                           path_slice, G, S, mstat);
+                           path_slice, G, S, resident, mstat);
     else
         hipLaunchKernelGGL(k_cam_merge<16>, dim3(blocks), dim3(kBlock), 0, stream, w, count_ptr, order, cam_vm,
-                           path_slice, G, S, mstat);
+                           path_slice, G, S, resident, mstat);
 }
 
 }  // namespace sgpu_vcm
