@@ -477,6 +477,8 @@ int sgpu_curve_launch(sgpu_context ctx, const TraceScene& scene, const uint32_t*
                       const sgpu_hits_soa* hits, uint32_t* occluded, uint32_t n, bool any_hit, const uint32_t* n_ptr,
                       uint32_t* comp_out, uint32_t* overflow, hipStream_t stream, uint32_t* spill,
                       uint32_t max_blocks = 0, uint64_t* stats = nullptr);
+// Words of stack a lane can need on the scene's 8-wide trees (the tests ask for it).
+uint32_t sgpu_trace_stack_words(sgpu_scene scene);
 // Words of a spill buffer for a traversal grid of `threads` lanes (sgpu_trace.hip).
 size_t sgpu_trace_spill_words(uint32_t stack_words, size_t threads);
 // Builds the curve tree of a scene of geometries from its segments, or of an instanced scene from

@@ -1018,6 +1018,8 @@ size_t sgpu_trace_spill_words(sgpu_context ctx, uint32_t stack_words)
     return sgpu_trace_spill_words(stack_words, (size_t)cus * kMaxTraceBlocksPerCu * SGPU_TRACE_BLOCK);
 }
 
+uint32_t sgpu_trace_stack_words(sgpu_scene scene) { return scene->wide_stack; }
+
 size_t sgpu_trace_spill_words(sgpu_scene scene) { return sgpu_trace_spill_words(scene->ctx, scene->stack_cap); }
 
 int sgpu_trace_launch(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t* occluded,

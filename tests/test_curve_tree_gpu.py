@@ -54,3 +54,42 @@ def test_axis_rays_hit_where_the_oracle_says(gpu_ctx, n_seg, n_rays):
     joint = (np.abs(gp - wp) == 1) & ((got["u"] < 1e-2) | (got["u"] > 1 - 1e-2))
     assert ((gp == wp) | joint).all()
     scene.release()
+
+
+@pytest.mark.parametrize("factor", [1, 5, 20])
+def test_axis_rays_from_afar(gpu_ctx, factor):
+    """The pass culls in single precision with a rounded reciprocal: rays whose origins are `factor` times
+    the scene's largest coordinate away still hit every segment aimed at. (Their own rounding, half an ulp
+    of the origin, is 2e-6 at 50: a five-thousandth of the radius.)"""
+    n_seg, n_rays = 300, 20000
+    verts, idx = _strand(1, n_seg), np.arange(n_seg, dtype=np.uint32)
+    verts[:, :3] *= np.float32(2.5 / np.abs(verts[:, :3]).max())
+    rng = np.random.default_rng(factor)
+    seg, u = rng.integers(0, n_seg, n_rays), rng.random(n_rays)
+    cp = verts[:, :3].astype(np.float64)
+    b = np.stack([(1 - u) ** 3, 3 * u ** 3 - 6 * u ** 2 + 4, -3 * u ** 3 + 3 * u ** 2 + 3 * u + 1, u ** 3], 1) / 6
+    axis = sum(b[:, j:j + 1] * cp[seg + j] for j in range(4))
+    way = rng.normal(size=(n_rays, 3))
+    way /= np.linalg.norm(way, axis=1, keepdims=True)
+    way[::5] = np.eye(3)[rng.integers(0, 3, way[::5].shape[0])] * rng.choice([-1.0, 1.0], (way[::5].shape[0], 1))
+    o, d = (axis - 2.5 * factor * way).astype(np.float32), way.astype(np.float32)
+    rays = {"org_x": o[:, 0], "org_y": o[:, 1], "org_z": o[:, 2], "dir_x": d[:, 0], "dir_y": d[:, 1], "dir_z": d[:, 2],
+            "tnear": np.zeros(n_rays, np.float32), "tfar": np.full(n_rays, np.inf, np.float32)}
+    rays = {k: np.ascontiguousarray(v) for k, v in rays.items()}
+    scene = N.Scene(gpu_ctx)
+    scene.add_curves(verts, idx)
+    scene.commit()
+    dr, dh = N.DeviceRays(gpu_ctx, rays), N.DeviceHits(gpu_ctx, n_rays)
+    scene.intersect(dr, dh)
+    occ = gpu_ctx.empty(4 * n_rays)
+    scene.occluded(dr, occ)
+    N.synchronize()
+    scene.check()
+    got = dh.to_host()
+    scene.release()
+    want = O.curves_closest(O.curve_segments({"curve_vertices": verts, "curves": idx}), dict(rays, tfar=np.full(n_rays, 1e30, np.float32)))
+    hit = want["prim"] != N.INVALID_ID
+    # a ray along the strand may start inside it; and one that grazes an earlier turn of it may go either way
+    assert hit.mean() > 0.999 and np.array_equal(got["geom_id"] == 0, occ.download(np.uint32, n_rays) == 1)
+    close = np.abs(got["t"] - want["t"]) <= 1e-5 * want["t"]
+    assert (hit & ~close).sum() <= 1 + 2e-4 * n_rays, (hit & ~close).sum()

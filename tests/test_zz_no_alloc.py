@@ -1,12 +1,14 @@
 """sgpu_intersect_noalloc (no device allocation: the traversal stacks spill into a fixed per-GPU
 array) against sgpu_intersect through the C ABI: bit-exact t, u, v, primID, geomID, Ng and
 instance ids on two calls in a row, the second with a smaller input, on a flat scene deep enough
-for the stacks to spill past their LDS part and on a two-level instanced scene; plus its argument
-errors. Collected last (its file name), so that it also runs after every other GPU test.
+for the stacks to spill past their LDS part, with more rays than go eight lanes each (which need no
+spill), and on a two-level instanced scene; plus its argument errors. (test_deep_trees_gpu.py holds it
+against the oracle.) Collected last (its file name), so that it also runs after every other GPU test.
 """
 import numpy as np
 import pytest
 
+import deep
 import instancing as I
 from selas_amd import native as N
 from selas_amd import workloads as W
@@ -40,12 +42,13 @@ def _subset(rays, start, n):
 def test_flat_scene_two_calls_match_intersect(gpu_ctx):
     t9 = N.gen_cluster_soup(3, 128, 1024, 0.03, 1e-3, 2e-2)
     scene = N.Scene(gpu_ctx)
-    scene.add_soup(t9)
+    scene.add_soup(np.concatenate([t9, deep.nested_soup(3, 17)]))
     scene.commit()
     try:
+        assert deep.stack_words(scene) > deep.LDS_WORDS
         cam = N.gen_camera_rays(W.CAMERA_POS, W.CAMERA_LOOK_AT, W.CAMERA_UP, 50.0, 256, 256, 1)
         bnc = N.gen_bounce_rays(4, t9, 65536)
-        rays = {k: np.concatenate([cam[k], bnc[k]]) for k in N.RAY_FIELDS}
+        rays = {k: np.concatenate([v[k] for v in (cam, bnc, deep.rays(5, 150000, 17))]) for k in N.RAY_FIELDS}
         info = scene.info()
         print(f"flat: {info}, {rays['org_x'].size} rays then 7000", flush=True)
         ref, got = _both(gpu_ctx, scene, rays, False)
