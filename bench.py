@@ -1055,8 +1055,8 @@ def bench_curves(args):
     mo = sum(b.elapsed_ms(c) for _, b, c in ev) / args.steps
     nodes, segs = st["curve_nodes_visited"] / n, st["curve_segments_tested"] / n
     hit_rate = float((h["prim_id"] != N.INVALID_ID).mean())
-    # per ray: ray 32 B + hit distance 4 B read, nodes x 64 B, segments x 80 B, 32 B hit record written
-    bytes_per_ray = 36 + nodes * 64 + segs * 80 + 32 * curve_hit
+    # per ray: ray 32 B + hit distance 4 B read, nodes x 64 B, segments x 64 B, 32 B hit record written
+    bytes_per_ray = 36 + nodes * 64 + segs * 64 + 32 * curve_hit
     achieved = n * bytes_per_ray / (mi / 1e3) / 1e9
     out = {
         "metric": "curve closest + any-hit Mrays/s",

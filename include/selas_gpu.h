@@ -83,7 +83,9 @@ typedef struct sgpu_hits_soa {
     uint32_t* inst_id1;
 } sgpu_hits_soa;
 
-/* Per-query traversal counters (filled by sgpu_intersect_stats). */
+/* Per-query traversal counters (filled by sgpu_intersect_stats). Which rays end a large launch eight
+ * lanes each depends on how its waves run, and those test some triangles more: the counts of two runs
+ * differ by some 1e-5. */
 typedef struct sgpu_trace_stats {
     uint64_t rays;
     uint64_t nodes_visited;  /* internal nodes whose child boxes were tested */
@@ -118,9 +120,13 @@ typedef struct sgpu_tuning {
                                      ray is done: 1..32 (default 8) */
     uint32_t trace_tree;          /* traversal tree: 0 binary nodes (64 B), 1 8-wide compressed
                                      nodes (128 B, default; the triangle records lie among
-                                     them); both are built at commit */
+                                     them); both are built at commit. The binary tree is walked by
+                                     one lane a ray, whatever the count; scenes of instances are
+                                     walked on the 8-wide tree */
     uint32_t trace_lds_nodes;     /* 8-wide single-scene launches: this many top nodes (breadth-first)
-                                     read from LDS instead of memory: 0..9 (default 0) */
+                                     read from LDS instead of memory: 0..9 (default 0). Launches
+                                     with it go one lane a ray: few rays do not get eight lanes each,
+                                     nor the last rays of a large launch */
     uint32_t vcm_graphs;          /* 1 (default): each VCM wavefront replays its light and camera
                                      passes as captured hipGraphs (queue counts read on the device);
                                      0: launches one by one, sized from counts read back per bounce */
@@ -266,11 +272,11 @@ int sgpu_occluded(sgpu_scene scene, const sgpu_rays_soa* rays, uint32_t* occlude
  * cannot allocate device memory (code under HIP stream capture, tight serving loops, hosts that
  * forbid hipMalloc). The traversal stacks' spill area, which sgpu_intersect allocates per call, is
  * a fixed 64 MiB array in device memory instead, one per GPU (looked up at sgpu_context_create and
- * held until the process ends); the grid is capped so that its spill fits (rays beyond it are taken
- * grid-stride). Results equal sgpu_intersect's. Fails with SGPU_E_RANGE when even one block's
+ * held until the process ends); the grid is capped so that its spill fits (its waves take the rays
+ * beyond it in chunks). Results equal sgpu_intersect's. Fails with SGPU_E_RANGE when even one block's
  * stacks would not fit (a scene whose stack bound exceeds 65,552 words a lane: the binary tree's depth,
- * or two words per level of the 8-wide tree). Calls that overlap on one GPU (other streams, other threads) share the array and race:
- * order them. */
+ * or two words per level of the 8-wide tree). Calls that overlap on one GPU (other streams, other
+ * threads) share the array and race: order them. */
 int sgpu_intersect_noalloc(sgpu_scene scene, const sgpu_rays_soa* rays, const sgpu_hits_soa* hits, uint32_t n,
                            void* stream);
 /* Same query as sgpu_intersect with per-ray node/triangle counters, summed into *stats.

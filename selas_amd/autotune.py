@@ -6,8 +6,9 @@ Two parameters decide how well the wavefront kernels fill an MI355X:
   vertex, photon-key and connection-slot queue of a render. Larger wavefronts put more rays into
   each traversal launch (hiding the latency of dependent node fetches) and more queries into each
   merge launch, at the cost of device memory (the server's footprint grows linearly).
-* trace_blocks_per_cu: the traversal grid. Rays beyond the grid are taken grid-stride, so more
-  blocks than fit on a CU at once balance the load between waves of uneven traversal length.
+* trace_blocks_per_cu: the traversal grid. Each wave starts with its own chunk of 64 rays and takes
+  the next ones from a counter; blocks that do not fit on their CU at once (the 8-wide kernels keep 5
+  there) start, with their first chunks, when others end.
 
 The search is coordinate-wise: wavefront sizes at the default grid, then grids at the best size,
 then sizes again at the best grid; a size whose server footprint does not fit the memory budget is

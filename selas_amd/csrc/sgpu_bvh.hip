@@ -835,9 +835,8 @@ uint32_t host_f2ord(float f)
 }
 
 // The binary tree over n primitive boxes (d_blo, d_bhi, centroids d_cent, bounds as k_prep
-// leaves them): Morton codes, radix sort, Karras hierarchy, bottom-up fit. On success *nodes_out
-// holds max(n - 1, 1) nodes, d_order the primitive of each leaf in leaf order and *depth the
-// deepest leaf.
+// leaves them): Morton codes, radix sort, box pyramid, Karras hierarchy. On success *nodes_out holds
+// max(n - 1, 1) nodes, d_order the primitive of each leaf in leaf order and *depth the deepest leaf.
 int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4* d_bhi, const float4* d_cent, const uint32_t* d_bounds,
                  hipStream_t stream, BvhNode** nodes_out, DevBuf<uint32_t>& d_order, uint32_t* depth_out,
                  uint32_t builder)
@@ -1532,7 +1531,6 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
     scene->n_inst = n;
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
-    scene->blas_stack_cap = blas_cap;
     // instance nodes name composed instances by their composition index (instance i, then its instance
     // j), so the closest-hit tie rule follows (inst_id0, inst_id1)
     rc = build_scene_wide(scene, S, nodes, n, stream, d_order.p, nullptr, d_inst);

@@ -13,8 +13,9 @@
 //
 // The tree is 8-wide, over the segments' tight boxes, and walked like the triangles' (sgpu_wide.h);
 // control points are slots like nodes, and a segment's points stay in the lane's slot in LDS for its
-// piece tests and searches. The closest entry does not depend on the order of the walk but where two
-// segments meet: the ball between them can be both segments' first entry at the same t. Such a tie goes
+// piece tests and searches. The closest entry of a ray that starts outside every tube does not depend on
+// the order of the walk but where two segments meet: the ball between them can be both segments' first
+// entry at the same t. Such a tie goes
 // to the segment that the binary tree over the control points' boxes, walked nearer child first,
 // comes to first.
 //

@@ -221,7 +221,6 @@ struct sgpu_scene_s {
     uint32_t* d_inst_ids = nullptr;    // inst_id0, inst_id1 per composed instance
     uint32_t n_inst = 0;
     uint32_t inst_levels = 0;          // 1 or 2 for an instanced scene
-    uint32_t blas_stack_cap = 0;       // the largest stack of the placed scenes' trees
     // shading data of an instanced scene, gathered at commit from the placed scenes: their
     // geometries numbered as one list (geometry g of placed scene m is d_inst_geom_base[k] + g for
     // every composed instance k of m), with the materials and textures those scenes held then

@@ -509,7 +509,8 @@ __device__ void trace_groups(const TraceScene& scene, const uint32_t* __restrict
 // address unit 69 %); 32 KB of LDS a block allow 5 waves per SIMD. Against the version that read nodes
 // and triangles lane by lane, sorted (distance, child) pairs and kept a stack of children: 16M rays in
 // 2M triangles 15.2 -> 10.2 ms, 4M shadow rays in 1M triangles 2.66 -> 1.57 ms, 250K rays 0.62 -> 0.32
-// ms, 4M rays through 256 instances (which had no refill) 9.8 -> 3.0 ms; hits the same bits.
+// ms (back to back; a call alone 0.35), 4M rays through 256 instances (which had no refill) 9.8 -> 3.0
+// ms; hits the same bits.
 template <bool ANY, bool STATS, bool MULTI, bool INST, bool TOP>
 __global__ __launch_bounds__(SGPU_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace8(
     TraceScene scene, const uint32_t* __restrict inst_ids, const TraceScene* __restrict table,
