@@ -459,7 +459,8 @@ __global__ __launch_bounds__(kBlock) void k_depth(int n, const int* __restrict p
 // of largest surface area (the first such child on ties) until it has 8 children or only leaves.
 // A task is a binary node and the slot its wide node goes to. k_wide_expand writes each task's
 // children (binary refs and boxes) and the counts of its internal children and of the slots its
-// children take; a scan of those counts numbers the next level's tasks and slots in task order, so the numbering (and the tree) is deterministic and a node's children are contiguous;
+// children take; a scan of those counts numbers the next level's tasks and slots in task order, so the
+// numbering (and the tree) is deterministic and a node's children are contiguous;
 // k_wide_emit quantizes the boxes and writes the node's first slot (internal children first), the
 // next level's tasks and the leaves' slots. In the top tree of an instanced scene leaves are nodes
 // too: a task ~k stands for leaf k, whose node is its instance's (InstNode). A node has 8 children
@@ -644,7 +645,7 @@ __global__ __launch_bounds__(kBlock) void k_wide_emit(uint32_t n_tasks, uint32_t
     out[level_base + t] = w;
 }
 
-// The nodes' first slots and the triangle records in their slots.
+// The nodes' first slots and the leaves' records in their slots.
 __global__ __launch_bounds__(kBlock) void k_place_nodes(const NodeSlot* __restrict in, const uint32_t* __restrict slot,
                                                         uint32_t n, NodeSlot* __restrict out)
 {
@@ -654,14 +655,16 @@ __global__ __launch_bounds__(kBlock) void k_place_nodes(const NodeSlot* __restri
     reinterpret_cast<uint4*>(out + slot[k / 4])[k % 4] = reinterpret_cast<const uint4*>(in + k / 4)[k % 4];
 }
 
-__global__ __launch_bounds__(kBlock) void k_place_tris(const TriRecord* __restrict in, const uint32_t* __restrict order,
-                                                       const uint32_t* __restrict leaf_slot, uint32_t n,
-                                                       NodeSlot* __restrict out)
+// (`stride` bytes from a record to the next, of which a slot's worth is placed)
+__global__ __launch_bounds__(kBlock) void k_place_records(const char* __restrict in, uint32_t stride,
+                                                          const uint32_t* __restrict order,
+                                                          const uint32_t* __restrict leaf_slot, uint32_t n,
+                                                          NodeSlot* __restrict out)
 {
     const size_t k = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const size_t j = k / 4;
     if (j >= n) return;
-    reinterpret_cast<uint4*>(out + leaf_slot[j])[k % 4] = reinterpret_cast<const uint4*>(in + order[j])[k % 4];
+    reinterpret_cast<uint4*>(out + leaf_slot[j])[k % 4] = reinterpret_cast<const uint4*>(in + (size_t)order[j] * stride)[k % 4];
 }
 
 // The binary tree's leaves named by their records' slots.
@@ -687,84 +690,98 @@ struct DevBuf {
     }
 };
 
-// Scratch bytes a build over n primitives takes: per primitive the records (64 for triangles, 80 for
-// curves), boxes and centroid (48), positions (40), codes and order (28), parents (8), the box pyramid
-// (64), the 8-wide tree's tasks (4/7 nodes of 348) and the sorts' own; in a top tree or with PLOC more,
-// taken as needed.
-size_t build_scratch(size_t n) { return 500 * n + ((size_t)1 << 20); }
+// Scratch bytes a build over n primitives takes at its widest, in the binary tree: per primitive the
+// record (64 for triangles, 80 for curves), order and places (12), positions (40, triangles), boxes and
+// centroid (48), sorted codes (8), parents (8) and the box pyramid (64); the sort before it and the 8-wide
+// tree after it take the same memory and need less. In a top tree or with PLOC more, taken as needed.
+size_t build_scratch(size_t n) { return 240 * n + ((size_t)1 << 20); }
 
 struct WideTree {
     WideNode* wide = nullptr;
     uint32_t n_slots = 0, n_wide = 0, depth = 0;
 };
 
-// Collapses the binary tree (nodes, root 0, over n leaves) into an 8-wide tree, with the records (64
-// bytes, triangles or curve segments) rec[order[j]] of its leaves j; d_leaf_slot: their slots. The top
-// tree of an instanced scene passes its instance records instead (order[j]: the instance of leaf j):
-// its leaves become nodes.
+// Collapses the binary tree (nodes, root 0, over n leaves) into an 8-wide tree, with the records rec[order[j]]
+// (rec_bytes apart, the first 64 a leaf's slot) of its leaves j; d_leaf_slot: their slots. The top tree of
+// an instanced scene passes its instance records instead (order[j]: the instance of leaf j): its leaves
+// become nodes.
 int build_wide(sgpu_scratch& S, const BvhNode* nodes, uint32_t n, hipStream_t stream, const uint32_t* order,
-               const TriRecord* rec, const InstRecord* insts, WideTree& tree, DevBuf<uint32_t>& d_leaf_slot)
+               const void* rec, uint32_t rec_bytes, const InstRecord* insts, WideTree& tree,
+               DevBuf<uint32_t>& d_leaf_slot)
 {
     const bool top = insts != nullptr;
     const uint32_t n_leaves = std::max(n, 2u);  // a tree of one leaf has a root with two children, the leaf twice
     const size_t max_nodes = (size_t)n_leaves * 4 / 7 + 2 + (top ? n_leaves : 0);
+    SGPU_HIP_TRY(d_leaf_slot.alloc(S, n_leaves));
+    sgpu_scratch::Frame frame(S);
     DevBuf<WideTask> d_tasks, d_next;
-    DevBuf<int> d_cref;
-    DevBuf<float> d_cbox;
-    DevBuf<uint32_t> d_nch, d_bad, d_slot;
-    DevBuf<uint64_t> d_cnt, d_off;
+    DevBuf<uint32_t> d_bad, d_slot;
     DevBuf<NodeSlot> d_all;
-    DevBuf<uint8_t> d_tmp;
     SGPU_HIP_TRY(d_tasks.alloc(S, max_nodes));
     SGPU_HIP_TRY(d_next.alloc(S, max_nodes));
-    SGPU_HIP_TRY(d_cref.alloc(S, 8 * max_nodes));
-    SGPU_HIP_TRY(d_cbox.alloc(S, 48 * max_nodes));
-    SGPU_HIP_TRY(d_nch.alloc(S, max_nodes));
-    SGPU_HIP_TRY(d_cnt.alloc(S, max_nodes));
-    SGPU_HIP_TRY(d_off.alloc(S, max_nodes));
     SGPU_HIP_TRY(d_bad.alloc(S, 1));
     SGPU_HIP_TRY(d_all.alloc(S, max_nodes));
     SGPU_HIP_TRY(d_slot.alloc(S, max_nodes));
-    SGPU_HIP_TRY(d_leaf_slot.alloc(S, n_leaves));
-    size_t tmp_bytes = 0;
-    SGPU_HIP_TRY(rocprim::inclusive_scan(nullptr, tmp_bytes, d_cnt.p, d_off.p, max_nodes, rocprim::plus<uint64_t>(),
-                                         stream));
-    SGPU_HIP_TRY(d_tmp.alloc(S, tmp_bytes));
     const WideTask root{0, 0};
     SGPU_HIP_TRY(hipMemcpyAsync(d_tasks.p, &root, sizeof(root), hipMemcpyHostToDevice, stream));
     SGPU_HIP_TRY(hipMemsetAsync(d_bad.p, 0, sizeof(uint32_t), stream));
     uint32_t level_base = 0, n_tasks = 1, depth = 0;
     uint64_t slot_base = 2;
+    // a level's tasks at most this many at a time: their children take 250 bytes a task, which for the last
+    // level of a top tree (its instances) would be the most of a build's scratch
+    const uint32_t chunk = std::max(1u << 17, n_leaves / 8);
     while (n_tasks > 0) {
-        const uint32_t grid = (n_tasks + kBlock - 1) / kBlock;
-        if (top)
-            hipLaunchKernelGGL(k_wide_expand<true>, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes,
-                               d_cref.p, d_cbox.p, d_nch.p, d_cnt.p);
-        else
-            hipLaunchKernelGGL(k_wide_expand<false>, dim3(grid), dim3(kBlock), 0, stream, d_tasks.p, n_tasks, nodes,
-                               d_cref.p, d_cbox.p, d_nch.p, d_cnt.p);
-        SGPU_HIP_TRY(hipGetLastError());
-        SGPU_HIP_TRY(rocprim::inclusive_scan(d_tmp.p, tmp_bytes, d_cnt.p, d_off.p, (size_t)n_tasks,
-                                             rocprim::plus<uint64_t>(), stream));
-        SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_off.p + n_tasks - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-        SGPU_HIP_TRY(hipStreamSynchronize(stream));
-        const uint64_t total = S.pinned()[0];
-        const uint32_t n_next = (uint32_t)(total & 0xFFFFFFFFull), n_new = (uint32_t)(total >> 32);
-        if ((uint64_t)level_base + n_tasks + n_next > max_nodes)
-            return sgpu_fail(SGPU_E_STATE, "wide tree larger than its bound");
-        if (slot_base + n_new > 0x7FFFFFFFull) return sgpu_fail(SGPU_E_RANGE, "wide tree takes more than 2^31 slots");
-        if (top)
-            hipLaunchKernelGGL(k_wide_emit<true>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
-                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
-                               d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
-        else
-            hipLaunchKernelGGL(k_wide_emit<false>, dim3(grid), dim3(kBlock), 0, stream, n_tasks, level_base,
-                               (uint32_t)slot_base, d_tasks.p, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p, d_slot.p,
-                               d_next.p, d_leaf_slot.p, insts, order, d_bad.p);
-        SGPU_HIP_TRY(hipGetLastError());
+        uint32_t n_next = 0;
+        for (uint32_t c0 = 0; c0 < n_tasks; c0 += chunk) {
+            const uint32_t nc = std::min(chunk, n_tasks - c0);
+            const WideTask* const tasks = d_tasks.p + c0;
+            sgpu_scratch::Frame children(S);
+            DevBuf<int> d_cref;
+            DevBuf<float> d_cbox;
+            DevBuf<uint32_t> d_nch;
+            DevBuf<uint64_t> d_cnt, d_off;
+            DevBuf<uint8_t> d_tmp;
+            SGPU_HIP_TRY(d_cref.alloc(S, 8 * (size_t)nc));
+            SGPU_HIP_TRY(d_cbox.alloc(S, 48 * (size_t)nc));
+            SGPU_HIP_TRY(d_nch.alloc(S, nc));
+            SGPU_HIP_TRY(d_cnt.alloc(S, nc));
+            SGPU_HIP_TRY(d_off.alloc(S, nc));
+            size_t tmp_bytes = 0;
+            SGPU_HIP_TRY(rocprim::inclusive_scan(nullptr, tmp_bytes, d_cnt.p, d_off.p, (size_t)nc,
+                                                 rocprim::plus<uint64_t>(), stream));
+            SGPU_HIP_TRY(d_tmp.alloc(S, tmp_bytes));
+            const uint32_t grid = (nc + kBlock - 1) / kBlock;
+            if (top)
+                hipLaunchKernelGGL(k_wide_expand<true>, dim3(grid), dim3(kBlock), 0, stream, tasks, nc, nodes, d_cref.p,
+                                   d_cbox.p, d_nch.p, d_cnt.p);
+            else
+                hipLaunchKernelGGL(k_wide_expand<false>, dim3(grid), dim3(kBlock), 0, stream, tasks, nc, nodes, d_cref.p,
+                                   d_cbox.p, d_nch.p, d_cnt.p);
+            SGPU_HIP_TRY(hipGetLastError());
+            SGPU_HIP_TRY(rocprim::inclusive_scan(d_tmp.p, tmp_bytes, d_cnt.p, d_off.p, (size_t)nc,
+                                                 rocprim::plus<uint64_t>(), stream));
+            SGPU_HIP_TRY(hipMemcpyAsync(S.pinned(), d_off.p + nc - 1, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
+            SGPU_HIP_TRY(hipStreamSynchronize(stream));
+            const uint64_t total = S.pinned()[0];
+            const uint32_t n_child = (uint32_t)(total & 0xFFFFFFFFull), n_new = (uint32_t)(total >> 32);
+            if ((uint64_t)level_base + n_tasks + n_next + n_child > max_nodes)
+                return sgpu_fail(SGPU_E_STATE, "wide tree larger than its bound");
+            if (slot_base + n_new > 0x7FFFFFFFull)
+                return sgpu_fail(SGPU_E_RANGE, "wide tree takes more than 2^31 slots");
+            if (top)
+                hipLaunchKernelGGL(k_wide_emit<true>, dim3(grid), dim3(kBlock), 0, stream, nc, level_base + c0,
+                                   (uint32_t)slot_base, tasks, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p,
+                                   d_slot.p, d_next.p + n_next, d_leaf_slot.p, insts, order, d_bad.p);
+            else
+                hipLaunchKernelGGL(k_wide_emit<false>, dim3(grid), dim3(kBlock), 0, stream, nc, level_base + c0,
+                                   (uint32_t)slot_base, tasks, d_off.p, d_cnt.p, d_cref.p, d_cbox.p, d_nch.p, d_all.p,
+                                   d_slot.p, d_next.p + n_next, d_leaf_slot.p, insts, order, d_bad.p);
+            SGPU_HIP_TRY(hipGetLastError());
+            n_next += n_child;
+            slot_base += n_new;
+        }
         std::swap(d_tasks.p, d_next.p);
         level_base += n_tasks;
-        slot_base += n_new;
         n_tasks = n_next;
         ++depth;
     }
@@ -781,7 +798,8 @@ int build_wide(sgpu_scratch& S, const BvhNode* nodes, uint32_t n, hipStream_t st
     hipLaunchKernelGGL(k_place_nodes, grid4(level_base), dim3(kBlock), 0, stream, d_all.p, d_slot.p, level_base, slots);
     SGPU_HIP_TRY(hipGetLastError());
     if (!top) {
-        hipLaunchKernelGGL(k_place_tris, grid4(n), dim3(kBlock), 0, stream, rec, order, d_leaf_slot.p, n, slots);
+        hipLaunchKernelGGL(k_place_records, grid4(n), dim3(kBlock), 0, stream, (const char*)rec, rec_bytes, order,
+                           d_leaf_slot.p, n, slots);
         SGPU_HIP_TRY(hipGetLastError());
         if (n == 1)  // a single leaf is both children of the root: slots 1 and 2
             for (int k = 1; k <= 2; ++k)
@@ -797,7 +815,7 @@ int build_scene_wide(sgpu_scene scene, sgpu_scratch& S, BvhNode* nodes, uint32_t
 {
     WideTree t;
     DevBuf<uint32_t> leaf_slot;
-    const int rc = build_wide(S, nodes, n, stream, order, rec, insts, t, leaf_slot);
+    const int rc = build_wide(S, nodes, n, stream, order, rec, sizeof(TriRecord), insts, t, leaf_slot);
     scene->d_wide = t.wide;
     scene->n_slots = t.n_slots;
     scene->n_wide = t.n_wide;
@@ -836,16 +854,18 @@ uint32_t host_f2ord(float f)
 
 // The binary tree over n primitive boxes (d_blo, d_bhi, centroids d_cent, bounds as k_prep
 // leaves them): Morton codes, radix sort, box pyramid, Karras hierarchy. On success *nodes_out holds
-// max(n - 1, 1) nodes, d_order the primitive of each leaf in leaf order and *depth the deepest leaf.
+// max(n - 1, 1) nodes (the caller's array, or where it is NULL a new one), d_order (the caller's) the
+// primitive of each leaf in leaf order and *depth the deepest leaf.
 int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4* d_bhi, const float4* d_cent, const uint32_t* d_bounds,
-                 hipStream_t stream, BvhNode** nodes_out, DevBuf<uint32_t>& d_order, uint32_t* depth_out,
+                 hipStream_t stream, BvhNode** nodes_out, const DevBuf<uint32_t>& d_order, uint32_t* depth_out,
                  uint32_t builder)
 {
+    sgpu_scratch::Frame frame(S);
     const uint32_t n_int = n > 1 ? n - 1 : 1;
-    BvhNode* nodes = nullptr;
-    SGPU_HIP_TRY(sgpu_device_malloc((void**)&nodes, (size_t)n_int * sizeof(BvhNode)));
+    BvhNode* nodes = *nodes_out;
+    if (!nodes) SGPU_HIP_TRY(sgpu_device_malloc((void**)&nodes, (size_t)n_int * sizeof(BvhNode)));
     auto fail_free = [&](int code, const std::string& msg) {
-        (void)hipFree(nodes);
+        if (!*nodes_out) (void)hipFree(nodes);
         return sgpu_fail(code, msg);
     };
 #define SGPU_BUILD_TRY(expr)                                                                  \
@@ -853,7 +873,6 @@ int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4*
         hipError_t _e = (expr);                                                               \
         if (_e != hipSuccess) return fail_free(SGPU_E_HIP, std::string(#expr) + ": " + hipGetErrorString(_e)); \
     } while (0)
-    SGPU_BUILD_TRY(d_order.alloc(S, n));
     if (n == 1) {
         hipLaunchKernelGGL(k_single, dim3(1), dim3(1), 0, stream, d_blo, d_bhi, d_bounds, nodes);
         SGPU_BUILD_TRY(hipGetLastError());
@@ -863,29 +882,25 @@ int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4*
         *depth_out = 1;
         return SGPU_OK;
     }
-    DevBuf<uint32_t> d_vals, d_depth;
-    DevBuf<uint64_t> d_keys, d_keys2;
-    DevBuf<int> d_pint, d_pleaf;
-    DevBuf<uint8_t> d_tmp;
-    SGPU_BUILD_TRY(d_keys.alloc(S, n));
-    SGPU_BUILD_TRY(d_keys2.alloc(S, n));
-    SGPU_BUILD_TRY(d_vals.alloc(S, n));
-    SGPU_BUILD_TRY(d_pint.alloc(S, n_int));
-    SGPU_BUILD_TRY(d_pleaf.alloc(S, n));
-    SGPU_BUILD_TRY(d_depth.alloc(S, 1));
-    SGPU_BUILD_TRY(hipMemsetAsync(d_pint.p, 0xFF, (size_t)n_int * sizeof(int), stream));
-    SGPU_BUILD_TRY(hipMemsetAsync(d_pleaf.p, 0xFF, (size_t)n * sizeof(int), stream));
-    SGPU_BUILD_TRY(hipMemsetAsync(d_depth.p, 0, sizeof(uint32_t), stream));
-
     const uint32_t grid = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_morton, dim3(grid), dim3(kBlock), 0, stream, d_cent, n, d_bounds, d_keys.p, d_vals.p);
-    SGPU_BUILD_TRY(hipGetLastError());
-    size_t tmp_bytes = 0;
-    SGPU_BUILD_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
-                                             (size_t)n, 0, 63, stream));
-    SGPU_BUILD_TRY(d_tmp.alloc(S, tmp_bytes));
-    SGPU_BUILD_TRY(rocprim::radix_sort_pairs(d_tmp.p, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
-                                             (size_t)n, 0, 63, stream));
+    DevBuf<uint64_t> d_keys2;
+    SGPU_BUILD_TRY(d_keys2.alloc(S, n));
+    {
+        sgpu_scratch::Frame sort(S);
+        DevBuf<uint64_t> d_keys;
+        DevBuf<uint32_t> d_vals;
+        DevBuf<uint8_t> d_tmp;
+        SGPU_BUILD_TRY(d_keys.alloc(S, n));
+        SGPU_BUILD_TRY(d_vals.alloc(S, n));
+        hipLaunchKernelGGL(k_morton, dim3(grid), dim3(kBlock), 0, stream, d_cent, n, d_bounds, d_keys.p, d_vals.p);
+        SGPU_BUILD_TRY(hipGetLastError());
+        size_t tmp_bytes = 0;
+        SGPU_BUILD_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
+                                                 (size_t)n, 0, 63, stream));
+        SGPU_BUILD_TRY(d_tmp.alloc(S, tmp_bytes));
+        SGPU_BUILD_TRY(rocprim::radix_sort_pairs(d_tmp.p, tmp_bytes, d_keys.p, d_keys2.p, d_vals.p, d_order.p,
+                                                 (size_t)n, 0, 63, stream));
+    }
     if (builder == 1) {
         // PLOC over the Morton-ordered leaves
         DevBuf<int> cid[2];
@@ -941,6 +956,14 @@ int build_binary(sgpu_scratch& S, uint32_t n, const float4* d_blo, const float4*
         *depth_out = h;
         return SGPU_OK;
     }
+    DevBuf<int> d_pint, d_pleaf;
+    DevBuf<uint32_t> d_depth;
+    SGPU_BUILD_TRY(d_pint.alloc(S, n_int));
+    SGPU_BUILD_TRY(d_pleaf.alloc(S, n));
+    SGPU_BUILD_TRY(d_depth.alloc(S, 1));
+    SGPU_BUILD_TRY(hipMemsetAsync(d_pint.p, 0xFF, (size_t)n_int * sizeof(int), stream));
+    SGPU_BUILD_TRY(hipMemsetAsync(d_pleaf.p, 0xFF, (size_t)n * sizeof(int), stream));
+    SGPU_BUILD_TRY(hipMemsetAsync(d_depth.p, 0, sizeof(uint32_t), stream));
     // the pyramid's levels one after another: level k has ceil(n / 2^k) boxes
     DevBuf<LeafBox> d_boxes;
     SGPU_BUILD_TRY(d_boxes.alloc(S, 2 * (size_t)n + 2 * kMaxBoxLevels));
@@ -1045,15 +1068,6 @@ __global__ __launch_bounds__(kBlock) void k_curve_prep(const CurveRecord* __rest
     }
 }
 
-// The control points alone, as leaf records.
-__global__ __launch_bounds__(kBlock) void k_curve_points(const CurveRecord* __restrict in, uint32_t n,
-                                                         CurvePoints* __restrict out)
-{
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    for (int j = 0; j < 4; ++j) out[i].p[j] = in[i].p[j];
-}
-
 // Each segment's place in the leaf order `order`.
 __global__ __launch_bounds__(kBlock) void k_curve_places(const uint32_t* __restrict order, uint32_t n,
                                                          uint32_t* __restrict place)
@@ -1094,55 +1108,50 @@ int sgpu_curve_build(sgpu_scene scene, const std::vector<float>& cp, const std::
         rec[s].inst = inst[s];
         rec[s].pad = 0;
     }
-    sgpu_scratch S(scene->ctx, stream, build_scratch(n));
+    sgpu_scratch S(scene->ctx, stream, build_scratch(n) + n * sizeof(BvhNode));
     DevBuf<CurveRecord> d_rec;
-    DevBuf<float4> d_blo, d_bhi, d_cent;
-    DevBuf<uint32_t> d_bounds, d_order;
+    DevBuf<uint32_t> d_bounds, d_order, d_place, d_leaf_slot;
     SGPU_HIP_TRY(d_rec.alloc(S, n));
-    SGPU_HIP_TRY(d_blo.alloc(S, n));
-    SGPU_HIP_TRY(d_bhi.alloc(S, n));
-    SGPU_HIP_TRY(d_cent.alloc(S, n));
     SGPU_HIP_TRY(d_bounds.alloc(S, 12));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_rec.p, rec.data(), n * sizeof(CurveRecord), hipMemcpyHostToDevice, stream));
-    SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
-    const uint32_t grid = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_curve_prep<false>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p, d_cent.p,
-                       d_bounds.p);
-    SGPU_HIP_TRY(hipGetLastError());
-    uint32_t hb[12];
-    SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
-    // the tree that orders hits at equal distance
-    uint32_t depth = 0;
-    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &scene->d_cnodes, d_order, &depth, 0);
-    if (rc != SGPU_OK) return rc;
-    if (depth + 1 > kCurveStack)
-        return sgpu_fail(SGPU_E_RANGE, "curve tree deeper than the curve traversal's stack");
-    DevBuf<uint32_t> d_place, d_order2, d_leaf_slot;
-    DevBuf<CurvePoints> d_points;
+    SGPU_HIP_TRY(d_order.alloc(S, n));
     SGPU_HIP_TRY(d_place.alloc(S, n));
-    SGPU_HIP_TRY(d_points.alloc(S, n));
-    hipLaunchKernelGGL(k_curve_places, dim3(grid), dim3(kBlock), 0, stream, d_order.p, n, d_place.p);
-    hipLaunchKernelGGL(k_curve_points, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_points.p);
-    SGPU_HIP_TRY(hipGetLastError());
-    // the tree that is walked, over the tight boxes
-    SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
-    hipLaunchKernelGGL(k_curve_prep<true>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p, d_cent.p,
-                       d_bounds.p);
-    SGPU_HIP_TRY(hipGetLastError());
-    struct Nodes {
-        BvhNode* p = nullptr;
-        ~Nodes() { (void)hipFree(p); }
-    } walked;
-    rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &walked.p, d_order2, &depth, 0);
+    SGPU_HIP_TRY(hipMemcpyAsync(d_rec.p, rec.data(), n * sizeof(CurveRecord), hipMemcpyHostToDevice, stream));
+    const uint32_t grid = (n + kBlock - 1) / kBlock;
+    uint32_t hb[12], depth = 0;
+    DevBuf<BvhNode> walked;
+    SGPU_HIP_TRY(walked.alloc(S, n));
+    // the tree that orders hits at equal distance, then the one that is walked, over the tight boxes
+    for (int tight = 0; tight < 2; ++tight) {
+        sgpu_scratch::Frame boxes(S);
+        DevBuf<float4> d_blo, d_bhi, d_cent;
+        SGPU_HIP_TRY(d_blo.alloc(S, n));
+        SGPU_HIP_TRY(d_bhi.alloc(S, n));
+        SGPU_HIP_TRY(d_cent.alloc(S, n));
+        SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
+        if (tight)
+            hipLaunchKernelGGL(k_curve_prep<true>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p,
+                               d_cent.p, d_bounds.p);
+        else
+            hipLaunchKernelGGL(k_curve_prep<false>, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, n, d_blo.p, d_bhi.p,
+                               d_cent.p, d_bounds.p);
+        SGPU_HIP_TRY(hipGetLastError());
+        if (!tight) SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
+        const int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream,
+                                    tight ? &walked.p : &scene->d_cnodes, d_order, &depth, 0);
+        if (rc != SGPU_OK) return rc;
+        if (tight) continue;
+        if (depth + 1 > kCurveStack)
+            return sgpu_fail(SGPU_E_RANGE, "curve tree deeper than the curve traversal's stack");
+        hipLaunchKernelGGL(k_curve_places, dim3(grid), dim3(kBlock), 0, stream, d_order.p, n, d_place.p);
+        SGPU_HIP_TRY(hipGetLastError());
+    }
     WideTree tree;
-    if (rc == SGPU_OK)
-        rc = build_wide(S, walked.p, n, stream, d_order2.p, reinterpret_cast<const TriRecord*>(d_points.p), nullptr, tree,
-                        d_leaf_slot);
+    const int rc = build_wide(S, walked.p, n, stream, d_order.p, d_rec.p, sizeof(CurveRecord), nullptr, tree, d_leaf_slot);
     scene->d_cwide = tree.wide;
     scene->n_cslots = tree.n_slots;
     if (rc != SGPU_OK) return rc;
     SGPU_HIP_TRY(sgpu_device_malloc((void**)&scene->d_cids, (size_t)tree.n_slots * sizeof(uint4)));
-    hipLaunchKernelGGL(k_curve_ids, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order2.p, d_leaf_slot.p, d_place.p, n,
+    hipLaunchKernelGGL(k_curve_ids, dim3(grid), dim3(kBlock), 0, stream, d_rec.p, d_order.p, d_leaf_slot.p, d_place.p, n,
                        scene->d_cids);
     SGPU_HIP_TRY(hipGetLastError());
     SGPU_HIP_TRY(hipStreamSynchronize(stream));
@@ -1173,42 +1182,44 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
     if (n > (1u << 30)) return sgpu_fail(SGPU_E_RANGE, "scene has more than 2^30 triangles");
 
     sgpu_scratch S(scene->ctx, stream, build_scratch(n));
-    DevBuf<float> d_pos;
-    DevBuf<uint32_t> d_geom, d_first, d_bounds, d_order;
+    DevBuf<uint32_t> d_bounds, d_order;
     DevBuf<TriRecord> d_rec;
-    DevBuf<float4> d_blo, d_bhi, d_cent;
-    SGPU_HIP_TRY(d_pos.alloc(S, (size_t)n * 9));
-    SGPU_HIP_TRY(d_geom.alloc(S, n));
-    SGPU_HIP_TRY(d_first.alloc(S, scene->geom_first.size()));
     SGPU_HIP_TRY(d_bounds.alloc(S, 12));
+    SGPU_HIP_TRY(d_order.alloc(S, n));
     SGPU_HIP_TRY(d_rec.alloc(S, n));
-    SGPU_HIP_TRY(d_blo.alloc(S, n));
-    SGPU_HIP_TRY(d_bhi.alloc(S, n));
-    SGPU_HIP_TRY(d_cent.alloc(S, n));
-
-    SGPU_HIP_TRY(hipMemcpyAsync(d_pos.p, scene->tri_pos.data(), (size_t)n * 9 * sizeof(float), hipMemcpyHostToDevice,
-                                stream));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_geom.p, scene->tri_geom.data(), (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice,
-                                stream));
-    // device copy of the geometries' first indices with bit 31 set for quad geometries
-    std::vector<uint32_t> first_flagged(scene->geom_first.size());
-    for (size_t g = 0; g < first_flagged.size(); ++g)
-        first_flagged[g] = scene->geom_first[g] | (scene->geom_quad[g] == 1 ? 0x80000000u : 0u);
-    SGPU_HIP_TRY(hipMemcpy(d_first.p, first_flagged.data(), first_flagged.size() * sizeof(uint32_t),
-                           hipMemcpyHostToDevice));
-    SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
-    const uint32_t grid = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_prep, dim3(grid), dim3(kBlock), 0, stream, d_pos.p, n, d_geom.p, d_first.p, d_rec.p, d_blo.p,
-                       d_bhi.p, d_cent.p, d_bounds.p);
-    SGPU_HIP_TRY(hipGetLastError());
-    uint32_t hb[12];
-    SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
-
     BvhNode* nodes = nullptr;
-    uint32_t depth = 0;
-    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
-                          scene->ctx->bvh_builder);
-    if (rc != SGPU_OK) return rc;
+    uint32_t depth = 0, hb[12];
+    {
+        sgpu_scratch::Frame input(S);
+        DevBuf<float> d_pos;
+        DevBuf<uint32_t> d_geom, d_first;
+        DevBuf<float4> d_blo, d_bhi, d_cent;
+        SGPU_HIP_TRY(d_pos.alloc(S, (size_t)n * 9));
+        SGPU_HIP_TRY(d_geom.alloc(S, n));
+        SGPU_HIP_TRY(d_first.alloc(S, scene->geom_first.size()));
+        SGPU_HIP_TRY(d_blo.alloc(S, n));
+        SGPU_HIP_TRY(d_bhi.alloc(S, n));
+        SGPU_HIP_TRY(d_cent.alloc(S, n));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_pos.p, scene->tri_pos.data(), (size_t)n * 9 * sizeof(float), hipMemcpyHostToDevice,
+                                    stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_geom.p, scene->tri_geom.data(), (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice,
+                                    stream));
+        // device copy of the geometries' first indices with bit 31 set for quad geometries
+        std::vector<uint32_t> first_flagged(scene->geom_first.size());
+        for (size_t g = 0; g < first_flagged.size(); ++g)
+            first_flagged[g] = scene->geom_first[g] | (scene->geom_quad[g] == 1 ? 0x80000000u : 0u);
+        SGPU_HIP_TRY(hipMemcpy(d_first.p, first_flagged.data(), first_flagged.size() * sizeof(uint32_t),
+                               hipMemcpyHostToDevice));
+        SGPU_HIP_TRY(hipMemsetAsync(d_bounds.p, 0xFF, 12 * sizeof(uint32_t), stream));
+        const uint32_t grid = (n + kBlock - 1) / kBlock;
+        hipLaunchKernelGGL(k_prep, dim3(grid), dim3(kBlock), 0, stream, d_pos.p, n, d_geom.p, d_first.p, d_rec.p, d_blo.p,
+                           d_bhi.p, d_cent.p, d_bounds.p);
+        SGPU_HIP_TRY(hipGetLastError());
+        SGPU_HIP_TRY(hipMemcpyAsync(hb, d_bounds.p, sizeof(hb), hipMemcpyDeviceToHost, stream));
+        const int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
+                                    scene->ctx->bvh_builder);
+        if (rc != SGPU_OK) return rc;
+    }
     for (int k = 0; k < 3; ++k) {
         scene->box[k] = host_ord2f(hb[k]);
         scene->box[3 + k] = host_ord2f(~hb[3 + k]);
@@ -1216,7 +1227,7 @@ int sgpu_bvh_build(sgpu_scene scene, hipStream_t stream)
     scene->d_nodes = nodes;
     scene->n_nodes = n > 1 ? n - 1 : 1;
     scene->max_depth = depth;
-    rc = build_scene_wide(scene, S, nodes, n, stream, d_order.p, d_rec.p, nullptr);
+    const int rc = build_scene_wide(scene, S, nodes, n, stream, d_order.p, d_rec.p, nullptr);
     scene->wide_stack = wide_stack_words(scene->wide_depth);
     // the binary tree's stack: a word per level
     scene->stack_cap = std::max(scene->max_depth + 1, scene->wide_stack);
@@ -1498,21 +1509,27 @@ int sgpu_bvh_build_instances(sgpu_scene scene, hipStream_t stream)
         scene->box[3 + r] = shi[r];
     }
     sgpu_scratch S(scene->ctx, stream, build_scratch(n));
-    DevBuf<float4> d_blo, d_bhi, d_cent;
-    DevBuf<uint32_t> d_bounds, d_order;
-    SGPU_HIP_TRY(d_blo.alloc(S, n));
-    SGPU_HIP_TRY(d_bhi.alloc(S, n));
-    SGPU_HIP_TRY(d_cent.alloc(S, n));
-    SGPU_HIP_TRY(d_bounds.alloc(S, 12));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_blo.p, blo.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_bhi.p, bhi.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_cent.p, cent.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
-    SGPU_HIP_TRY(hipMemcpyAsync(d_bounds.p, hb, sizeof(hb), hipMemcpyHostToDevice, stream));
+    DevBuf<uint32_t> d_order;
+    SGPU_HIP_TRY(d_order.alloc(S, n));
     BvhNode* nodes = nullptr;
     uint32_t depth = 0;
-    int rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
+    int rc = SGPU_OK;
+    {
+        sgpu_scratch::Frame boxes(S);
+        DevBuf<float4> d_blo, d_bhi, d_cent;
+        DevBuf<uint32_t> d_bounds;
+        SGPU_HIP_TRY(d_blo.alloc(S, n));
+        SGPU_HIP_TRY(d_bhi.alloc(S, n));
+        SGPU_HIP_TRY(d_cent.alloc(S, n));
+        SGPU_HIP_TRY(d_bounds.alloc(S, 12));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_blo.p, blo.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_bhi.p, bhi.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_cent.p, cent.data(), n * sizeof(float4), hipMemcpyHostToDevice, stream));
+        SGPU_HIP_TRY(hipMemcpyAsync(d_bounds.p, hb, sizeof(hb), hipMemcpyHostToDevice, stream));
+        rc = build_binary(S, n, d_blo.p, d_bhi.p, d_cent.p, d_bounds.p, stream, &nodes, d_order, &depth,
                           scene->ctx->bvh_builder);
-    if (rc != SGPU_OK) return rc;
+        if (rc != SGPU_OK) return rc;
+    }
     InstRecord* d_inst = nullptr;
     uint32_t* d_ids = nullptr;
     hipError_t e = sgpu_device_malloc((void**)&d_inst, rec.size() * sizeof(InstRecord));

@@ -305,22 +305,36 @@ void sgpu_scratch_trim(sgpu_context ctx);
 // the context keeps: allocating and freeing it per call took longer than the work (a 256 x 256 image
 // 16.4 -> 5.9 ms, a 500K-triangle commit 12.7 -> 4.6 ms). A block is one call's alone until the call's
 // stream has drained, so calls on other threads and streams take others. Larger than `first` in all:
-// further blocks are taken as needed.
+// further blocks are taken as needed. What is cut while a Frame lives is free again after it, for what
+// the call's stream does next.
 struct sgpu_scratch {
     sgpu_context ctx;
     hipStream_t stream;
     hipError_t err;
     std::vector<ScratchBlock> blocks;
-    size_t used = 0;
+    size_t cur = 0, used = 0;  // the block being cut, and how much of it is
     sgpu_scratch(sgpu_context c, hipStream_t s, size_t first) : ctx(c), stream(s), err(hipSuccess) { grow(first); }
     sgpu_scratch(const sgpu_scratch&) = delete;
     sgpu_scratch& operator=(const sgpu_scratch&) = delete;
+    struct Frame {
+        sgpu_scratch& s;
+        const size_t cur, used;
+        explicit Frame(sgpu_scratch& S) : s(S), cur(S.cur), used(S.used) {}
+        Frame(const Frame&) = delete;
+        Frame& operator=(const Frame&) = delete;
+        ~Frame()
+        {
+            s.cur = cur;
+            s.used = used;
+        }
+    };
     bool grow(size_t bytes)
     {
         ScratchBlock b;
         err = sgpu_scratch_take(ctx, bytes, b);
         if (err != hipSuccess) return false;
         blocks.push_back(b);
+        cur = blocks.size() - 1;
         used = 0;
         return true;
     }
@@ -329,8 +343,15 @@ struct sgpu_scratch {
     {
         const size_t bytes = (count * sizeof(T) + 511) & ~(size_t)255;
         if (err != hipSuccess) return nullptr;
-        if (used + bytes > blocks.back().bytes && !grow(std::max(bytes, blocks.back().bytes / 2))) return nullptr;
-        T* p = (T*)(blocks.back().dev + used);
+        while (used + bytes > blocks[cur].bytes) {
+            if (cur + 1 < blocks.size()) {
+                ++cur;
+                used = 0;
+            } else if (!grow(std::max(bytes, blocks.back().bytes / 2)) && !grow(bytes)) {
+                return nullptr;
+            }
+        }
+        T* p = (T*)(blocks[cur].dev + used);
         used += bytes;
         return p;
     }

@@ -46,6 +46,15 @@ def test_refused_commit_leaves_nothing(limit_lib, kind):
     _child(limit_lib, "refused " + kind)
 
 
+# bytes a primitive of device memory that a commit gets by with, the scene's own included
+COMMIT_BYTES = {"triangles": 480, "curves": 580, "instances": 613}
+
+
+@pytest.mark.parametrize("kind", list(COMMIT_BYTES))
+def test_commit_memory(limit_lib, kind):
+    _child(limit_lib, "memory " + kind)
+
+
 # ---- the child ---------------------------------------------------------------------------------------
 
 def _main(so, call):
@@ -80,6 +89,25 @@ def _main(so, call):
         return dh.to_host()
 
     lim_off = lambda: lim.alloc_limit_set(ctypes.c_size_t(-1).value)
+    if call.startswith("memory"):
+        kind, n = call.split()[1], 64000
+        s = N.Scene(ctx)
+        if kind == "triangles":
+            s.add_soup(soup(1, n))
+        elif kind == "curves":
+            for k in range(n // 2000):
+                s.add_curves(strands + np.float32([0.1 * k, 0, 0, 0]), np.arange(2000, dtype=np.uint32))
+        else:
+            model, n = scene(ctx, 16), 400000
+            m = np.eye(4, dtype=np.float32).reshape(-1)
+            for k in range(n):
+                m[12:15] = (k % 71, k // 71 % 73, k // 5183)
+                N.check(N.lib.sgpu_scene_add_instance(s.handle, model.handle, N.fptr(m), None))
+        lim.alloc_limit_set(lim.alloc_limit_used() + COMMIT_BYTES[kind] * n)
+        s.commit()
+        lim_off()
+        print(f"{call}: ok", flush=True)
+        return
     sc = W.room_scene(1)
     room = N.build_render_scene(ctx, sc)
     bare = scene(ctx, 1600)  # (a small scratch block for the calls that take one)
