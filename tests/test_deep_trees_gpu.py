@@ -139,22 +139,28 @@ def _deep_scene(levels):
 
 @pytest.mark.parametrize("levels", [SPILLS, TOO_DEEP])
 def test_several_scenes_at_once(gpu_ctx, levels):
-    """Jobs on a deep instanced scene and on a flat one in one wavefront (the scene-table launches), past
-    the counts that eight lanes a ray take: each job's image is that of the job alone (launches over its
-    one scene) but for the order of its splats and merged photons."""
+    """Jobs on a deep instanced scene and on a flat one in one wavefront (the scene-table launches, as
+    graphs and one by one), past the counts that eight lanes a ray take: each job's image is that of the
+    job alone launched one by one (over its one scene, without the table) but for the order of its splats
+    and merged photons."""
     deep_sc, flat_sc = _deep_scene(levels), W.sized_vcm_scene(5, 1e4, textures=False)
     sd, sf = N.build_render_scene(gpu_ctx, deep_sc), N.build_render_scene(gpu_ctx, flat_sc)
     _check_words(sd, levels == TOO_DEEP)
     print(f"several scenes, {levels} levels", flush=True)
-    # (the alone runs: 500 x 500 paths a launch too, then 64 x 64)
     jobs = [(sd, deep_sc["camera"], 500, 500, 1, 6), (sf, flat_sc["camera"], 200, 200, 2, 7), (sd, deep_sc["camera"], 64, 64, 2, 8)]
-    alone = [N.render_vcm(s, cam, w, h, its, 6, 0.01, 0.75, seed) for s, cam, w, h, its, seed in jobs]
-    batch = N.render_vcm_batch([dict(scene=s, camera=cam, width=w, height=h, iterations=its, max_path_length=6,
-                                     base_radius=0.01, radius_alpha=0.75, seed=seed) for s, cam, w, h, its, seed in jobs])
-    for a, b in zip(alone, batch):
-        assert a.mean() > 1e-3
-        # sums of one sign of some hundred terms in another order: 100 x 2^-24 = 6e-6 relative
-        np.testing.assert_allclose(b, a, rtol=1e-5, atol=1e-6 * float(a.max()))
+    try:
+        gpu_ctx.set_tuning(vcm_graphs=0)
+        alone = [N.render_vcm(s, cam, w, h, its, 6, 0.01, 0.75, seed) for s, cam, w, h, its, seed in jobs]
+        for graphs in (0, 1):
+            gpu_ctx.set_tuning(vcm_graphs=graphs)
+            batch = N.render_vcm_batch([dict(scene=s, camera=cam, width=w, height=h, iterations=its, max_path_length=6,
+                                             base_radius=0.01, radius_alpha=0.75, seed=seed) for s, cam, w, h, its, seed in jobs])
+            for a, b in zip(alone, batch):
+                assert a.mean() > 1e-3
+                # sums of one sign of some hundred terms in another order: 100 x 2^-24 = 6e-6 relative
+                np.testing.assert_allclose(b, a, rtol=1e-5, atol=1e-6 * float(a.max()))
+    finally:
+        gpu_ctx.set_tuning(vcm_graphs=1)
     sd.release()
     sf.release()
 
